@@ -175,8 +175,9 @@ int kore_gemm_a8w8_blockscale(const void* xq, int64_t ldx, const void* wq, int64
  *   element strides (ldx_m, ldx_k); wq [N,K] with (ldw_n, ldw_k); xs [M] and ws [N]
  *   fp32 with element strides xs_stride / ws_stride (x_scale [M,1], w_scale [1,N] or
  *   [N,1] views); Y row stride ldy.  Per-tensor scales are equal entries.  Any K and
- *   any strides (K % 128 == 0, N % 128 == 0, K-contiguous 16-byte aligned rows take the
- *   MFMA kernels; everything else a generic kernel); int8 sums are exact in int32.
+ *   any strides (K-contiguous rows with K >= 128 take the MFMA kernels, fastest with
+ *   K % 128 == 0, N % 128 == 0 and 16-byte aligned rows; everything else a generic
+ *   kernel); int8 sums are exact in int32.
  * Replaces: gemm(xq, wq, x_scale, w_scale)
  *           kore/tasks/gemm_fp8_a8w8/seed_triton.py (per-tensor),
  *           kore/tasks/gemm_fp8_a8w8_pertoken/seed_triton.py,

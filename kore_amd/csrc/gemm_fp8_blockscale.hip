@@ -258,6 +258,13 @@ __device__ __forceinline__ void buf_lds(__amdgpu_buffer_rsrc_t r, uint32_t voff,
 
 __device__ __forceinline__ int f8_key(int r) { return (r ^ (r >> 3)) & 7; }
 
+// ---- ragged row-scale problems (RAG: any N, any K >= 128, rows at any byte alignment) ----
+// Loads take rows at any byte alignment (direct-to-LDS and register loads alike).  Weight
+// rows past N repeat row N - 1 and are never stored.  A K tail is one more 128-wide block
+// read from K - 128, so no load passes K, whose first 128 - K % 128 bytes (which the full
+// blocks cover too) are zeroed in the weight fragment: the products they meet are
+// then zero, or NaN where x itself holds a NaN that belongs to the sum anyway.
+
 // 32 K-consecutive bytes of one row: two 16-byte chunks at their swizzled positions.
 __device__ __forceinline__ i32x8_t lds_frag32(const uint8_t* row, const int (&off)[2]) {
   const u32x4_t lo = *(const u32x4_t*)(row + off[0]);
@@ -274,13 +281,16 @@ __device__ __forceinline__ i32x8_t lds_frag32(const uint8_t* row, const int (&of
 // at most kFp8GroupM row tiles (launched side by side, sharing it through L2), or, in
 // the grouped mode, by one expert's row blocks.  The policy is an instruction immediate,
 // hence a template flag (a branch would split the tile loop).
-template <typename C, bool FULL_M, bool GROUPED = false, bool BNT = false>
+// RAG (row-scale modes): ragged N, K and row alignment, see zero_lead above; the K tail is
+// multiplied before the pipelined loop, from registers, while the loop's first stages land.
+template <typename C, bool FULL_M, bool GROUPED = false, bool BNT = false, bool RAG = false>
 __global__ void __launch_bounds__(C::NW * 64)
     gemm_fp8_pipe_kernel(const Fp8Params p) {
   constexpr int NW = C::NW, MI = C::MI, NI = C::NI, NT = C::NT, TB = C::TB;
   constexpr int AQ = C::AQ, BQ = C::BQ, LPS = C::LPS, PER = C::PER, NSLOT = C::NSLOT;
   constexpr bool XS4 = C::XS4, ROW = C::ROW, I8 = C::MODE == Q_ROW_I8;
   static_assert(!GROUPED || (ROW && !FULL_M), "grouped tiles use row scales and gathered rows");
+  static_assert(!RAG || (ROW && !FULL_M), "ragged tiles use row scales and clamped rows");
   using AccT = std::conditional_t<I8, i32x16_t, f32x16_t>;
 
   __shared__ __attribute__((aligned(1024))) uint8_t lds[C::LDS];
@@ -325,8 +335,9 @@ __global__ void __launch_bounds__(C::NW * 64)
   // ---- buffer resources (tile-based) and per-lane load offsets ----
   const __amdgpu_buffer_rsrc_t ra = GROUPED ? make_rsrc(p.xq, (uint32_t)((int64_t)p.M * p.ldx))
                                             : make_rsrc(p.xq + (int64_t)m0 * p.ldx, (uint32_t)(rows_a * p.ldx));
+  const int rows_b = RAG ? min(p.N - n0, C::BN) : C::BN;
   const __amdgpu_buffer_rsrc_t rb =
-      make_rsrc(p.wq + (int64_t)expert * p.w_estride + (int64_t)n0 * p.ldw, (uint32_t)(C::BN * p.ldw));
+      make_rsrc(p.wq + (int64_t)expert * p.w_estride + (int64_t)n0 * p.ldw, (uint32_t)(rows_b * p.ldw));
   const __amdgpu_buffer_rsrc_t rx =
       make_rsrc(p.xs + (int64_t)m0 * p.xs_m, (uint32_t)(((rows_a - 1) * p.xs_m + (nk - 1) * p.xs_k + 1) * 4));
   const __amdgpu_buffer_rsrc_t rw = make_rsrc(
@@ -343,7 +354,10 @@ __global__ void __launch_bounds__(C::NW * 64)
 #pragma unroll
     for (int q = 0; q < AQ; ++q) a_voff[q] = (uint32_t)(grow(lrow + 8 * (wave + NW * q)) * p.ldx + 16 * dchunk);
   }
-  const uint32_t b_voff = (uint32_t)((lrow + 8 * wave) * p.ldw + 16 * dchunk);
+  uint32_t b_voff[RAG ? BQ : 1];
+#pragma unroll
+  for (int q = 0; q < (RAG ? BQ : 1); ++q)
+    b_voff[q] = (uint32_t)((RAG ? min(lrow + 8 * (wave + NW * q), rows_b - 1) : lrow + 8 * wave) * p.ldw + 16 * dchunk);
   const uint32_t x_voff = (uint32_t)(min(64 * (wave & 3) + lane, rows_a - 1) * p.xs_m * 4);
   const uint32_t a_rstep = (uint32_t)(8 * NW * p.ldx), b_rstep = (uint32_t)(8 * NW * p.ldw);
   const uint32_t xs_kstep = (uint32_t)(p.xs_k * 4), ws_kstep = (uint32_t)(p.ws_k * 4);
@@ -360,7 +374,8 @@ __global__ void __launch_bounds__(C::NW * 64)
       const uint32_t so = (uint32_t)kb * 128u + (FULL_M ? (uint32_t)q * a_rstep : 0u);
       buf_lds(ra, v, so, base + (wave + NW * q) * 1024, 16);
     } else if (q < AQ + BQ) {
-      buf_lds<(GROUPED || BNT) ? kCpolNT : kCpolDefault>(rb, b_voff, (uint32_t)kb * 128u + (uint32_t)(q - AQ) * b_rstep,
+      buf_lds<(GROUPED || BNT) ? kCpolNT : kCpolDefault>(rb, b_voff[RAG ? q - AQ : 0],
+                                                (uint32_t)kb * 128u + (RAG ? 0u : (uint32_t)(q - AQ) * b_rstep),
                                                 base + C::A_BYTES + (wave + NW * (q - AQ)) * 1024, 16);
     } else if constexpr (!ROW) {
       // scale load (wave-uniform selects): activation scales, or weight-scale copies
@@ -422,6 +437,32 @@ __global__ void __launch_bounds__(C::NW * 64)
   for (int st = 0; st + 1 < NSLOT; ++st)
 #pragma unroll
     for (int q = 0; q < LPS; ++q) issue(st, min(st, nk - 1), q);
+  if constexpr (RAG) {
+    const int ktail = p.K & 127;
+    if (ktail != 0) {  // uniform
+      const uint8_t* wt = p.wq + (int64_t)expert * p.w_estride + (int64_t)n0 * p.ldw + (p.K - 128);
+      const uint8_t* xt = p.xq + (GROUPED ? (int64_t)0 : (int64_t)m0 * p.ldx) + (p.K - 128);
+      auto frag = [&](const uint8_t* row, int h, int lead) {
+        const int k = 64 * h + 32 * hh;
+        const u32x4_t lo = zero_lead(ld16_any(row + k), lead - k);
+        const u32x4_t hi = zero_lead(ld16_any(row + k + 16), lead - k - 16);
+        return i32x8_t{(int)lo[0], (int)lo[1], (int)lo[2], (int)lo[3], (int)hi[0], (int)hi[1], (int)hi[2], (int)hi[3]};
+      };
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        i32x8_t tb[NI], ta[MI];
+#pragma unroll
+        for (int j = 0; j < NI; ++j)
+          tb[j] = frag(wt + (int64_t)min(rowB0 + 32 * j + lr, rows_b - 1) * p.ldw, h, 128 - ktail);
+#pragma unroll
+        for (int i = 0; i < MI; ++i) ta[i] = frag(xt + (int64_t)grow(rowA0 + 32 * i + lr) * p.ldx, h, 0);
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+          for (int j = 0; j < NI; ++j) row_mma(acc[i][j], tb[j], ta[i]);
+      }
+    }
+  }
   wait_vmcnt<C::WAITN>();
   exec_barrier();
   af[0][0] = lds_frag32(lds + rowA0 * 128, off[0]);
@@ -541,9 +582,9 @@ __global__ void __launch_bounds__(C::NW * 64)
     for (int g = 0; g < 4; ++g) {
       float wcol[4] = {1.0f, 1.0f, 1.0f, 1.0f};
       if constexpr (ROW) {
-        const int64_t n = n0 + rowB0 + out_col(j, g, lane);  // n + 3 < N: N % BN == 0
+        const int64_t n = n0 + rowB0 + out_col(j, g, lane);  // n + 3 < N unless RAG: N % BN == 0
 #pragma unroll
-        for (int e = 0; e < 4; ++e) wcol[e] = wsx[(n + e) * p.ws_n];
+        for (int e = 0; e < 4; ++e) wcol[e] = wsx[(RAG ? min(n + e, (int64_t)p.N - 1) : n + e) * p.ws_n];
       }
 #pragma unroll
       for (int i = 0; i < MI; ++i) {
@@ -566,11 +607,15 @@ __global__ void __launch_bounds__(C::NW * 64)
   });
 }
 
-template <typename C>
+template <typename C, bool RAG = false>
 int launch_fp8_pipe(Fp8Params p, hipStream_t st) {
   p.tiles_m = (p.M + C::BM - 1) / C::BM;
-  p.tiles_n = p.N / C::BN;
+  p.tiles_n = (p.N + C::BN - 1) / C::BN;
   const dim3 grid((unsigned)((int64_t)p.tiles_m * p.tiles_n)), block(C::NW * 64);
+  if constexpr (RAG) {
+    hipLaunchKernelGGL((gemm_fp8_pipe_kernel<C, false, false, false, true>), grid, block, 0, st, p);
+    return check_launch("gemm_fp8_pipe_kernel");
+  }
   // Block scales with one group of row tiles (kFp8GroupM of them sweep the column tiles
   // together): each weight tile is read once from memory.  Same process, cold cache:
   // M=256 / 512 33.5 / 33.3 -> 27.7 / 28.3 us, warm 21.1 / 24.0 -> 23.1 / 25.0 us.
@@ -1196,7 +1241,8 @@ struct SkinnyCfg {
 // M=16..64 within 3% -- the kernel's time is its L2-to-LDS operand stream, not LDS reads.
 __device__ __forceinline__ int sk_key(int r) { return (r ^ (r >> 3)) & 7; }
 
-template <typename C>
+// RAG: ragged N, K and row alignment (row-scale modes, see zero_lead).
+template <typename C, bool RAG = false>
 __global__ void __launch_bounds__(C::NW_ * 64)
     gemm_fp8_skinny_kernel(const Fp8Params p) {
   constexpr int MT = C::MT_, NW = C::NW_, S = C::S_, MB = C::MB, NB = C::NB, BN = C::BN;
@@ -1209,12 +1255,14 @@ __global__ void __launch_bounds__(C::NW_ * 64)
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 15, g = lane >> 4;
   const int n0 = (int)blockIdx.x * BN;
-  const int nk = p.K / 128;
+  static_assert(!RAG || ROW, "ragged problems use row scales");
+  const int nk = RAG ? (p.K + 127) / 128 : p.K / 128;
   const int cnt = nk > wave ? (nk - wave + NW - 1) / NW : 0;  // K blocks of this wave
+  const int rows_b = RAG ? min(BN, p.N - n0) : BN;
 
   // buffer resources: X rows [0, M), this workgroup's BN rows of W
   const __amdgpu_buffer_rsrc_t rx = make_rsrc(p.xq, (uint32_t)((int64_t)(p.M - 1) * p.ldx + p.K));
-  const __amdgpu_buffer_rsrc_t rw = make_rsrc(p.wq + (int64_t)n0 * p.ldw, (uint32_t)((BN - 1) * p.ldw + p.K));
+  const __amdgpu_buffer_rsrc_t rw = make_rsrc(p.wq + (int64_t)n0 * p.ldw, (uint32_t)((rows_b - 1) * p.ldw + p.K));
   // DMA load q covers LDS rows 8q .. 8q+7; lane l fetches row 8q + l/8, logical chunk
   // (l % 8) ^ key(row) into position l % 8
   uint32_t xoff[XQ], woff[WQ];
@@ -1226,7 +1274,7 @@ __global__ void __launch_bounds__(C::NW_ * 64)
 #pragma unroll
   for (int q = 0; q < WQ; ++q) {
     const int row = 8 * q + (lane >> 3);
-    woff[q] = (uint32_t)((int64_t)row * p.ldw + 16 * ((lane & 7) ^ sk_key(row)));
+    woff[q] = (uint32_t)((int64_t)(RAG ? min(row, rows_b - 1) : row) * p.ldw + 16 * ((lane & 7) ^ sk_key(row)));
   }
   const __amdgpu_buffer_rsrc_t rxs =
       make_rsrc(p.xs, (uint32_t)(((int64_t)(p.M - 1) * p.xs_m + (int64_t)(nk - 1) * p.xs_k + 1) * 4));
@@ -1243,7 +1291,8 @@ __global__ void __launch_bounds__(C::NW_ * 64)
 
   // issue the loads of block j into stage slot s (DMA operands, then scales)
   auto issue = [&](int s, int j) {
-    const uint32_t ko = (uint32_t)(wave + NW * j) * 128u;
+    // the last block of a K tail ends at K
+    const uint32_t ko = RAG ? (uint32_t)min((wave + NW * j) * 128, p.K - 128) : (uint32_t)(wave + NW * j) * 128u;
     uint8_t* st = ring + s * STAGE;
 #pragma unroll
     for (int q = 0; q < XQ; ++q) buf_lds(rx, xoff[q], ko, st + q * 1024, 16);
@@ -1290,8 +1339,13 @@ __global__ void __launch_bounds__(C::NW_ * 64)
         for (int nb = 0; nb < NB; ++nb) {
           const uint8_t* row = st + (MT + nb * 16 + r) * 128;
           const int key = (k0 ^ (2 * nb)) & 7;
-          const u32x4_t lo = *(const u32x4_t*)(row + ((g ^ key) << 4));
-          const u32x4_t hi = *(const u32x4_t*)(row + (((4 + g) ^ key) << 4));
+          u32x4_t lo = *(const u32x4_t*)(row + ((g ^ key) << 4));
+          u32x4_t hi = *(const u32x4_t*)(row + (((4 + g) ^ key) << 4));
+          if (RAG && wave + NW * j == nk - 1) {  // uniform: the columns a K tail repeats
+            const int lead = 128 * nk - p.K;
+            lo = zero_lead(lo, lead - 16 * g);
+            hi = zero_lead(hi, lead - 64 - 16 * g);
+          }
           wf[nb] = i32x8_t{(int)lo[0], (int)lo[1], (int)lo[2], (int)lo[3], (int)hi[0], (int)hi[1], (int)hi[2], (int)hi[3]};
         }
         float sc[MB];
@@ -1331,37 +1385,41 @@ __global__ void __launch_bounds__(C::NW_ * 64)
   // ---- cross-wave reduction: red[wave][m][n] over the (now idle) ring, fixed-order sum ----
   wait_vmcnt<0>();
   __syncthreads();
-  float* red = (float*)lds;
+  // (int8 partials stay int32, so the sum over the waves is exact too)
+  using RedT = std::conditional_t<I8, int, float>;
+  RedT* red = (RedT*)lds;
 #pragma unroll
   for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb)
-      *(f32x4_t*)(red + (wave * MT + mb * 16 + r) * BNP + nb * 16 + 4 * g) =
-          f32x4_t{(float)acc[mb][nb][0], (float)acc[mb][nb][1], (float)acc[mb][nb][2], (float)acc[mb][nb][3]};
+      *(AccT*)(red + (wave * MT + mb * 16 + r) * BNP + nb * 16 + 4 * g) = acc[mb][nb];
   __syncthreads();
   constexpr int ITEMS = MT * BN / 8;  // 8 consecutive columns per item
   const bool vec = p.vec_store != 0;
   for (int it = tid; it < ITEMS; it += NW * 64) {
     const int m = it / (BN / 8), c8 = (it % (BN / 8)) * 8;
     if (m >= p.M) continue;
-    float sum[8];
+    RedT tot[8];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) sum[e] = 0.0f;
+    for (int e = 0; e < 8; ++e) tot[e] = 0;
 #pragma unroll
     for (int w = 0; w < NW; ++w) {
-      const f32x4_t a = *(const f32x4_t*)(red + (w * MT + m) * BNP + c8);
-      const f32x4_t b = *(const f32x4_t*)(red + (w * MT + m) * BNP + c8 + 4);
+      const AccT a = *(const AccT*)(red + (w * MT + m) * BNP + c8);
+      const AccT b = *(const AccT*)(red + (w * MT + m) * BNP + c8 + 4);
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        sum[e] += a[e];
-        sum[e + 4] += b[e];
+        tot[e] += a[e];
+        tot[e + 4] += b[e];
       }
     }
+    float sum[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) sum[e] = (float)tot[e];
     const int gn = n0 + c8;
     if constexpr (ROW) {
       const float xv = p.xs[(int64_t)m * p.xs_m];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) sum[e] = sum[e] * xv * p.ws[(int64_t)(gn + e) * p.ws_n];
+      for (int e = 0; e < 8; ++e) sum[e] = sum[e] * xv * p.ws[(int64_t)(RAG ? min(gn + e, p.N - 1) : gn + e) * p.ws_n];
     }
     using Op = MfmaOp<BF16>;
     const u32x4_t v{Op::pack2(sum[0], sum[1]), Op::pack2(sum[2], sum[3]), Op::pack2(sum[4], sum[5]),
@@ -1370,10 +1428,10 @@ __global__ void __launch_bounds__(C::NW_ * 64)
   }
 }
 
-template <typename C>
+template <typename C, bool RAG = false>
 int launch_fp8_skinny(const Fp8Params& p, hipStream_t st) {
-  const dim3 grid((unsigned)(p.N / C::BN)), block(C::NW_ * 64);
-  hipLaunchKernelGGL((gemm_fp8_skinny_kernel<C>), grid, block, 0, st, p);
+  const dim3 grid((unsigned)((p.N + C::BN - 1) / C::BN)), block(C::NW_ * 64);
+  hipLaunchKernelGGL((gemm_fp8_skinny_kernel<C, RAG>), grid, block, 0, st, p);
   return check_launch("gemm_fp8_skinny_kernel");
 }
 
@@ -1478,8 +1536,8 @@ extern "C" int kore_gemm_a8w8_blockscale(const void* xq, int64_t ldx, const void
 // a8w8 GEMM with per-row activation and per-column weight scales (fp8 e4m3 or
 // int8): Y[M,N] = bf16((sum_k xq[m,k] * wq[n,k]) * xs[m] * ws[n]).  The tiled and
 // skinny kernels above run it in their row-scale modes (the K loop accumulates in
-// the MFMA registers, scales are applied once in the epilogue); anything they cannot
-// take (a K not a multiple of 128, strided or unaligned rows) runs a generic kernel.
+// the MFMA registers, scales are applied once in the epilogue), ragged N, K and row
+// alignments included; K < 128 and rows that are not K-contiguous run a generic kernel.
 // ==============================================================================
 namespace kore {
 namespace {
@@ -1566,8 +1624,9 @@ __global__ void __launch_bounds__(256) gemm_a8w8_generic_kernel(const A8GenericP
 // accumulators stay in place in AGPRs.  int8: 16x16x64 MFMAs on the same 16-byte chunks as
 // the 16x16x32 bf16 ones (mainloop16), int32 accumulators; fp8: 16x16x128 MFMAs on both
 // chunks of a stage (mainloop_f8).  Epilogue as the row-scale pipe kernel: float(acc) *
-// xs[m] * ws[n], one bf16 rounding.  Requires N % 256 == 0, K % 128 == 0, 16-byte aligned rows.
-template <int MODE>
+// xs[m] * ws[n], one bf16 rounding.  Requires N % 256 == 0, K % 128 == 0, 16-byte aligned rows
+// unless RAG (any N, K >= 128 and row alignment; a K tail runs as the first stage).
+template <int MODE, bool RAG>
 __global__ void __launch_bounds__(256) gemm_a8w8_buf_kernel(const Fp8Params p) {
   constexpr bool I8 = MODE == Q_ROW_I8;
   using E = BufPipeEngine<std::conditional_t<I8, INT8, FP8>, 256, 256, 2, 2, 1, B_KC, kCpolDefault, true, A_KC>;
@@ -1582,7 +1641,7 @@ __global__ void __launch_bounds__(256) gemm_a8w8_buf_kernel(const Fp8Params p) {
   const int gsz = min(p.tiles_m - first_m, kFp8GroupM);
   const int tl = bid - grp * width;
   const int m0 = (first_m + tl % gsz) * 256, n0 = (tl / gsz) * 256;
-  const int rows_a = min(256, p.M - m0);
+  const int rows_a = min(256, p.M - m0), rows_b = RAG ? min(256, p.N - n0) : 256;
   E eng;
   eng.ra = make_rsrc(p.xq + (int64_t)m0 * p.ldx, (uint32_t)((int64_t)(rows_a - 1) * p.ldx + p.K));
 #pragma unroll
@@ -1590,16 +1649,19 @@ __global__ void __launch_bounds__(256) gemm_a8w8_buf_kernel(const Fp8Params p) {
     const int r = E::a_row(wave, lane, j);
     eng.a_voff[j] = (uint32_t)((int64_t)min(r, rows_a - 1) * p.ldx + 16 * E::chunk(r, lane));
   }
-  eng.rb = make_rsrc(p.wq + (int64_t)n0 * p.ldw, (uint32_t)(255 * p.ldw + p.K));
+  eng.rb = make_rsrc(p.wq + (int64_t)n0 * p.ldw, (uint32_t)((int64_t)(rows_b - 1) * p.ldw + p.K));
 #pragma unroll
   for (int j = 0; j < E::BJ; ++j) {
     const int r = E::b_row(wave, lane, j);
-    eng.b_voff[j] = (uint32_t)((int64_t)r * p.ldw + 16 * E::chunk(r, lane));
+    eng.b_voff[j] = (uint32_t)((int64_t)(RAG ? min(r, rows_b - 1) : r) * p.ldw + 16 * E::chunk(r, lane));
   }
   f32x4_t acc[MI][NI][4];
   E::zero16(acc);
-  if constexpr (I8) eng.mainloop16(lds, p.K / 2, acc);  // K in 16-bit units: 64 per 128-byte stage
-  else eng.mainloop_f8(lds, p.K / 2, acc);
+  const int kst = (p.K + 127) / 128 * 64;  // K in 16-bit units: 64 per 128-byte stage
+  eng.a_klast = (uint32_t)(p.K - 128);
+  eng.kdup = 2 * kst - p.K;
+  if constexpr (I8) eng.template mainloop16<false, RAG>(lds, kst, acc);
+  else eng.template mainloop_f8<RAG>(lds, kst, acc);
 
   using St = Stager<E::WROWS, E::WCOLS>;
   using Op = MfmaOp<BF16>;
@@ -1621,7 +1683,10 @@ __global__ void __launch_bounds__(256) gemm_a8w8_buf_kernel(const Fp8Params p) {
 #pragma unroll
     for (int h = 0; h < 2; ++h)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) wcol[j][h][e] = p.ws[(int64_t)(nw0 + acc_col<true>(j, h, lane) + e) * p.ws_n];
+      for (int e = 0; e < 4; ++e) {
+        const int n = nw0 + acc_col<true>(j, h, lane) + e;
+        wcol[j][h][e] = p.ws[(int64_t)(RAG ? min(n, p.N - 1) : n) * p.ws_n];
+      }
 #pragma unroll
   for (int j = 0; j < NI; ++j)
 #pragma unroll
@@ -1655,36 +1720,38 @@ __global__ void __launch_bounds__(256) gemm_a8w8_buf_kernel(const Fp8Params p) {
   });
 }
 
-template <int MODE>
+template <int MODE, bool RAG>
 int launch_a8w8_buf(Fp8Params p, hipStream_t st) {
   p.tiles_m = (p.M + 255) / 256;
-  p.tiles_n = p.N / 256;
+  p.tiles_n = (p.N + 255) / 256;
   const int64_t blocks = (int64_t)p.tiles_m * p.tiles_n;
   if (blocks > 0x7fffffff) return set_error(KORE_EUNSUPPORTED, "gemm_a8w8: grid too large");
-  hipLaunchKernelGGL((gemm_a8w8_buf_kernel<MODE>), dim3((unsigned)blocks), dim3(256), 0, st, p);
+  hipLaunchKernelGGL((gemm_a8w8_buf_kernel<MODE, RAG>), dim3((unsigned)blocks), dim3(256), 0, st, p);
   return check_launch("gemm_a8w8_buf_kernel");
 }
 
-template <int MODE>
+template <int MODE, bool RAG>
 int launch_a8w8(const Fp8Params& p0, bool skinny, hipStream_t st) {
   Fp8Params p = p0;
   if (skinny) {
     // 16-column workgroups when 32-column ones would leave CUs idle (N < 8192)
     if (p.N / 32 < 256) {
-      if (p.M <= 16) return launch_fp8_skinny<SkinnyCfg<16, 8, 3, MODE, 1>>(p, st);
-      if (p.M <= 32) return launch_fp8_skinny<SkinnyCfg<32, 8, 3, MODE, 1>>(p, st);
-      if (p.M <= 64) return launch_fp8_skinny<SkinnyCfg<64, 8, 2, MODE, 1>>(p, st);
-      return launch_fp8_skinny<SkinnyCfg<128, 4, 2, MODE, 1>>(p, st);
+      if (p.M <= 16) return launch_fp8_skinny<SkinnyCfg<16, 8, 3, MODE, 1>, RAG>(p, st);
+      if (p.M <= 32) return launch_fp8_skinny<SkinnyCfg<32, 8, 3, MODE, 1>, RAG>(p, st);
+      if (p.M <= 64) return launch_fp8_skinny<SkinnyCfg<64, 8, 2, MODE, 1>, RAG>(p, st);
+      return launch_fp8_skinny<SkinnyCfg<128, 4, 2, MODE, 1>, RAG>(p, st);
     }
-    if (p.M <= 16) return launch_fp8_skinny<SkinnyCfg<16, 8, 3, MODE>>(p, st);
-    if (p.M <= 32) return launch_fp8_skinny<SkinnyCfg<32, 8, 2, MODE>>(p, st);
-    if (p.M <= 64) return launch_fp8_skinny<SkinnyCfg<64, 4, 3, MODE>>(p, st);
-    return launch_fp8_skinny<SkinnyCfg<128, 4, 2, MODE>>(p, st);
+    if (p.M <= 16) return launch_fp8_skinny<SkinnyCfg<16, 8, 3, MODE>, RAG>(p, st);
+    if (p.M <= 32) return launch_fp8_skinny<SkinnyCfg<32, 8, 2, MODE>, RAG>(p, st);
+    if (p.M <= 64) return launch_fp8_skinny<SkinnyCfg<64, 4, 3, MODE>, RAG>(p, st);
+    return launch_fp8_skinny<SkinnyCfg<128, 4, 2, MODE>, RAG>(p, st);
   }
   // tile choice as for the block-scale kernels
-  const int64_t tiles256 = (int64_t)(p.M + 255) / 256 * (p.N / 256);
-  const int64_t tiles256x128 = (int64_t)(p.M + 255) / 256 * (p.N / 128);
-  const int64_t tiles128 = (int64_t)(p.M + 127) / 128 * (p.N / 128);
+  // (ragged N: the last column tile is partly empty)
+  const bool n256 = RAG || p.N % 256 == 0;
+  const int64_t tiles256 = (int64_t)(p.M + 255) / 256 * ((p.N + 255) / 256);
+  const int64_t tiles256x128 = (int64_t)(p.M + 255) / 256 * ((p.N + 127) / 128);
+  const int64_t tiles128 = (int64_t)(p.M + 127) / 128 * ((p.N + 127) / 128);
   // the dense 4-wave tile with the accumulators in AGPRs, where K is deep enough to carry
   // its prologue and its 4-wave epilogue (same process, bit-equal, against the 8-wave pipe
   // kernel).  int8: 4096^3 65.6 -> 56.6 us, 8192 x 4096 x 4096 128.4 -> 112.1 us,
@@ -1693,11 +1760,11 @@ int launch_a8w8(const Fp8Params& p0, bool skinny, hipStream_t st) {
   // 3072 44.4 -> 41.0 us, 4096 x 8192 x 2048 61.8 -> 57.7 us, 4096^2 x 2048 32.7 -> 30.9 us;
   // at K = 1024 a tie (4096^2 21.4 either way, 3072 x 4096 19.3 against 19.6 us).
   const int kmin_buf = MODE == Q_ROW_I8 ? 1024 : 2048;
-  if (p.N % 256 == 0 && tiles256 >= 192 && p.K >= kmin_buf) return launch_a8w8_buf<MODE>(p, st);
-  if (p.N % 256 == 0 && tiles256 >= 192) return launch_fp8_pipe<F8Cfg<256, 256, 8, 2, false, MODE>>(p, st);
+  if (n256 && tiles256 >= 192 && p.K >= kmin_buf) return launch_a8w8_buf<MODE, RAG>(p, st);
+  if (n256 && tiles256 >= 192) return launch_fp8_pipe<F8Cfg<256, 256, 8, 2, false, MODE>, RAG>(p, st);
   if (tiles256x128 >= 192 || tiles128 > device_cus())
-    return launch_fp8_pipe<F8Cfg<256, 128, 8, 3, false, MODE>>(p, st);
-  return launch_fp8_pipe<F8Cfg<128, 128, 4, 4, false, MODE>>(p, st);
+    return launch_fp8_pipe<F8Cfg<256, 128, 8, 3, false, MODE>, RAG>(p, st);
+  return launch_fp8_pipe<F8Cfg<128, 128, 4, 4, false, MODE>, RAG>(p, st);
 }
 
 template <typename C>
@@ -1750,10 +1817,17 @@ extern "C" int kore_gemm_a8w8(int qtype, const void* xq, int64_t ldx_m, int64_t 
   if (M >= (1ll << 31) || N >= (1ll << 31) || K >= (1ll << 31))
     return set_error(KORE_EUNSUPPORTED, "gemm_a8w8: dimension >= 2^31");
   hipStream_t st = (hipStream_t)stream;
-  const bool fast = ldx_k == 1 && ldw_k == 1 && K % 128 == 0 && N % 128 == 0 && ldx_m % 16 == 0 &&
-                    ldw_n % 16 == 0 && aligned16(xq) && aligned16(wq) && 256 * ldx_m + K < (1ll << 31) &&
-                    256 * ldw_n + K < (1ll << 31) && ldx_m >= K && ldw_n >= K;
-  if (fast) {
+  // K-contiguous rows and K >= 128 run the MFMA kernels: as they are with whole tiles and
+  // 16-byte aligned rows, in their ragged form with any N, K and row alignment.  Against the
+  // generic kernel, which took these before (K < 128 and other strides stay there: no whole
+  // block to read, or no 16 bytes along K): int8 64 x 4096 x 4095 549 -> 12.3 us (aligned
+  // K = 4096: 7.4), fp8 2048 x 11967 x 1280 1595 -> 78 us, 1024 x 2714 x 1408 269 -> 13.8 us,
+  // 3 x 781 x 5735 596 -> 6.9 us, 256 x 640 x 625 93 -> 13 us.
+  const bool kc = ldx_k == 1 && ldw_k == 1 && K >= 128 && 256 * ldx_m + K < (1ll << 31) &&
+                  256 * ldw_n + K < (1ll << 31) && ldx_m >= K && ldw_n >= K;
+  const bool whole = K % 128 == 0 && N % 128 == 0 && ldx_m % 16 == 0 && ldw_n % 16 == 0 && aligned16(xq) &&
+                     aligned16(wq);
+  if (kc) {
     Fp8Params p{};
     p.xq = (const uint8_t*)xq;
     p.wq = (const uint8_t*)wq;
@@ -1773,7 +1847,11 @@ extern "C" int kore_gemm_a8w8(int qtype, const void* xq, int64_t ldx_m, int64_t 
     p.tiles_m = p.tiles_n = 0;
     p.vec_store = (ldy % 8 == 0) && aligned16(y);
     const bool skinny = M <= 128;
-    return qtype == KORE_Q_FP8 ? launch_a8w8<Q_ROW_FP8>(p, skinny, st) : launch_a8w8<Q_ROW_I8>(p, skinny, st);
+    if (whole)
+      return qtype == KORE_Q_FP8 ? launch_a8w8<Q_ROW_FP8, false>(p, skinny, st)
+                                 : launch_a8w8<Q_ROW_I8, false>(p, skinny, st);
+    return qtype == KORE_Q_FP8 ? launch_a8w8<Q_ROW_FP8, true>(p, skinny, st)
+                               : launch_a8w8<Q_ROW_I8, true>(p, skinny, st);
   }
   A8GenericParams g{(const uint8_t*)xq, (const uint8_t*)wq, xs, ws, (uint16_t*)y, (int)M, (int)N, (int)K,
                     ldx_m, ldx_k, ldw_n, ldw_k, xs_stride, ws_stride, ldy};

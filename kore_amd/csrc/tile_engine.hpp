@@ -25,6 +25,20 @@ constexpr int kBK = 64;  // K elements per step (128 bytes per row)
 
 __device__ __forceinline__ u32x4_t ld16(const void* p) { return *(const u32x4_t*)p; }
 __device__ __forceinline__ u32x4_t zero4() { return u32x4_t{0u, 0u, 0u, 0u}; }
+__device__ __forceinline__ u32x4_t ld16_any(const void* p) {  // any byte alignment
+  u32x4_t v;
+  __builtin_memcpy(&v, p, 16);
+  return v;
+}
+// `lead` leading bytes of a 16-byte chunk zeroed (none below 1, all from 16 on).
+__device__ __forceinline__ u32x4_t zero_lead(u32x4_t v, int lead) {
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    const int n = lead - 4 * w;
+    v[w] = n <= 0 ? v[w] : (n >= 4 ? 0u : v[w] & (0xffffffffu << (8 * n)));
+  }
+  return v;
+}
 
 // 8x8 transpose of 16-bit values: in[r] holds row r (8 values); out[c] holds column c.
 __device__ __forceinline__ void transpose8x8(const u32x4_t in[8], u32x4_t out[8]) {
@@ -470,6 +484,19 @@ struct BufPipeEngine {
     }
   }
 
+  // K tail of 8-bit operands (KF modes of the main loops, K % 128 != 0): the block that ends
+  // at K runs first, as stage 0 read from byte a_klast = K - 128 of each row, and the full
+  // blocks follow as stages 1 .. nk - 1.  Its first kdup bytes, which the full blocks cover
+  // too, are zeroed in the B operand; the zeroing sits in the prologue, outside the loop.
+  __device__ __forceinline__ void zero_lead_b(uint16_t* st) const {
+    static_assert(BN == NW * 64 && !NC, "one B row per thread");
+    const int r = threadIdx.x;
+    for (int c = 0; 16 * c < kdup; ++c) {
+      u32x4_t* q = (u32x4_t*)(st + B_OFF + r * kBK + ((c ^ row_key(r)) << 3));
+      *q = zero_lead(*q, kdup - 16 * c);
+    }
+  }
+
   __device__ __forceinline__ void issue_one(uint16_t* lds, int slot, uint32_t soff, uint32_t soffb, int wave,
                                             int q) {
     uint16_t* sA = lds + slot * STAGE;
@@ -618,8 +645,9 @@ struct BufPipeEngine {
 #pragma unroll
         for (int g = 0; g < 4; ++g) c4[i][j][g] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   }
-  // KT: K tail mode (K here is the padded length 64 nk; see a_klast / kdup).
-  template <bool KT = false>
+  // KT: K tail mode (K here is the padded length 64 nk; see a_klast / kdup).  KF: K tail of
+  // 8-bit operands (zero_lead_b).
+  template <bool KT = false, bool KF = false>
   __device__ __forceinline__ void mainloop16(uint16_t* lds, int K, f32x4_t (&c4)[MI][NI][4]) {
     using Op = MfmaOp<T>;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -695,6 +723,7 @@ struct BufPipeEngine {
     const uint32_t kmax = (uint32_t)(nk - 1) * (kBK * 2);
     auto soff_of = [&](int stage) -> uint32_t {
       if constexpr (KT) return stage >= nk - 1 ? a_klast : (uint32_t)stage * (kBK * 2);
+      else if constexpr (KF) return stage == 0 ? a_klast : (uint32_t)(min(stage, nk - 1) - 1) * (kBK * 2);
       else return min((uint32_t)stage * (kBK * 2), kmax);
     };
     auto soffb_of = [&](int stage) -> uint32_t {
@@ -714,6 +743,11 @@ struct BufPipeEngine {
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         exec_barrier();
       }
+    }
+    if constexpr (KF) {
+      zero_lead_b(lds);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      exec_barrier();
     }
     // 8 waves: A fragments are single-buffered: A block (pl, i, half sm) of the next
     // sub-step is read right after its last MFMA in this one (tile j = NI - 1, sub-tile
@@ -803,6 +837,7 @@ struct BufPipeEngine {
   // the slot stage s leaves; each fragment of the next stage is read right after its last
   // use in this one (A blocks after their row of tiles, B blocks in the last row; 32-byte
   // fragments of two stages do not fit the registers).  K in 16-bit units (64 per stage).
+  template <bool KF = false>
   __device__ __forceinline__ void mainloop_f8(uint16_t* lds, int K, f32x4_t (&c4)[MI][NI][4]) {
     static_assert(NW == 4 && !NC && !AMC && AP == 1 && M16, "fp8 main loop: 4 waves, K-contiguous operands");
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -841,13 +876,21 @@ struct BufPipeEngine {
     constexpr int NMMA = MI * NI * 4;
     static_assert(NFB <= NMMA && LPS <= NMMA && LPS <= 32, "interleave needs enough MFMAs; vmcnt range");
     const uint32_t kmax = (uint32_t)(nk - 1) * (kBK * 2);
-    auto soff_of = [&](int stage) { return min((uint32_t)stage * (kBK * 2), kmax); };
+    auto soff_of = [&](int stage) -> uint32_t {
+      if constexpr (KF) return stage == 0 ? a_klast : (uint32_t)(min(stage, nk - 1) - 1) * (kBK * 2);
+      else return min((uint32_t)stage * (kBK * 2), kmax);
+    };
 #pragma unroll
-    for (int q = 0; q < LPS; ++q) issue_one(lds, 0, 0u, 0u, wave, q);
+    for (int q = 0; q < LPS; ++q) issue_one(lds, 0, soff_of(0), soff_of(0), wave, q);
 #pragma unroll
     for (int q = 0; q < LPS; ++q) issue_one(lds, 1, soff_of(1), soff_of(1), wave, q);
     wait_vmcnt<LPS>();
     exec_barrier();
+    if constexpr (KF) {
+      zero_lead_b(lds);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      exec_barrier();
+    }
     i32x8_t fa[NFA], fb[NFB];
 #pragma unroll
     for (int f = 0; f < NFA; ++f) read_f(0, f, fa[f]);

@@ -145,6 +145,53 @@ def test_a8w8_buffer_tile(gpu, kind, M, N, K):
     verdict(out, ref, "north_star", kind, label + " (1e-2)")
 
 
+@pytest.mark.parametrize("kind", ["fp8", "int8"])
+@pytest.mark.parametrize("M,N,K", [(1, 1, 128), (16, 127, 129), (17, 513, 255), (64, 4096, 4095), (128, 129, 1000),
+                                   (129, 300, 131), (600, 1000, 515), (1500, 2050, 641), (3000, 4095, 2049),
+                                   (2000, 8191, 129), (4, 8200, 384)])
+def test_a8w8_ragged(gpu, kind, M, N, K):
+    """Any N, any K >= 128 and rows at any byte alignment on the MFMA kernels: skinny (M <= 128,
+    16- and 32-column workgroups), 128x128, 256x128 and 256x256 pipe tiles and the 4-wave buffer
+    tile.  int8 sums are exact, so the result equals the zero-padded aligned problem's bit for
+    bit; fp8 meets the oracle on a row sample.  A base one byte off the allocation and a row
+    stride larger than K give the same bits.  A NaN code in the columns that the tail block
+    repeats stays in its own row or column."""
+    xq, wq, xs, ws = W.a8w8_inputs(M, N, K, kind, "pertoken", seed=M + N + K)
+    xg, wg, xsg, wsg = xq.to(gpu), wq.to(gpu), xs.to(gpu), ws.to(gpu)
+    y = kore_amd.gemm_a8w8(xg, wg, xsg, wsg)
+    assert bit_equal(kore_amd.gemm_a8w8(xg, wg, xsg, wsg), y)
+
+    def off(t, ld):  # the same rows at byte offset 1, row stride ld
+        buf = torch.empty(t.shape[0] * ld + 1, dtype=torch.uint8, device=gpu)
+        v = buf[1:].view(t.shape[0], ld)[:, :t.shape[1]]
+        v.copy_(t.view(torch.uint8))
+        return v.view(t.dtype) if t.dtype != torch.float8_e4m3fn else v.view(torch.float8_e4m3fn)
+
+    assert bit_equal(kore_amd.gemm_a8w8(off(xg, K + 3), off(wg, K + 5), xsg, wsg), y)
+    if kind == "int8":
+        Np, Kp = -(-N // 128) * 128, -(-K // 128) * 128
+        xp = torch.zeros(M, Kp, dtype=torch.int8, device=gpu)
+        xp[:, :K] = xg
+        wp = torch.zeros(Np, Kp, dtype=torch.int8, device=gpu)
+        wp[:N, :K] = wg
+        wsp = torch.ones(1, Np, device=gpu)
+        wsp[:, :N] = wsg
+        assert bit_equal(kore_amd.gemm_a8w8(xp, wp, xsg, wsp)[:, :N].contiguous(), y)
+    else:
+        xn, wn = xq.view(torch.uint8).clone(), wq.view(torch.uint8).clone()
+        xn[M - 1, K - 100] = 0x7F
+        wn[N - 1, K - 101] = 0xFF
+        yn = kore_amd.gemm_a8w8(xn.view(xq.dtype).to(gpu), wn.view(wq.dtype).to(gpu), xsg, wsg).isnan().cpu()
+        want = torch.zeros(M, N, dtype=torch.bool)
+        want[M - 1, :] = True
+        want[:, N - 1] = True
+        assert torch.equal(yn, want)
+    rows = torch.unique(torch.cat([torch.arange(0, M, max(1, M // 32)), torch.tensor([M - 1])]))
+    ref = matmul_a8w8_ref(xq[rows], wq, xs[rows], ws)
+    verdict(y.cpu()[rows], ref, "a8w8", kind, f"{kind} ragged {M}x{N}x{K}")
+    verdict(y.cpu()[rows], ref, "north_star", kind, f"{kind} ragged {M}x{N}x{K} (1e-2)")
+
+
 def test_a8w8_rejects_bad_inputs(gpu):
     xq, wq, xs, ws = W.a8w8_inputs(8, 128, 128, "fp8", "pertoken")
     with pytest.raises(ValueError):
