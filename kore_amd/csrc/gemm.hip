@@ -332,6 +332,24 @@ __global__ void __launch_bounds__(256) gemm_splitk_kernel(const TileParams p, fl
   }
 }
 
+// Activation (runtime code) of N values in place.
+template <int N>
+__device__ __forceinline__ void act8(int act, float (&v)[N]) {
+  auto fin = [&](auto act_tag) {
+    constexpr int ACT = decltype(act_tag)::value;
+#pragma unroll
+    for (int e = 0; e < N; ++e) v[e] = apply_act<ACT>(v[e]);
+  };
+  switch (act) {
+    case ACT_RELU: fin(std::integral_constant<int, ACT_RELU>{}); break;
+    case ACT_GELU: fin(std::integral_constant<int, ACT_GELU>{}); break;
+    case ACT_SILU: fin(std::integral_constant<int, ACT_SILU>{}); break;
+    case ACT_TANH: fin(std::integral_constant<int, ACT_TANH>{}); break;
+    case ACT_SIGMOID: fin(std::integral_constant<int, ACT_SIGMOID>{}); break;
+    default: break;
+  }
+}
+
 // Fixed-order sum of the split-K partials (slice 0, 1, ...), then bias, activation and
 // the store.  CW columns per thread: 4 with 16-byte partial loads when N % 4 == 0 -- the
 // loads of four slices go out before their adds, so their latencies overlap (a decode
@@ -379,19 +397,7 @@ __global__ void __launch_bounds__(256) splitk_reduce_kernel(const float* part, i
     for (int e = 0; e < CW; ++e)
       if (n + e < N) v[e] += Op::to_f32(bias[n + e]);
   }
-  auto fin = [&](auto act_tag) {
-    constexpr int ACT = decltype(act_tag)::value;
-#pragma unroll
-    for (int e = 0; e < CW; ++e) v[e] = apply_act<ACT>(v[e]);
-  };
-  switch (act) {
-    case ACT_RELU: fin(std::integral_constant<int, ACT_RELU>{}); break;
-    case ACT_GELU: fin(std::integral_constant<int, ACT_GELU>{}); break;
-    case ACT_SILU: fin(std::integral_constant<int, ACT_SILU>{}); break;
-    case ACT_TANH: fin(std::integral_constant<int, ACT_TANH>{}); break;
-    case ACT_SIGMOID: fin(std::integral_constant<int, ACT_SIGMOID>{}); break;
-    default: break;
-  }
+  act8(act, v);
   uint16_t* out = C + (int64_t)m * ldc + n;
   if (vec && n + CW <= N) {
     if constexpr (CW == 4)
@@ -403,6 +409,160 @@ __global__ void __launch_bounds__(256) splitk_reduce_kernel(const float* part, i
 #pragma unroll
     for (int e = 0; e < CW; ++e)
       if (n + e < N) out[e] = (uint16_t)(Op::pack2(v[e], 0.0f) & 0xffffu);
+  }
+}
+
+// ---------------------------------------------------------------------------------
+// Skinny kernel: M <= 128 against K-contiguous weights (decode), one launch.  The product
+// is bound by streaming W once; a workgroup owns BN = 16 NB columns and every row of A, and
+// its NW waves split the 64-wide K blocks (wave w takes blocks w, w + NW, ...), so W is
+// read once by N / BN workgroups and the K split needs no partials in memory.  Each wave
+// has a private ring of S stages (one K block: MT rows of A, BN rows of W, 128 bytes each)
+// filled by direct-to-LDS loads of 8 whole 128-byte rows, waits only for its own loads
+// (vmcnt) and meets the other waves once, to sum the partials in wave order through LDS
+// (bit-reproducible).  Rows of A past M lie outside the buffer resource (zeros, no
+// traffic); rows of W past N repeat row N - 1 and are never stored.  Rows may start at any
+// 2-byte address, and a K tail is a last block that ends at K with the columns it repeats
+// zeroed in both fragments.  16x16x32 MFMAs, W first: lane l holds column m = l % 16,
+// n = 4 (l / 16) + i, and the 16-byte chunks l / 16 and 4 + l / 16 of its row.
+// ---------------------------------------------------------------------------------
+template <int MT_, int NW_, int S_, int NB_>
+struct SkinnyCfg16 {
+  static constexpr int MT = MT_, NW = NW_, S = S_, NB = NB_, BN = 16 * NB, MB = MT / 16;
+  static constexpr int XQ = MT / 8, WQ = BN / 8, LPB = XQ + WQ;  // loads of a block
+  static constexpr int STAGE = (MT + BN) * kBK;                  // elements
+  static constexpr int BNP = BN + 4;                             // padded fp32 row of the reduction
+  static constexpr int RING = NW * S * STAGE * 2, RED = NW * MT * BNP * 4;
+  static constexpr int LDS = RING > RED ? RING : RED;
+  static_assert(LDS <= 160 * 1024 && S >= 1 && S <= 4 && LPB * (S - 1) <= 63, "LDS budget, vmcnt range");
+};
+
+template <typename T, typename C>
+__global__ void __launch_bounds__(C::NW * 64) gemm_skinny_kernel(const TileParams p) {
+  constexpr int MT = C::MT, NW = C::NW, S = C::S, MB = C::MB, NB = C::NB, BN = C::BN, LPB = C::LPB, BNP = C::BNP;
+  using Op = MfmaOp<T>;
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[C::LDS];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r = lane & 15, g = lane >> 4;
+  const int n0 = (int)blockIdx.x * BN, rows_b = min(BN, p.N - n0);
+  const int nk = (p.K + kBK - 1) / kBK;
+  const int cnt = nk > wave ? (nk - wave + NW - 1) / NW : 0;  // K blocks of this wave
+  const uint32_t abytes = (uint32_t)(((int64_t)(p.M - 1) * p.lda + p.K) * 2);
+  const __amdgpu_buffer_rsrc_t ra = make_rsrc(p.a, abytes);
+  const __amdgpu_buffer_rsrc_t rb =
+      make_rsrc(p.b + (int64_t)n0 * p.ldb, (uint32_t)(((int64_t)(rows_b - 1) * p.ldb + p.K) * 2));
+  // load q covers stage rows 8q .. 8q + 7; lane l fetches chunk (l % 8) ^ key(row)
+  uint32_t xoff[C::XQ], woff[C::WQ];
+#pragma unroll
+  for (int q = 0; q < C::XQ; ++q) {
+    const int row = 8 * q + (lane >> 3);
+    xoff[q] = row < p.M ? (uint32_t)(((int64_t)row * p.lda + 8 * ((lane & 7) ^ swz16(row))) * 2) : abytes;
+  }
+#pragma unroll
+  for (int q = 0; q < C::WQ; ++q) {
+    const int row = 8 * q + (lane >> 3);
+    woff[q] = (uint32_t)(((int64_t)min(row, rows_b - 1) * p.ldb + 8 * ((lane & 7) ^ swz16(row))) * 2);
+  }
+  uint16_t* ring = (uint16_t*)lds + wave * (S * C::STAGE);
+  auto issue = [&](int s, int j) {
+    const uint32_t ko = (uint32_t)min((wave + NW * j) * kBK, p.K - kBK) * 2u;
+    uint16_t* st = ring + s * C::STAGE;
+#pragma unroll
+    for (int q = 0; q < C::XQ; ++q) buf_lds16(ra, xoff[q], ko, st + q * 8 * kBK);
+#pragma unroll
+    for (int q = 0; q < C::WQ; ++q) buf_lds16_cp<kCpolNT>(rb, woff[q], ko, st + (MT + 8 * q) * kBK);  // read once
+  };
+  f32x4_t acc[MB][NB];
+#pragma unroll
+  for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) acc[mb][nb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  const int o0 = (g ^ swz16(r)) << 3, o1 = ((4 + g) ^ swz16(r)) << 3;  // key(16 b + r) = key(r)
+#pragma unroll
+  for (int s = 0; s < S; ++s)
+    if (s < cnt) issue(s, s);
+  for (int j0 = 0; j0 < cnt; j0 += S) {
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+      const int j = j0 + s;
+      if (j < cnt) {
+        const int later = min(S - 1, cnt - 1 - j);  // blocks issued after j
+        if (S >= 4 && later >= 3) wait_vmcnt<(S >= 4 ? 3 * LPB : 0)>();
+        else if (S >= 3 && later >= 2) wait_vmcnt<(S >= 3 ? 2 * LPB : 0)>();
+        else if (S >= 2 && later >= 1) wait_vmcnt<(S >= 2 ? LPB : 0)>();
+        else wait_vmcnt<0>();
+        const uint16_t* st = ring + s * C::STAGE;
+        u32x4_t xf[MB][2], wf[NB][2];
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb) {
+          const uint16_t* row = st + (mb * 16 + r) * kBK;
+          xf[mb][0] = *(const u32x4_t*)(row + o0);
+          xf[mb][1] = *(const u32x4_t*)(row + o1);
+        }
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) {
+          const uint16_t* row = st + (MT + nb * 16 + r) * kBK;
+          wf[nb][0] = *(const u32x4_t*)(row + o0);
+          wf[nb][1] = *(const u32x4_t*)(row + o1);
+        }
+        // the slot is free once its fragments are in registers
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        if (j + S < cnt) issue(s, j + S);
+        const int lead = 2 * (kBK * nk - p.K);
+        if (lead > 0 && wave + NW * j == nk - 1) {  // uniform: the columns a K tail repeats
+#pragma unroll
+          for (int mb = 0; mb < MB; ++mb) {
+            xf[mb][0] = zero_lead(xf[mb][0], lead - 16 * g);
+            xf[mb][1] = zero_lead(xf[mb][1], lead - 64 - 16 * g);
+          }
+#pragma unroll
+          for (int nb = 0; nb < NB; ++nb) {
+            wf[nb][0] = zero_lead(wf[nb][0], lead - 16 * g);
+            wf[nb][1] = zero_lead(wf[nb][1], lead - 64 - 16 * g);
+          }
+        }
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+          for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb) acc[mb][nb] = Op::mma16(wf[nb][h], xf[mb][h], acc[mb][nb]);
+      }
+    }
+  }
+  // cross-wave sum over the (now idle) ring, in wave order; bias, activation, store
+  wait_vmcnt<0>();
+  __syncthreads();
+  float* red = (float*)lds;
+#pragma unroll
+  for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb)
+      *(f32x4_t*)(red + (wave * MT + mb * 16 + r) * BNP + nb * 16 + 4 * g) = acc[mb][nb];
+  __syncthreads();
+  for (int it = tid; it < MT * BN / 8; it += NW * 64) {  // 8 consecutive columns per item
+    const int m = it / (BN / 8), gn = n0 + (it % (BN / 8)) * 8;
+    if (m >= p.M || gn >= p.N) continue;
+    const float* q = red + m * BNP + gn - n0;
+    float v[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = 0.0f;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      const f32x4_t a = *(const f32x4_t*)(q + w * MT * BNP), b = *(const f32x4_t*)(q + w * MT * BNP + 4);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        v[e] += a[e];
+        v[e + 4] += b[e];
+      }
+    }
+    if (p.bias != nullptr) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] += Op::to_f32(p.bias[min(gn + e, p.N - 1)]);
+    }
+    act8(p.act, v);
+    store_row8(p.c + (int64_t)m * p.ldc + gn, gn, p.N, p.vec_store != 0,
+               u32x4_t{Op::pack2(v[0], v[1]), Op::pack2(v[2], v[3]), Op::pack2(v[4], v[5]), Op::pack2(v[6], v[7])});
   }
 }
 
@@ -1208,6 +1368,76 @@ int launch_splitk(const GemmDesc& d, int splits, int kper, Ws& ws, hipStream_t s
   return rc;
 }
 
+template <typename T, typename C>
+int launch_skinny(const GemmDesc& d, hipStream_t stream) {
+  TileParams p{};
+  p.a = (const uint16_t*)d.a;
+  p.b = (const uint16_t*)d.b;
+  p.bias = (const uint16_t*)d.bias;
+  p.c = (uint16_t*)d.c;
+  p.M = (int)d.M;
+  p.N = (int)d.N;
+  p.K = (int)d.K;
+  p.lda = d.sam;
+  p.ldb = d.sbn;
+  p.ldc = d.scm;
+  p.act = d.act;
+  p.vec_store = (d.scm % 8 == 0) && aligned16(d.c);
+  hipLaunchKernelGGL((gemm_skinny_kernel<T, C>), dim3((unsigned)((d.N + C::BN - 1) / C::BN)), dim3(C::NW * 64), 0,
+                     stream, p);
+  return check_launch("gemm_skinny_kernel");
+}
+
+// Columns per workgroup (16 nb) of the skinny kernel, by its estimated time in us: a fixed
+// 2.5 us, and the longer of what a CU takes in for its workgroups, (M + 16 nb) rows of K, at
+// 60 (M <= 32) or 70 KB/us, and the weights' stream at 5.6 TB/s; rows off 16-byte alignment
+// cost half as much again.  Measured (bf16, one process, M = 1 / 16 / 64 / 128), nb = 1 | 2 | 4:
+//   4096 x 4096     6.6 7.4 11.3 18.0 | 6.5 9.7 14.7 21.6 | 12.1 13.8 20.1 33.0
+//   7168 x 2048     7.9 8.5 13.2 19.3 | 6.5 6.8  9.0 12.9 |  8.1  8.6 11.7 19.8
+//   14336 x 4096   23.2 25.8 45.7 69.2 | 23.0 24.6 33.8 46.0 | 19.2 19.3 25.0 35.0
+// and 4096 x 4095 (odd rows) 8.2 10.6 18.0 28.6 with nb = 1.
+struct SkinnyPick {
+  int nb;
+  double us;
+};
+inline SkinnyPick pick_skinny(const GemmDesc& d, bool aligned, int64_t cus) {
+  const double stream_us = (double)(d.N * d.K * 2) / 5.6e6;
+  SkinnyPick best{1, 1e300};
+  for (int nb : {1, 2, 4}) {
+    const int64_t wgs = (d.N + 16 * nb - 1) / (16 * nb);
+    const double intake_us = (double)((wgs + cus - 1) / cus * (d.M + 16 * nb) * d.K * 2) / (d.M <= 32 ? 60e3 : 70e3);
+    const double us = 2.5 + std::max(intake_us, stream_us) * (aligned ? 1.0 : 1.5);
+    if (us < best.us) best = {nb, us};
+  }
+  return best;
+}
+// Estimated time of the path an aligned problem (K % 64 == 0) takes otherwise.  32x128 ring
+// tiles: 3 us and 160 rows of K per round at 80 KB/us (bf16 200 x 4096 x 4096 19.4, 64 x
+// 14336 x 4096 20.3, 100 x 14336 x 4096 36.7, 128 x 8192 x 8192 34.5, 100 x 7168 x 2048 11.3
+// us).  With K split (few tiles): two launches, about 8 us back to back, and a share of the
+// weights' stream (32 x 4096 x 4096 11.3, 64 14.6, 128 19.6; 32 x 2048 x 7168 11.2, 64 12.6;
+// 64 x 1024 x 8192 10.0, 128 11.5 us).  Wider problems run the mid-size
+// tiles, which win from M = 33 on.
+inline double skinny_alternative_us(const GemmDesc& d, int64_t cus) {
+  const int64_t t32 = (d.M + 31) / 32 * ((d.N + 127) / 128);
+  if ((d.M + 127) / 128 * ((d.N + 127) / 128) >= 128) return d.M <= 32 ? 1e300 : 0.0;
+  if (d.K >= 1024 && t32 * 2 <= cus) return 8.0 + (double)(d.N * d.K * 2) / 5.6e6 * (d.M <= 32 ? 0.55 : d.M <= 64 ? 1.0 : 1.8);
+  return 3.0 + (double)((t32 + cus - 1) / cus * 160 * d.K * 2) / 80e3;
+}
+template <typename T>
+int launch_skinny_nb(const GemmDesc& d, int nb, hipStream_t st) {
+  // waves and stages per configuration: as much in flight as 160 KiB of LDS holds
+  auto pick = [&](auto c1, auto c2, auto c4) {
+    return nb == 1   ? launch_skinny<T, decltype(c1)>(d, st)
+           : nb == 2 ? launch_skinny<T, decltype(c2)>(d, st)
+                     : launch_skinny<T, decltype(c4)>(d, st);
+  };
+  if (d.M <= 16) return pick(SkinnyCfg16<16, 8, 4, 1>{}, SkinnyCfg16<16, 8, 3, 2>{}, SkinnyCfg16<16, 8, 2, 4>{});
+  if (d.M <= 32) return pick(SkinnyCfg16<32, 8, 3, 1>{}, SkinnyCfg16<32, 8, 2, 2>{}, SkinnyCfg16<32, 4, 3, 4>{});
+  if (d.M <= 64) return pick(SkinnyCfg16<64, 8, 2, 1>{}, SkinnyCfg16<64, 4, 3, 2>{}, SkinnyCfg16<64, 4, 2, 4>{});
+  return pick(SkinnyCfg16<128, 4, 2, 1>{}, SkinnyCfg16<128, 4, 2, 2>{}, SkinnyCfg16<128, 2, 3, 4>{});
+}
+
 // Tile shape for the direct-to-LDS engines.  Every CU runs one tile at a time, so a
 // launch costs about (rounds of tiles over the CUs) x (time of one tile); a tile's time
 // is its area over its engine's efficiency (the 256x256 pipelined engine is best;
@@ -1329,6 +1559,22 @@ int dispatch_typed(const GemmDesc& d, Ws& ws, hipStream_t stream) {
   const bool b_kc = d.sbk == 1 && d.sbn % 8 == 0 && aligned16(d.b) && d.sb % 8 == 0;
   const bool b_nc = d.sbn == 1 && d.sbk % 8 == 0 && aligned16(d.b) && d.sb % 8 == 0 && d.N % 8 == 0;
   const bool fits32 = d.M < (1ll << 31) && d.N < (1ll << 31) && d.K < (1ll << 31);
+  // M <= 128 against K-contiguous weights: the skinny kernel, unless the aligned paths below
+  // are estimated faster, or K < 512: 64x64 tiles then, which have no cross-wave sum to pay
+  // for (20 x 11000 x 256 4.8 us against 6.0).
+  if (d.batch == 1 && d.sak == 1 && d.sbk == 1 && d.M <= 128 && d.K >= 64 && fits32 &&
+      (d.sam >= d.K || d.M == 1) && (d.sbn >= d.K || d.N == 1) && d.M * d.sam * 2 + d.K * 2 < (1ll << 31) &&
+      64 * d.sbn * 2 + d.K * 2 < (1ll << 31)) {
+    const bool aligned = a_ok && b_kc && d.K % 64 == 0;
+    if (!aligned || d.K >= 512) {
+      const int64_t cus = device_cus();
+      const SkinnyPick k = pick_skinny(d, aligned, cus);
+      if (!aligned || k.us < skinny_alternative_us(d, cus)) {
+        if (ws.plan) return KORE_OK;
+        return launch_skinny_nb<T>(d, k.nb, stream);
+      }
+    }
+  }
   // M-contiguous A (a transposed view, e.g. dY^T of the backward) on the 256x256 buffer
   // engine, read in place through LDS transpose reads; smaller grids pack A instead.
   const bool a_mc = d.sam == 1 && d.sak % 8 == 0 && aligned16(d.a) && d.sa % 8 == 0 && d.M % 8 == 0 &&
@@ -1406,6 +1652,22 @@ int dispatch_typed(const GemmDesc& d, Ws& ws, hipStream_t stream) {
     const int64_t t32 = ((d.M + 31) / 32) * ((d.N + 127) / 128);
     if (d.batch == 1 && (b_kc ? buf_ok : buf_nc_ok) && d.K >= 1024 && t32 * 2 <= device_cus()) {
       const int nk = (int)(d.K / 64);
+      // One tile of 64 or 128 rows where 32-row tiles would read a large weight matrix two to
+      // four times (N-contiguous B, same process: 64 x 4096 x 4096 17.3 -> 14.6 us, 128 x
+      // 4096 x 4096 28.6 -> 19.6 us, with a slice of K for every other CU: twice the slices,
+      // 15.8 and 23.7 us, write and read more partials than they save).  32 rows stay for
+      // weights up to 24 MB (64 x 1024 x 8192 9.9 against 11.0 us) and where they leave at
+      // least five slices of K (64 x 2048 x 7168 13.1 against 14.5 us).
+      if (d.M > 32 && d.M <= 128 && t32 * 4 >= device_cus() && d.N * d.K * 2 > (24ll << 20)) {
+        const int64_t tn = (d.N + 127) / 128;
+        const int want = (int)std::max<int64_t>(1, std::min<int64_t>(device_cus() / 2 / tn, nk / 4));
+        const int per = (nk + want - 1) / want, splits = (nk + per - 1) / per;
+        if (d.M <= 64)
+          return b_kc ? launch_splitk<T, B_KC, 64, 128, 2, 2, 6>(d, splits, per * 64, ws, stream)
+                      : launch_splitk<T, B_NC, 64, 128, 2, 2, 6>(d, splits, per * 64, ws, stream);
+        return b_kc ? launch_splitk<T, B_KC, 128, 128, 2, 2, 4>(d, splits, per * 64, ws, stream)
+                    : launch_splitk<T, B_NC, 128, 128, 2, 2, 4>(d, splits, per * 64, ws, stream);
+      }
       const int want = (int)std::min<int64_t>(device_cus() / t32, nk / 4);
       const int per = (nk + want - 1) / want, splits = (nk + per - 1) / per;
       return b_kc ? launch_splitk<T, B_KC, 32, 128, 1, 4, 7>(d, splits, per * 64, ws, stream)

@@ -265,6 +265,11 @@ struct Stager {
 __device__ __forceinline__ void store_row8(uint16_t* dst, int gn, int N, bool vec, u32x4_t v) {
   if (vec && gn + 8 <= N) {
     *(u32x4_t*)dst = v;
+  } else if (gn + 8 <= N) {
+    // one 16-byte store at any alignment (eight 2-byte ones before: 8 x 512 x 513 x 512
+    // batched 12.6 -> 9.3 us).  A branch of its own: without the aligned store above, tiles
+    // with N % 8 == 0 compiled to code 2-5% slower (168 x 320 x 1816 24.3 -> 25.5 us).
+    __builtin_memcpy(dst, &v, 16);
   } else {
 #pragma unroll
     for (int e = 0; e < 8; ++e)

@@ -732,3 +732,45 @@ def test_workspace_paths_under_graph_capture(gpu):
         assert torch.equal(y_split, e_split), f"split-K replay {r} on a second stream"
         assert torch.equal(eager, e_split), f"eager split-K beside replay {r}"
     del graph
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,N,K", [(1, 1, 64), (16, 17, 65), (17, 300, 900), (33, 823, 1984), (64, 4096, 512),
+                                   (64, 513, 127), (65, 1000, 1001), (128, 4097, 129), (100, 7168, 2048),
+                                   (5, 14339, 640), (128, 16, 4095)])
+def test_gemm_skinny(gpu, dtype, M, N, K):
+    """M <= 128 against K-contiguous weights (the skinny kernel): row, column and K tails,
+    16-, 32- and 64-column workgroups, bias and activation, rows at odd element offsets (the
+    same bits as aligned rows when both take this kernel), and an infinity in a column that
+    the tail block repeats, which must reach exactly its own row and column."""
+    g = torch.Generator().manual_seed(M + N + K)
+    a = (torch.randn((M, K), generator=g) / K ** 0.5).to(dtype)
+    w = torch.randn((N, K), generator=g).to(dtype)
+    bias = torch.randn((N,), generator=g).to(dtype)
+    ag, wg, bg = a.to(gpu), w.to(gpu), bias.to(gpu)
+    name = "bf16" if dtype == torch.bfloat16 else "fp16"
+    for act in ("none", "gelu"):
+        out = kore_amd.gemm_fused(ag, wg.t(), bg, act)
+        assert bit_equal(kore_amd.gemm_fused(ag, wg.t(), bg, act), out)
+        pair_only(out.cpu(), gemm_fusion_ref(a, w.t(), bias, act), name, f"skinny {M}x{N}x{K} {act}")
+
+    def odd(t, ld):  # the same rows one element off the allocation, row stride ld
+        buf = torch.full((t.shape[0] * ld + 1,), float("nan"), dtype=dtype, device=gpu)
+        v = buf[1:].view(t.shape[0], ld)[:, :t.shape[1]]
+        v.copy_(t)
+        return v
+
+    o1 = kore_amd.gemm_fused(odd(ag, K + 1), odd(wg, K + 3).t(), bg, "none")
+    o2 = kore_amd.gemm_fused(odd(ag, K + 2), odd(wg, K + 1).t(), bg, "none")
+    assert bit_equal(o1, o2)
+    pair_only(o1.cpu(), gemm_fusion_ref(a, w.t(), bias, "none"), name, f"skinny {M}x{N}x{K} odd rows")
+    if K > 100:
+        a2, w2 = a.float().abs().to(dtype), w.float().abs().to(dtype) + 1
+        a2[M - 1, K - 60] = float("inf")
+        w2[N - 1, K - 61] = float("inf")
+        got = kore_amd.gemm_fused(odd(a2.to(gpu), K), odd(w2.to(gpu), K).t(), None, "none").cpu()
+        want = torch.zeros(M, N, dtype=torch.bool)
+        want[M - 1, :] = True
+        want[:, N - 1] = True
+        nz = (a2[:, K - 61] != 0)  # inf * 0 is NaN in the reference too
+        assert torch.equal(got.isinf()[nz], want[nz])
