@@ -18,11 +18,11 @@
 //  4. moe_combine_kernel: out[t] = bf16(sum_k Yw[t*topk + k]) in fixed k order over
 //     the slots whose id is in [0, E): no atomics, bit-reproducible.
 // Grids are sized for the worst case (every expert adds < 1 block of padding) and
-// blocks past the real end exit after reading offsets[E].  Up to 128 slots per expert
-// (decode and small batches) blocks are 32 or 128 rows and both GEMMs stream the expert
+// blocks past the real end exit after reading offsets[E].  Up to about 112 slots per expert
+// (decode and small batches, see moe_block_rows) blocks are 32 or 128 rows and both GEMMs stream the expert
 // weights once per block on a direct-to-LDS ring with non-temporal loads
 // (moe_decode_kernel); padding rows of a block are zero-filled by the buffer range
-// check at no memory cost.  Beyond 128 slots per expert: 256-row prefill tiles.
+// check at no memory cost.  Beyond: 256-row prefill tiles.
 #include "../../include/kore_amd.h"
 #include "kore_common.hpp"
 #include "tile_engine.hpp"
@@ -469,22 +469,29 @@ __global__ void __launch_bounds__(64 * NWV)
   E eng;
   // A: gathered token rows (gate_up, plain) or the H planes of this block (down)
   if constexpr (MODE != MOE_DOWN) {
-    eng.ra = make_rsrc(p.x, (uint32_t)((int64_t)p.T * p.ldx * 2));
+    // A padding row's offset lies at the end of the resource (as in moe_decode_kernel): its
+    // loads return zeros with no memory traffic, and it is never stored.  Against re-reading
+    // token 0 (gate_up) and the unused H rows (down), one process: E=8 top-2 D=4096 I=14336
+    // T=4096 3.58 -> 3.45 ms, T=700 903 -> 863 us; E=32 top-8 D=1024 I=768 T=512 on 256-row
+    // blocks 74.8 -> 69.3 us.  The plain grouped GEMM did not change.
+    const uint32_t bytes = (uint32_t)((int64_t)p.T * p.ldx * 2);
+    eng.ra = make_rsrc(p.x, bytes);
 #pragma unroll
     for (int j = 0; j < E::AJ; ++j) {
       const int r = E::a_row(wave, lane, j);
       const int sl = p.sorted[pos0 + r];
-      const int64_t row = (sl < p.S) ? sl / p.topk : 0;  // padding rows read token 0; never stored
-      eng.a_voff[j] = (uint32_t)((row * p.ldx + 8 * E::chunk(r, lane)) * 2);
+      eng.a_voff[j] = sl < p.S ? (uint32_t)(((int64_t)(sl / p.topk) * p.ldx + 8 * E::chunk(r, lane)) * 2) : bytes;
     }
   } else {
-    const int64_t tile_bytes = (int64_t)BM * p.ldx * 2;
-    eng.ra = make_rsrc(p.x + (int64_t)pos0 * p.ldx, (uint32_t)tile_bytes);
-    eng.ra2 = make_rsrc(p.h_lo + (int64_t)pos0 * p.ldx, (uint32_t)tile_bytes);
+    const uint32_t tile_bytes = (uint32_t)((int64_t)BM * p.ldx * 2);
+    eng.ra = make_rsrc(p.x + (int64_t)pos0 * p.ldx, tile_bytes);
+    eng.ra2 = make_rsrc(p.h_lo + (int64_t)pos0 * p.ldx, tile_bytes);
+    const bool last = pos0 / p.abm == p.offsets[e + 1] / p.abm - 1;  // only an expert's last block has padding
 #pragma unroll
     for (int j = 0; j < E::AJ; ++j) {
       const int r = E::a_row(wave, lane, j);
-      eng.a_voff[j] = (uint32_t)(((int64_t)r * p.ldx + 8 * E::chunk(r, lane)) * 2);
+      const bool pad = last && p.sorted[pos0 + r] >= p.S;
+      eng.a_voff[j] = pad ? tile_bytes : (uint32_t)(((int64_t)r * p.ldx + 8 * E::chunk(r, lane)) * 2);
     }
   }
   // B: interleaved gate/up rows of w1[e] (gate_up) or consecutive rows of w[e]
@@ -651,10 +658,21 @@ inline int64_t align_capacity(int64_t S, int64_t E, int64_t block) {
 }
 
 // Block size of the fused MoE GEMMs: skinny blocks when experts see few rows.
-// Up to 16 slots per expert on average: 32-row blocks; up to 128: 128-row blocks, so
+// Up to 16 slots per expert on average: 32-row blocks; up to 112: 128-row blocks, so
 // nearly every expert's weights are streamed once (padding rows cost MFMA cycles, which
-// are idle on these weight-bound shapes, but no memory traffic); beyond: 256.
-inline int moe_block_rows(int64_t S, int64_t E) { return S <= 16 * E ? 32 : S <= 128 * E ? 128 : 256; }
+// are idle on these weight-bound shapes, but no memory traffic); beyond: 256.  At a mean of
+// 128 half of the experts spill into a second 128-row block and stream their weights
+// twice: 256-row blocks there measured, in one process, E=32 top-8 D=1024 I=768 T=512 98.5
+// -> 69.3 us, E=8 top-2 D=4096 I=14336 T=512 1021 -> 832 us (a mean of 100: 61.4 against
+// 67.3, 648 against 788).  Where one block per expert leaves the CUs half empty (E * I / 128
+// below 128) the time is one tile's latency, so the smaller blocks last longer: E=8 top-2
+// D=1024 I=1408, T=200 / 300 / 512 / 800: 32 rows 47.7 / 61.4 / 76.1 / 121, 128 rows 55.5 /
+// 58.0 / 64.6 / 66.1, 256 rows 67.3 / 68.1 / 69.3 / 70.9 us.
+inline int moe_block_rows(int64_t S, int64_t E, int64_t I) {
+  const bool sparse = E * (I / 128) < 128;
+  if (S <= (sparse ? 52 : 16) * E) return 32;
+  return S <= (sparse ? 208 : 112) * E ? 128 : 256;
+}
 
 struct MoeWorkspace {
   int32_t* offsets;
@@ -668,7 +686,7 @@ struct MoeWorkspace {
 
 inline MoeWorkspace carve(void* base, int64_t T, int64_t topk, int64_t E, int64_t D, int64_t I) {
   const int64_t S = T * topk;
-  const int BM = moe_block_rows(S, E);
+  const int BM = moe_block_rows(S, E, I);
   const int64_t cap = align_capacity(S, E, BM);
   MoeWorkspace w{};
   size_t off = 0;
@@ -803,7 +821,7 @@ extern "C" int kore_fused_moe(const void* hidden, int64_t ldh, const void* w1, c
   if (workspace_bytes < ws.bytes)
     return set_error(KORE_EWORKSPACE, "fused_moe: workspace %zu bytes < required %zu", workspace_bytes, ws.bytes);
   hipStream_t st = (hipStream_t)stream;
-  const int BM = moe_block_rows(S, E);
+  const int BM = moe_block_rows(S, E, I);
   const int64_t cap = align_capacity(S, E, BM);
   int rc = launch_align(topk_ids, S, E, BM, ws.offsets, ws.sorted, ws.block_expert, cap, st);
   if (rc) return rc;
@@ -833,9 +851,22 @@ extern "C" int kore_fused_moe(const void* hidden, int64_t ldh, const void* w1, c
   // offset) below 4 GiB and K % 64 == 0
   const bool buf_ok = T * ldh * 2 + 4 * D < (1ll << 32) && 2 * I * D * 2 < (1ll << 32) && D % 64 == 0 &&
                       I % 64 == 0 && !g_force_generic;
+  // Stages of the decode rings: what one workgroup keeps in flight, against two workgroups
+  // per CU whose prologues and epilogues overlap.  With enough live tiles (one block per
+  // expert that can receive a slot) two fit: 32 rows, 4 against 7 stages, E=64 top-4 D=2048
+  // I=1024 T=200 181 -> 167 us, E=8 top-2 D=4096 I=14336 T=64 474 -> 462, E=32 top-8 D=1024
+  // I=768 T=64 44.6 -> 42.7; with few tiles the deep ring wins (the last at T=1: 25.6 against
+  // 30.4 us).  128 rows, 3 against 2 stages where no CU has two tiles: E=8 top-2 D=1024
+  // I=1408 T=400 60.2 -> 52.7 us.  Down, 3 against 6 stages: E=64 as above, T=200 181 -> 176 us.
+  const int64_t live = std::min(E, S), cus = device_cus();
+  const bool two_gu = live * (I / 64) * 4 >= 5 * cus;
+  const bool one_gu = live * (I / 64) <= cus && S <= 112 * E;  // beyond, many experts have two blocks
+  const bool two_dn = live * (D / 128) * 4 >= 5 * cus;
   // 128-row blocks without the buffer engine run 32-row tiles (four per aligned block)
-  rc = (BM == 32 && buf_ok) ? launch_moe_decode<MOE_GATEUP, 128, 7>(p, cap, st)
-       : (BM == 128 && buf_ok) ? launch_moe_decode<MOE_GATEUP, 128, 2, 128>(p, cap, st)
+  rc = (BM == 32 && buf_ok) ? (two_gu ? launch_moe_decode<MOE_GATEUP, 128, 4>(p, cap, st)
+                                      : launch_moe_decode<MOE_GATEUP, 128, 7>(p, cap, st))
+       : (BM == 128 && buf_ok) ? (one_gu ? launch_moe_decode<MOE_GATEUP, 128, 3, 128>(p, cap, st)
+                                         : launch_moe_decode<MOE_GATEUP, 128, 2, 128>(p, cap, st))
        : (BM <= 128) ? launch_moe_gemm<MOE_GATEUP, 32, 256, 1, 4>(p, cap, st)
        : buf_ok   ? launch_moe_buf<MOE_GATEUP, 256, 256>(p, cap, st)
                   : launch_moe_gemm<MOE_GATEUP, 256, 256, 2, 2>(p, cap, st);
@@ -851,7 +882,7 @@ extern "C" int kore_fused_moe(const void* hidden, int64_t ldh, const void* w1, c
   // two A planes double the A tile: prefill runs 128-row tiles (halves of a 256-row
   // aligned block) to stay inside the 160 KiB LDS budget.
   if (BM == 32 && buf_ok) {
-    rc = launch_moe_decode<MOE_DOWN, 128, 6>(p, cap, st);
+    rc = two_dn ? launch_moe_decode<MOE_DOWN, 128, 3>(p, cap, st) : launch_moe_decode<MOE_DOWN, 128, 6>(p, cap, st);
   } else if (BM == 128 && buf_ok) {
     rc = launch_moe_decode<MOE_DOWN, 128, 3, 128>(p, cap, st);
   } else if (BM <= 128) {

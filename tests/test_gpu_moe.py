@@ -100,6 +100,23 @@ def test_fused_moe_128row_blocks(gpu, T, E, topk, D, I):
     verdict(out, ref, "north_star", "bf16", f"128-row blocks T{T} (1e-2)")
 
 
+@pytest.mark.parametrize("T,E,topk,D,I", [(416, 8, 1, 256, 256), (417, 8, 1, 256, 256), (1664, 8, 1, 256, 256),
+                                          (1665, 8, 1, 256, 384), (448, 32, 8, 256, 512), (449, 32, 8, 256, 512),
+                                          (16, 64, 4, 384, 640), (100, 64, 8, 256, 512)])
+def test_fused_moe_block_choice(gpu, T, E, topk, D, I):
+    """Both sides of the block-size and stage-count rules: 32 / 128 / 256 rows where one block
+    per expert leaves the CUs half empty (E * I / 128 < 128: 52 and 208 slots per expert) and
+    where it does not (16 and 112), decode rings with one and two workgroups per CU, and
+    256-row blocks whose padding rows lie outside the buffer resources.  Invalid ids add
+    padding that no expert owns."""
+    hidden, w1, w2, tw, ti = W.moe_inputs(T, E, topk, D, I, seed=T + 3, wscale=0.05)
+    for ids in (ti, torch.where(torch.arange(T)[:, None] % 7 == 3, torch.full_like(ti, -1), ti)):
+        out = kore_amd.fused_moe(*[t.to(gpu) for t in (hidden, w1, w2, tw, ids)])
+        ref = moe_ref(hidden, w1, w2, tw, ids)
+        verdict(out, ref, "fused_moe", "bf16", f"block choice T{T} E{E} k{topk} D{D} I{I}")
+        verdict(out, ref, "north_star", "bf16", f"block choice T{T} (1e-2)")
+
+
 def test_fused_moe_decode_config(gpu):
     """BASELINE config 5 decode variant: T=64, E=8, top-2, D=4096, I=14336, weights
     N(0,1)*0.02, plain softmax/top-2/renorm router."""
