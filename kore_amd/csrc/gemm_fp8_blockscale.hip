@@ -37,6 +37,7 @@ struct Fp8Params {
   const int32_t* sorted;
   const int32_t* block_expert;
   int64_t w_estride, ws_estride;
+  int rot_mask;  // skinny kernel: mask of the workgroup's first K block
 };
 
 constexpr int kFp8GroupM = 4;
@@ -1216,21 +1217,25 @@ inline bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 // in the reference oracle.  The per-wave partials are summed through LDS in wave
 // order (fixed order: bit-reproducible) and written as bf16.
 // ------------------------------------------------------------------------------
-template <int MT, int NW, int S, int MODE = Q_BLOCK_FP8, int NB_ = 2>
+template <int MT, int NW, int S, int MODE = Q_BLOCK_FP8, int NB_ = 2, bool PRE_ = false>
 struct SkinnyCfg {
+  // PRE (block scales): all scales of the workgroup are copied to LDS first, xs as
+  // [K block][MT] and ws as [K block], instead of travelling with each block's operands
+  static constexpr bool PRE = PRE_;
   static constexpr int MT_ = MT, NW_ = NW, S_ = S, MODE_ = MODE;
   static constexpr bool ROW = MODE != Q_BLOCK_FP8;          // scales in the epilogue only
   static constexpr int NB = NB_, BN = 16 * NB, MB = MT / 16;  // 16-column blocks per workgroup
   static constexpr int XQ = MT / 8, WQ = BN / 8;          // 8-row DMA loads per block
-  static constexpr int SQ = ROW ? 0 : (MT + 63) / 64;      // 64-row activation-scale loads
-  static constexpr int LPB = XQ + WQ + (ROW ? 0 : SQ + 1); // DMA instructions per block
+  static constexpr int SQ = ROW || PRE ? 0 : (MT + 63) / 64;      // 64-row activation-scale loads
+  static constexpr int LPB = XQ + WQ + (ROW || PRE ? 0 : SQ + 1); // DMA instructions per block
   static constexpr int XS_OFF = (MT + BN) * 128;           // xs[m] of the block (fp32)
   static constexpr int WS_OFF = XS_OFF + SQ * 256;         // ws of the block (64 copies)
-  static constexpr int STAGE = WS_OFF + (ROW ? 0 : 256);   // bytes
+  static constexpr int STAGE = WS_OFF + (ROW || PRE ? 0 : 256);   // bytes
   static constexpr int RING = NW * S * STAGE;
   static constexpr int BNP = BN + 4;                       // padded fp32 row of the reduction
   static constexpr int RED = NW * MT * BNP * 4;
-  static constexpr int LDS = RING > RED ? RING : RED;
+  static constexpr int PRE_USE = PRE ? 64 : 0;  // K blocks whose scales fit beside the ring
+  static constexpr int LDS = (RING > RED ? RING : RED) + PRE_USE * (MT + 1) * 4;
   static_assert(LDS <= 160 * 1024, "LDS budget");
   static_assert(S >= 1 && S <= 3 && LPB * (S - 1) <= 63, "vmcnt range");
 };
@@ -1247,7 +1252,7 @@ __global__ void __launch_bounds__(C::NW_ * 64)
     gemm_fp8_skinny_kernel(const Fp8Params p) {
   constexpr int MT = C::MT_, NW = C::NW_, S = C::S_, MB = C::MB, NB = C::NB, BN = C::BN;
   constexpr int XQ = C::XQ, WQ = C::WQ, SQ = C::SQ, LPB = C::LPB, STAGE = C::STAGE, BNP = C::BNP;
-  constexpr bool ROW = C::ROW, I8 = C::MODE_ == Q_ROW_I8;
+  constexpr bool ROW = C::ROW, PRE = C::PRE, I8 = C::MODE_ == Q_ROW_I8;
   using AccT = std::conditional_t<I8, i32x4_t, f32x4_t>;
   __shared__ __attribute__((aligned(1024))) uint8_t lds[C::LDS];
 
@@ -1290,16 +1295,19 @@ __global__ void __launch_bounds__(C::NW_ * 64)
   const int k0 = sk_key(r);  // key(R + r) = (key(r) ^ (R / 8)) & 7 for R % 16 == 0
 
   // issue the loads of block j into stage slot s (DMA operands, then scales)
+  // K blocks are taken from a start of the workgroup's own (rot < nk), see skinny_rot_mask
+  const int rot = (int)((blockIdx.x >> 3) * 5) & p.rot_mask;
+  auto kb_of = [&](int j) { const int k = wave + NW * j + rot; return k >= nk ? k - nk : k; };
   auto issue = [&](int s, int j) {
     // the last block of a K tail ends at K
-    const uint32_t ko = RAG ? (uint32_t)min((wave + NW * j) * 128, p.K - 128) : (uint32_t)(wave + NW * j) * 128u;
+    const uint32_t ko = RAG ? (uint32_t)min(kb_of(j) * 128, p.K - 128) : (uint32_t)kb_of(j) * 128u;
     uint8_t* st = ring + s * STAGE;
 #pragma unroll
     for (int q = 0; q < XQ; ++q) buf_lds(rx, xoff[q], ko, st + q * 1024, 16);
 #pragma unroll
     for (int q = 0; q < WQ; ++q) buf_lds<kCpolNT>(rw, woff[q], ko, st + MT * 128 + q * 1024, 16);  // W: read once
-    if constexpr (!ROW) {
-      const uint32_t kb = (uint32_t)(wave + NW * j);
+    if constexpr (!ROW && !PRE) {
+      const uint32_t kb = (uint32_t)kb_of(j);
 #pragma unroll
       for (int q = 0; q < SQ; ++q) buf_lds(rxs, xsoff[q], kb * (uint32_t)(p.xs_k * 4), st + C::XS_OFF + q * 256, 4);
       buf_lds(rws, 0u, ws_base + kb * (uint32_t)(p.ws_k * 4), st + C::WS_OFF, 4);
@@ -1315,6 +1323,26 @@ __global__ void __launch_bounds__(C::NW_ * 64)
 #pragma unroll
   for (int s = 0; s < S; ++s)
     if (s < cnt) issue(s, s);
+  float* xsl = (float*)(lds + (C::RING > C::RED ? C::RING : C::RED));
+  float* wsl = xsl + C::PRE_USE * MT;
+  if constexpr (PRE) {
+    // four K blocks of a row per item; lanes walk along the contiguous direction
+    const int nk4 = (nk + 3) / 4, items = p.M * nk4;
+    const bool kc = p.xs_k == 1;
+    for (int it = tid; it < items; it += NW * 64) {
+      const int m = kc ? it / nk4 : it % p.M, kb = (kc ? it % nk4 : it / p.M) * 4;
+      const float* q = p.xs + (int64_t)m * p.xs_m + (int64_t)kb * p.xs_k;
+      float v[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = kb + e < nk ? q[e * p.xs_k] : 0.0f;
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (kb + e < nk) xsl[(kb + e) * MT + m] = v[e];
+    }
+    for (int kb = tid; kb < nk; kb += NW * 64) wsl[kb] = p.ws[(int64_t)(n0 / 128) * p.ws_n + (int64_t)kb * p.ws_k];
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    exec_barrier();
+  }
   for (int j0 = 0; j0 < cnt; j0 += S) {
 #pragma unroll
     for (int s = 0; s < S; ++s) {
@@ -1341,7 +1369,7 @@ __global__ void __launch_bounds__(C::NW_ * 64)
           const int key = (k0 ^ (2 * nb)) & 7;
           u32x4_t lo = *(const u32x4_t*)(row + ((g ^ key) << 4));
           u32x4_t hi = *(const u32x4_t*)(row + (((4 + g) ^ key) << 4));
-          if (RAG && wave + NW * j == nk - 1) {  // uniform: the columns a K tail repeats
+          if (RAG && kb_of(j) == nk - 1) {  // uniform: the columns a K tail repeats
             const int lead = 128 * nk - p.K;
             lo = zero_lead(lo, lead - 16 * g);
             hi = zero_lead(hi, lead - 64 - 16 * g);
@@ -1349,7 +1377,12 @@ __global__ void __launch_bounds__(C::NW_ * 64)
           wf[nb] = i32x8_t{(int)lo[0], (int)lo[1], (int)lo[2], (int)lo[3], (int)hi[0], (int)hi[1], (int)hi[2], (int)hi[3]};
         }
         float sc[MB];
-        if constexpr (!ROW) {
+        if constexpr (PRE) {
+          const float wsv = wsl[kb_of(j)];
+          const float* xk = xsl + kb_of(j) * MT + r;
+#pragma unroll
+          for (int mb = 0; mb < MB; ++mb) sc[mb] = xk[mb * 16] * wsv;  // (rows past M: never stored)
+        } else if constexpr (!ROW) {
           const float wsv = *(const float*)(st + C::WS_OFF);
 #pragma unroll
           for (int mb = 0; mb < MB; ++mb) sc[mb] = *(const float*)(st + C::XS_OFF + (mb * 16 + r) * 4) * wsv;
@@ -1428,8 +1461,23 @@ __global__ void __launch_bounds__(C::NW_ * 64)
   }
 }
 
+// Mask that keeps a skinny workgroup's first K block below nk; 0: in order.  Starts of their
+// own spread the workgroups over the memory channels: with every one at the same block, rows
+// a power of two apart crowd a few (M=1 7168 x 8192 11.2 -> 9.2 us, 14336 x 4096 11.5 ->
+// 10.8, M=64 3072 x 3840 8.6 -> 7.8).  One round of M <= 16 and up to 32 blocks measured
+// faster in order (M=1 7168 x 4096 5.3 against 5.6 us), and so did a few workgroups, which
+// fetch each line of X once for all (M=64 512 x 4096 7.1 against 8.2 us).
+inline int skinny_rot_mask(int mt, int nk, int64_t wgs) {
+  if (wgs < 96) return 0;
+  if (nk <= 32 && mt <= 16 && wgs <= device_cus()) return 0;
+  int m = 1;
+  while (2 * m <= nk) m *= 2;
+  return m - 1;
+}
+
 template <typename C, bool RAG = false>
-int launch_fp8_skinny(const Fp8Params& p, hipStream_t st) {
+int launch_fp8_skinny(Fp8Params p, hipStream_t st) {
+  p.rot_mask = skinny_rot_mask(C::MT_, (p.K + 127) / 128, (p.N + C::BN - 1) / C::BN);
   const dim3 grid((unsigned)((p.N + C::BN - 1) / C::BN)), block(C::NW_ * 64);
   hipLaunchKernelGGL((gemm_fp8_skinny_kernel<C, RAG>), grid, block, 0, st, p);
   return check_launch("gemm_fp8_skinny_kernel");
@@ -1482,8 +1530,26 @@ extern "C" int kore_gemm_a8w8_blockscale(const void* xq, int64_t ldx, const void
     // weight streaming: every CU reads its own 32 columns of W once
     hipStream_t st = (hipStream_t)stream;
     if (M <= 16) return launch_fp8_skinny<SkinnyCfg<16, 8, 3>>(p, st);
-    if (M <= 32) return launch_fp8_skinny<SkinnyCfg<32, 8, 2>>(p, st);
-    if (M <= 64) return launch_fp8_skinny<SkinnyCfg<64, 4, 3>>(p, st);
+    // Scales copied to LDS up front (up to 64 K blocks): per block they are a gather of MT
+    // cache lines, as many as the X rows themselves.  Without them in the ring, and with one
+    // stage per wave, six or seven waves fit where M = 128 had two: a wave's wait for its
+    // block then hides under the others' work.  M = 128, one process: 7168 x 4096 17.0 ->
+    // 14.7 us (M = 65: 15.4 -> 12.0), 14336 x 4096 32.7 -> 28.6; with 16-column workgroups
+    // where they fit one round, 4096 x 4096 16.9 -> 12.2, 3072 x 3840 15.0 -> 9.1, and
+    // below, M = 64 4096 x 4096 10.1 -> 8.6, M = 32 7.8 -> 6.7 us.
+    // Fewer than 16 K blocks or, up to M = 64, few workgroups (N < 2048) do not repay the copy
+    // (M = 65 4480 x 1152 6.4 against 6.8 us, M = 64 512 x 8192 10.6 against 13.1).
+    const bool pre = K / 128 >= 16 && K / 128 <= 64 && (M > 64 || N >= 2048);
+    const bool narrow = pre && N <= 16ll * device_cus();
+    if (M <= 32)
+      return narrow ? launch_fp8_skinny<SkinnyCfg<32, 8, 3, Q_BLOCK_FP8, 1, true>>(p, st)
+                           : launch_fp8_skinny<SkinnyCfg<32, 8, 2>>(p, st);
+    if (M <= 64)
+      return narrow ? launch_fp8_skinny<SkinnyCfg<64, 7, 2, Q_BLOCK_FP8, 1, true>>(p, st)
+                           : launch_fp8_skinny<SkinnyCfg<64, 4, 3>>(p, st);
+    if (pre)
+      return narrow ? launch_fp8_skinny<SkinnyCfg<128, 7, 1, Q_BLOCK_FP8, 1, true>>(p, st)
+                    : launch_fp8_skinny<SkinnyCfg<128, 6, 1, Q_BLOCK_FP8, 2, true>>(p, st);
     return launch_fp8_skinny<SkinnyCfg<128, 2, 2>>(p, st);  // 2 stages: 16.8 us at M=128 (3: 19.7)
   }
   if (pipe_ok) {

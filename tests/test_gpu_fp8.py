@@ -200,3 +200,20 @@ def test_fp8_skinny_layouts(gpu, M):
     padw[:, :K] = wq
     assert bit_equal(_run(gpu, pad[:, :K], padw[:, :K], xs, ws), base)
     assert bit_equal(_run(gpu, xq, wq, xs * 2, ws), base * 2)
+
+
+@pytest.mark.parametrize("M", [17, 32, 33, 64, 65, 100, 128])
+@pytest.mark.parametrize("N,K", [(128, 128), (384, 896), (4096, 1024), (4224, 640), (256, 8192), (4224, 8192),
+                                 (128, 8320)])
+def test_fp8_skinny_scales_in_lds(gpu, M, N, K):
+    """17 <= M <= 128 with the scales copied to LDS first (up to 64 K blocks; 65 keep them in
+    the operand stream), in 16- and 32-column workgroups (N to 4096 and beyond), fewer K
+    blocks than waves, and K orders that start at the workgroup's own block.  Column-major
+    scales give the same bits; reruns too."""
+    xq, wq, xs, ws = W.fp8_inputs(M, N, K, seed=M + N + K, scale=0.2)
+    out = _run(gpu, xq, wq, xs, ws)
+    ref = matmul_blockscale_ref(xq, wq, xs, ws)
+    verdict(out, ref, "blockscale", "fp8", f"{M}x{N}x{K}")
+    verdict(out, ref, "blockscale_genv", "fp8", f"{M}x{N}x{K} (1e-2)")
+    assert bit_equal(out, _run(gpu, xq, wq, xs, ws))
+    assert bit_equal(out, _run(gpu, xq, wq, xs.t().contiguous().t(), ws.t().contiguous().t()))
