@@ -413,7 +413,7 @@ __global__ void __launch_bounds__(256) splitk_reduce_kernel(const float* part, i
 }
 
 // ---------------------------------------------------------------------------------
-// Skinny kernel: M <= 128 against K-contiguous weights (decode), one launch.  The product
+// Skinny kernel: M <= 128 (decode), weights K-contiguous or N-contiguous, one launch.  The product
 // is bound by streaming W once; a workgroup owns BN = 16 NB columns and every row of A, and
 // its NW waves split the 64-wide K blocks (wave w takes blocks w, w + NW, ...), so W is
 // read once by N / BN workgroups and the K split needs no partials in memory.  Each wave
@@ -422,9 +422,11 @@ __global__ void __launch_bounds__(256) splitk_reduce_kernel(const float* part, i
 // (vmcnt) and meets the other waves once, to sum the partials in wave order through LDS
 // (bit-reproducible).  Rows of A past M lie outside the buffer resource (zeros, no
 // traffic); rows of W past N repeat row N - 1 and are never stored.  Rows may start at any
-// 2-byte address, and a K tail is a last block that ends at K with the columns it repeats
+// 2-byte address, and N be any number; a K tail is a last block that ends at K with the columns it repeats
 // zeroed in both fragments.  16x16x32 MFMAs, W first: lane l holds column m = l % 16,
-// n = 4 (l / 16) + i, and the 16-byte chunks l / 16 and 4 + l / 16 of its row.
+// n = 4 (l / 16) + i, and the 16-byte chunks l / 16 and 4 + l / 16 of its row.  N-contiguous
+// W: a stage holds 64 K-rows of BN columns as they are in memory, read back through LDS
+// transpose reads, which give each lane the same eight K values of one column.
 // ---------------------------------------------------------------------------------
 template <int MT_, int NW_, int S_, int NB_>
 struct SkinnyCfg16 {
@@ -437,20 +439,29 @@ struct SkinnyCfg16 {
   static_assert(LDS <= 160 * 1024 && S >= 1 && S <= 4 && LPB * (S - 1) <= 63, "LDS budget, vmcnt range");
 };
 
-template <typename T, typename C>
+template <typename T, typename C, int BL>
 __global__ void __launch_bounds__(C::NW * 64) gemm_skinny_kernel(const TileParams p) {
+  constexpr bool NC = BL == B_NC;
   constexpr int MT = C::MT, NW = C::NW, S = C::S, MB = C::MB, NB = C::NB, BN = C::BN, LPB = C::LPB, BNP = C::BNP;
   using Op = MfmaOp<T>;
   __shared__ __attribute__((aligned(1024))) uint8_t lds[C::LDS];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 15, g = lane >> 4;
-  const int n0 = (int)blockIdx.x * BN, rows_b = min(BN, p.N - n0);
+  const int n0 = (NC ? xcd_remap((int)blockIdx.x, (int)gridDim.x) : (int)blockIdx.x) * BN;
+  const int rows_b = min(BN, p.N - n0);
   const int nk = (p.K + kBK - 1) / kBK;
   const int cnt = nk > wave ? (nk - wave + NW - 1) / NW : 0;  // K blocks of this wave
   const uint32_t abytes = (uint32_t)(((int64_t)(p.M - 1) * p.lda + p.K) * 2);
   const __amdgpu_buffer_rsrc_t ra = make_rsrc(p.a, abytes);
   const __amdgpu_buffer_rsrc_t rb =
-      make_rsrc(p.b + (int64_t)n0 * p.ldb, (uint32_t)(((int64_t)(rows_b - 1) * p.ldb + p.K) * 2));
+      NC ? make_rsrc(p.b + n0, (uint32_t)(((int64_t)(p.K - 1) * p.ldb + rows_b) * 2))
+         : make_rsrc(p.b + (int64_t)n0 * p.ldb, (uint32_t)(((int64_t)(rows_b - 1) * p.ldb + p.K) * 2));
+  // N-contiguous B: a chunk past the last column's repeats that one; the last column's own
+  // chunk may run into the next K-row (columns never stored) and, on the last K-row, past
+  // the end of B, where the resource cuts it off by whole dwords: with an odd count of
+  // columns that takes the last element along, which is then put into LDS by hand.
+  const bool patch = NC && (rows_b & 1) != 0;
+  const uint16_t last_b = patch ? p.b[(int64_t)(p.K - 1) * p.ldb + n0 + rows_b - 1] : (uint16_t)0;
   // load q covers stage rows 8q .. 8q + 7; lane l fetches chunk (l % 8) ^ key(row)
   uint32_t xoff[C::XQ], woff[C::WQ];
 #pragma unroll
@@ -460,17 +471,33 @@ __global__ void __launch_bounds__(C::NW * 64) gemm_skinny_kernel(const TileParam
   }
 #pragma unroll
   for (int q = 0; q < C::WQ; ++q) {
-    const int row = 8 * q + (lane >> 3);
-    woff[q] = (uint32_t)(((int64_t)min(row, rows_b - 1) * p.ldb + 8 * ((lane & 7) ^ swz16(row))) * 2);
+    if constexpr (NC) {  // 512 / BN whole K-rows of BN columns
+      woff[q] = (uint32_t)(((int64_t)(q * (512 / BN) + lane / (BN / 8)) * p.ldb +
+                            8 * min(lane % (BN / 8), (rows_b - 1) / 8)) * 2);
+    } else {
+      const int row = 8 * q + (lane >> 3);
+      woff[q] = (uint32_t)(((int64_t)min(row, rows_b - 1) * p.ldb + 8 * ((lane & 7) ^ swz16(row))) * 2);
+    }
   }
   uint16_t* ring = (uint16_t*)lds + wave * (S * C::STAGE);
   auto issue = [&](int s, int j) {
-    const uint32_t ko = (uint32_t)min((wave + NW * j) * kBK, p.K - kBK) * 2u;
+    const uint32_t k0 = (uint32_t)min((wave + NW * j) * kBK, p.K - kBK);
     uint16_t* st = ring + s * C::STAGE;
+    if constexpr (NC) {
+      // transpose reads follow: loads the compiler does not track (buf_lds16_asm).  Below 64
+      // columns the workgroups share cache lines of B.
 #pragma unroll
-    for (int q = 0; q < C::XQ; ++q) buf_lds16(ra, xoff[q], ko, st + q * 8 * kBK);
+      for (int q = 0; q < C::XQ; ++q) buf_lds16_asm(ra, xoff[q], k0 * 2u, st + q * 8 * kBK);
 #pragma unroll
-    for (int q = 0; q < C::WQ; ++q) buf_lds16_cp<kCpolNT>(rb, woff[q], ko, st + (MT + 8 * q) * kBK);  // read once
+      for (int q = 0; q < C::WQ; ++q)
+        buf_lds16_asm<BN >= 64 ? kCpolNT : kCpolDefault>(rb, woff[q], k0 * (uint32_t)p.ldb * 2u,
+                                                         st + (MT + 8 * q) * kBK);
+    } else {
+#pragma unroll
+      for (int q = 0; q < C::XQ; ++q) buf_lds16(ra, xoff[q], k0 * 2u, st + q * 8 * kBK);
+#pragma unroll
+      for (int q = 0; q < C::WQ; ++q) buf_lds16_cp<kCpolNT>(rb, woff[q], k0 * 2u, st + (MT + 8 * q) * kBK);  // read once
+    }
   };
   f32x4_t acc[MB][NB];
 #pragma unroll
@@ -491,7 +518,13 @@ __global__ void __launch_bounds__(C::NW * 64) gemm_skinny_kernel(const TileParam
         else if (S >= 3 && later >= 2) wait_vmcnt<(S >= 3 ? 2 * LPB : 0)>();
         else if (S >= 2 && later >= 1) wait_vmcnt<(S >= 2 ? LPB : 0)>();
         else wait_vmcnt<0>();
-        const uint16_t* st = ring + s * C::STAGE;
+        uint16_t* st = ring + s * C::STAGE;
+        if constexpr (NC) {
+          if (patch && wave + NW * j == nk - 1) {  // uniform; the last K-row is row 63 of the last block
+            if (lane == 0) *(volatile uint16_t*)(st + MT * kBK + (kBK - 1) * BN + rows_b - 1) = last_b;
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+          }
+        }
         u32x4_t xf[MB][2], wf[NB][2];
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb) {
@@ -501,9 +534,18 @@ __global__ void __launch_bounds__(C::NW * 64) gemm_skinny_kernel(const TileParam
         }
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) {
-          const uint16_t* row = st + (MT + nb * 16 + r) * kBK;
-          wf[nb][0] = *(const u32x4_t*)(row + o0);
-          wf[nb][1] = *(const u32x4_t*)(row + o1);
+          if constexpr (NC) {  // lane (g, c) points at K-row 32 h + 8 g + c / 4 (+ 4), columns + 4 (c % 4)
+            const uint16_t* q = st + MT * kBK + (8 * g + (r >> 2)) * BN + nb * 16 + 4 * (r & 3);
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+              const u32x2_t lo = lds_read_tr16(q + 32 * h * BN), hi = lds_read_tr16(q + (32 * h + 4) * BN);
+              wf[nb][h] = u32x4_t{lo[0], lo[1], hi[0], hi[1]};
+            }
+          } else {
+            const uint16_t* row = st + (MT + nb * 16 + r) * kBK;
+            wf[nb][0] = *(const u32x4_t*)(row + o0);
+            wf[nb][1] = *(const u32x4_t*)(row + o1);
+          }
         }
         // the slot is free once its fragments are in registers
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -1368,7 +1410,7 @@ int launch_splitk(const GemmDesc& d, int splits, int kper, Ws& ws, hipStream_t s
   return rc;
 }
 
-template <typename T, typename C>
+template <typename T, int BL, typename C>
 int launch_skinny(const GemmDesc& d, hipStream_t stream) {
   TileParams p{};
   p.a = (const uint16_t*)d.a;
@@ -1379,11 +1421,11 @@ int launch_skinny(const GemmDesc& d, hipStream_t stream) {
   p.N = (int)d.N;
   p.K = (int)d.K;
   p.lda = d.sam;
-  p.ldb = d.sbn;
+  p.ldb = BL == B_KC ? d.sbn : d.sbk;
   p.ldc = d.scm;
   p.act = d.act;
   p.vec_store = (d.scm % 8 == 0) && aligned16(d.c);
-  hipLaunchKernelGGL((gemm_skinny_kernel<T, C>), dim3((unsigned)((d.N + C::BN - 1) / C::BN)), dim3(C::NW * 64), 0,
+  hipLaunchKernelGGL((gemm_skinny_kernel<T, C, BL>), dim3((unsigned)((d.N + C::BN - 1) / C::BN)), dim3(C::NW * 64), 0,
                      stream, p);
   return check_launch("gemm_skinny_kernel");
 }
@@ -1418,19 +1460,59 @@ inline SkinnyPick pick_skinny(const GemmDesc& d, bool aligned, int64_t cus) {
 // weights' stream (32 x 4096 x 4096 11.3, 64 14.6, 128 19.6; 32 x 2048 x 7168 11.2, 64 12.6;
 // 64 x 1024 x 8192 10.0, 128 11.5 us).  Wider problems run the mid-size
 // tiles, which win from M = 33 on.
-inline double skinny_alternative_us(const GemmDesc& d, int64_t cus) {
+inline double skinny_alternative_us(const GemmDesc& d, int64_t cus, double beyond_caches = 1.2) {
   const int64_t t32 = (d.M + 31) / 32 * ((d.N + 127) / 128);
   if ((d.M + 127) / 128 * ((d.N + 127) / 128) >= 128) return d.M <= 32 ? 1e300 : 0.0;
-  if (d.K >= 1024 && t32 * 2 <= cus) return 8.0 + (double)(d.N * d.K * 2) / 5.6e6 * (d.M <= 32 ? 0.55 : d.M <= 64 ? 1.0 : 1.8);
+  if (d.K >= 1024 && t32 * 2 <= cus) {
+    // (beyond the 48 MB or so that caches help with, M = 1: 8192 x 8192 45.7 us, N-contiguous 24.7)
+    const double bytes = (double)(d.N * d.K * 2);
+    return 8.0 + bytes / 5.6e6 * (d.M <= 32 ? (bytes > 48e6 ? beyond_caches : 0.4) : d.M <= 64 ? 1.0 : 1.8);
+  }
   return 3.0 + (double)((t32 + cus - 1) / cus * 160 * d.K * 2) / 80e3;
 }
-template <typename T>
+// The same for N-contiguous B: 2 us per round plus the longest of the weights' stream
+// (slower through short row pieces: 32, 64 or 128 bytes), a workgroup's own weights (64-column
+// ones leave CUs idle and pull 30 KB/us), and what a CU takes in, at 65 KB/us with most CUs
+// busy; misaligned rows cost half as much again.  Measured (bf16, M = 1 / 16 / 64 / 128, best
+// nb) against the split-K, ring, tile, packed and generic paths: 4096 x 1024 4.7 4.7 5.2 6.8
+// (8.4 8.5 9.0 12.2), 1024 x 1024 4.2 4.2 4.3 6.5 (7.9 8.0 8.2 8.3), 7168 x 2048 6.4 6.9 9.2
+// 12.9 (9.6 9.7 15.2 11.4), 4096 x 4096 8.6 10.4 14.0 18.7 (10.2 9.9 14.9 19.5), 823 x 1984 5.4
+// 5.4 7.6 10.2 (96 96 99 21), 320 x 1816 4.5 4.5 5.8 9.5 (24), 9473 x 565 6.2 6.4 9.3 13.5 (33
+// 32 21 22), 4096 x 4095 8.8 11.2 18.2 27.3 (191 21.5 21.9 22.0 us).
+inline SkinnyPick pick_skinny_nc(const GemmDesc& d, bool a_ok, bool b_nc, int64_t cus) {
+  SkinnyPick best{1, 1e300};
+  for (int nb : {1, 2, 4}) {
+    const int64_t bn = 16 * nb, wgs = (d.N + bn - 1) / bn, rounds = (wgs + cus - 1) / cus;
+    const double k2 = (double)(d.K * 2);
+    const double stream = (double)d.N * k2 / (nb == 1 ? 4.2e6 : nb == 2 ? 5.5e6 : 5.8e6);
+    const double own = (double)(rounds * bn) * k2 / (nb == 4 ? 30e3 : 60e3);
+    const double intake = (double)(rounds * (d.M + bn)) * k2 / (wgs >= 128 ? 65e3 : 105e3);
+    double slow = 1.0;
+    if (!a_ok) slow += 0.5 * (double)d.M / (double)(d.M + bn);
+    if (!b_nc) slow += 0.5 * (double)bn / (double)(d.M + bn);
+    const bool two_waves = nb == 4 && d.M > 64;  // what the LDS holds
+    double us = std::max(std::max(stream, own), two_waves ? 1.35 * intake : intake) * slow;
+    us += 0.5 + 2.0 * (double)rounds + (two_waves ? 2.0 : 0.0);
+    if (us < best.us) best = {nb, us};
+  }
+  return best;
+}
+// Its alternatives: the aligned paths, or with rows off 16-byte alignment a pack of A (and of
+// B unless it is read in place) before them; small unaligned problems have only the generic
+// kernel, one workgroup per 128 x 128 tile.
+inline double skinny_nc_alternative_us(const GemmDesc& d, bool aligned, bool b_nc, int64_t cus) {
+  const double us = d.K < 512 ? 5.5 : skinny_alternative_us(d, cus, 0.7);
+  if (aligned) return us;
+  if (d.M * d.N * d.K < (1ll << 27)) return 1e300;
+  return us + 6.0 + (b_nc ? 0.0 : 2.0 + (double)(d.N * d.K * 4) / 4.5e6);
+}
+template <typename T, int BL>
 int launch_skinny_nb(const GemmDesc& d, int nb, hipStream_t st) {
   // waves and stages per configuration: as much in flight as 160 KiB of LDS holds
   auto pick = [&](auto c1, auto c2, auto c4) {
-    return nb == 1   ? launch_skinny<T, decltype(c1)>(d, st)
-           : nb == 2 ? launch_skinny<T, decltype(c2)>(d, st)
-                     : launch_skinny<T, decltype(c4)>(d, st);
+    return nb == 1   ? launch_skinny<T, BL, decltype(c1)>(d, st)
+           : nb == 2 ? launch_skinny<T, BL, decltype(c2)>(d, st)
+                     : launch_skinny<T, BL, decltype(c4)>(d, st);
   };
   if (d.M <= 16) return pick(SkinnyCfg16<16, 8, 4, 1>{}, SkinnyCfg16<16, 8, 3, 2>{}, SkinnyCfg16<16, 8, 2, 4>{});
   if (d.M <= 32) return pick(SkinnyCfg16<32, 8, 3, 1>{}, SkinnyCfg16<32, 8, 2, 2>{}, SkinnyCfg16<32, 4, 3, 4>{});
@@ -1571,8 +1653,19 @@ int dispatch_typed(const GemmDesc& d, Ws& ws, hipStream_t stream) {
       const SkinnyPick k = pick_skinny(d, aligned, cus);
       if (!aligned || k.us < skinny_alternative_us(d, cus)) {
         if (ws.plan) return KORE_OK;
-        return launch_skinny_nb<T>(d, k.nb, stream);
+        return launch_skinny_nb<T, B_KC>(d, k.nb, stream);
       }
+    }
+  }
+  if (d.batch == 1 && d.sak == 1 && d.sbn == 1 && d.sbk != 1 && d.M <= 128 && d.K >= 64 && fits32 &&
+      (d.sam >= d.K || d.M == 1) && d.sbk >= d.N && d.M * d.sam * 2 + d.K * 2 < (1ll << 31) &&
+      (d.K + 64) * d.sbk * 2 < (1ll << 31)) {
+    const bool aligned = a_ok && b_nc && d.K % 64 == 0;
+    const int64_t cus = device_cus();
+    const SkinnyPick k = pick_skinny_nc(d, a_ok, b_nc, cus);
+    if (k.us * 1.15 < skinny_nc_alternative_us(d, aligned, b_nc, cus)) {
+      if (ws.plan) return KORE_OK;
+      return launch_skinny_nb<T, B_NC>(d, k.nb, stream);
     }
   }
   // M-contiguous A (a transposed view, e.g. dY^T of the backward) on the 256x256 buffer

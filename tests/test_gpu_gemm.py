@@ -774,3 +774,42 @@ def test_gemm_skinny(gpu, dtype, M, N, K):
         want[:, N - 1] = True
         nz = (a2[:, K - 61] != 0)  # inf * 0 is NaN in the reference too
         assert torch.equal(got.isinf()[nz], want[nz])
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,N,K", [(1, 1, 64), (1, 7, 65), (16, 9, 127), (17, 823, 1984), (33, 320, 1816),
+                                   (64, 512, 512), (64, 4095, 129), (65, 1001, 1000), (128, 9473, 565),
+                                   (128, 4096, 256), (100, 7168, 2048), (5, 14337, 640), (128, 16, 4095),
+                                   (40, 1030, 192)])
+def test_gemm_skinny_nc(gpu, dtype, M, N, K):
+    """M <= 128 against N-contiguous weights on the skinny kernel: any N (the last element of
+    B, which the buffer range check cuts off when an odd count of columns ends mid-dword),
+    K tails, 16- to 64-column workgroups, and a B that is a view with odd row stride and
+    offset, whose neighbours are NaN."""
+    g = torch.Generator().manual_seed(M + N + K)
+    a = (torch.randn((M, K), generator=g) / K ** 0.5).to(dtype)
+    b = torch.randn((K, N), generator=g).to(dtype)
+    b[K - 1] = 8.0  # the last K-row carries weight in every column
+    bias = torch.randn((N,), generator=g).to(dtype)
+    ag, bg, biasg = a.to(gpu), b.to(gpu), bias.to(gpu)
+    name = "bf16" if dtype == torch.bfloat16 else "fp16"
+    for act in ("none", "silu"):
+        out = kore_amd.gemm_fused(ag, bg, biasg, act)
+        assert bit_equal(kore_amd.gemm_fused(ag, bg, biasg, act), out)
+        pair_only(out.cpu(), gemm_fusion_ref(a, b, bias, act), name, f"skinny nc {M}x{N}x{K} {act}")
+    ld = N + 3
+    buf = torch.full((K * ld + 1,), float("nan"), dtype=dtype, device=gpu)
+    v = buf[1:].view(K, ld)[:, :N]
+    v.copy_(bg)
+    out = kore_amd.gemm_fused(ag, v, biasg, "none")
+    pair_only(out.cpu(), gemm_fusion_ref(a, b, bias, "none"), name, f"skinny nc {M}x{N}x{K} view")
+    if K > 100:
+        a2, b2 = a.float().abs().to(dtype), b.float().abs().to(dtype) + 1
+        a2[M - 1, K - 60] = float("inf")
+        b2[K - 61, N - 1] = float("inf")
+        got = kore_amd.gemm_fused(a2.to(gpu), b2.to(gpu), None, "none").cpu()
+        want = torch.zeros(M, N, dtype=torch.bool)
+        want[M - 1, :] = True
+        want[:, N - 1] = True
+        nz = (a2[:, K - 61] != 0)  # inf * 0 is NaN in the reference too
+        assert torch.equal(got.isinf()[nz], want[nz])
