@@ -955,9 +955,24 @@ __global__ void __launch_bounds__(256)
   }
 }
 
-// Block rows of the fp8 grouped tiles: 256x256 when experts average >= 64 rows (one
-// round of large tiles beats ~3 rounds of 128x128 tiles despite the padding).
-inline int grouped_fp8_block_rows(int64_t M, int64_t E) { return M >= 64 * E ? 256 : 128; }
+// Tiles of 256x256 to expect: M / 256 full blocks, and for about half of the (unevenly
+// loaded) experts one more that is mostly padding.
+inline int64_t grouped_tiles256(int64_t M, int64_t E, int64_t N) { return (M / 256 + E / 2) * (N / 256); }
+
+// Block rows of the fp8 grouped tiles: 256x256 when experts average over 64 rows (one round
+// of large tiles beats ~3 rounds of 128x128 tiles despite the padding) and those tiles occupy
+// enough CUs to stream the weights: M=4096 E=32 N=2048 K=4096 71 us against 78 on 128x128,
+// but M=512 E=8 60 against 28 and M=2048 E=32 71 against 61 us (one process, jagged routing).
+inline int grouped_fp8_block_rows(int64_t M, int64_t E, int64_t N) {
+  return M > 64 * E && grouped_tiles256(M, E, N) >= 100 ? 256 : 128;
+}
+// bf16: the 32-row ring up to 64 rows per expert, from 48 on only where 256-row tiles would
+// not fill the CUs (M=2048 E=32 N=2048 K=4096 149 us on the ring, 113 on 256x256 tiles; M=512
+// E=8 59 against 98 us).
+inline int grouped_bf16_block_rows(int64_t M, int64_t E, int64_t N) {
+  if (M <= 48 * E) return 32;
+  return M <= 64 * E && (N % 256 != 0 || grouped_tiles256(M, E, N) < 192) ? 32 : 256;
+}
 
 }  // namespace
 }  // namespace kore
@@ -984,7 +999,7 @@ extern "C" int kore_moe_grouped_gemm(const void* x, int64_t ldx, const void* w, 
       ((uintptr_t)out & 15u))
     return set_error(KORE_EINVAL, "moe_grouped_gemm: rows must be 16-byte aligned (ldx, ldo %% 8 == 0)");
   if (M >= (1ll << 30) || N * K >= (1ll << 40)) return set_error(KORE_EUNSUPPORTED, "moe_grouped_gemm: too large");
-  const int BM = M <= 64 * E ? 32 : 256;  // the 32-row ring or 256-row tiles
+  const int BM = grouped_bf16_block_rows(M, E, N);
   const GroupedWorkspace ws = carve_grouped(workspace, M, E, BM);
   if (workspace_bytes < kore_moe_grouped_gemm_workspace_bytes(M, E))
     return set_error(KORE_EWORKSPACE, "moe_grouped_gemm: workspace %zu bytes < required %zu", workspace_bytes,
@@ -1044,7 +1059,7 @@ extern "C" int kore_moe_grouped_gemm_fp8(const void* xq, int64_t ldx, const void
   if (workspace_bytes < kore_moe_grouped_gemm_workspace_bytes(M, E))
     return set_error(KORE_EWORKSPACE, "moe_grouped_gemm_fp8: workspace %zu bytes < required %zu", workspace_bytes,
                      kore_moe_grouped_gemm_workspace_bytes(M, E));
-  const int BM = N % 256 == 0 ? grouped_fp8_block_rows(M, E) : 128;
+  const int BM = N % 256 == 0 ? grouped_fp8_block_rows(M, E, N) : 128;
   const GroupedWorkspace w = carve_grouped(workspace, M, E, BM);
   const int64_t cap = align_capacity(M, E, BM);
   hipStream_t st = (hipStream_t)stream;
