@@ -967,10 +967,14 @@ inline int grouped_fp8_block_rows(int64_t M, int64_t E, int64_t N) {
   return M > 64 * E && grouped_tiles256(M, E, N) >= 100 ? 256 : 128;
 }
 // bf16: the 32-row ring up to 64 rows per expert, from 48 on only where 256-row tiles would
-// not fill the CUs (M=2048 E=32 N=2048 K=4096 149 us on the ring, 113 on 256x256 tiles; M=512
-// E=8 59 against 98 us).
-inline int grouped_bf16_block_rows(int64_t M, int64_t E, int64_t N) {
+// not fill the CUs (M=2048 E=32 N=2048 K=4096 149 us on the ring, 113 on 256x256 tiles).
+// Where those tiles leave half of the CUs idle, 128-row blocks on the decode ring from 56
+// rows per expert on (one process, against what ran before: M=600 E=8 N=2048 K=4096 98.7 ->
+// 50.0 us, M=2000 E=8 N=512 K=2048 61.6 -> 33.8, M=2000 E=16 N=1024 K=4096 104 -> 57, M=4096
+// E=16 N=1024 K=2048 68 -> 54, M=512 E=8 59.6 -> 50.6; M=300 E=8 N=1024 20.3 against 31.1).
+inline int grouped_bf16_block_rows(int64_t M, int64_t E, int64_t N, bool buf_ok) {
   if (M <= 48 * E) return 32;
+  if (buf_ok && N % 256 == 0 && M > 56 * E && grouped_tiles256(M, E, N) < 130) return 128;
   return M <= 64 * E && (N % 256 != 0 || grouped_tiles256(M, E, N) < 192) ? 32 : 256;
 }
 
@@ -999,7 +1003,9 @@ extern "C" int kore_moe_grouped_gemm(const void* x, int64_t ldx, const void* w, 
       ((uintptr_t)out & 15u))
     return set_error(KORE_EINVAL, "moe_grouped_gemm: rows must be 16-byte aligned (ldx, ldo %% 8 == 0)");
   if (M >= (1ll << 30) || N * K >= (1ll << 40)) return set_error(KORE_EUNSUPPORTED, "moe_grouped_gemm: too large");
-  const int BM = grouped_bf16_block_rows(M, E, N);
+  const bool buf_ok =
+      K % 64 == 0 && M * ldx * 2 + 4 * K < (1ll << 32) && N * K * 2 < (1ll << 32) && !g_force_generic;
+  const int BM = grouped_bf16_block_rows(M, E, N, buf_ok);
   const GroupedWorkspace ws = carve_grouped(workspace, M, E, BM);
   if (workspace_bytes < kore_moe_grouped_gemm_workspace_bytes(M, E))
     return set_error(KORE_EWORKSPACE, "moe_grouped_gemm: workspace %zu bytes < required %zu", workspace_bytes,
@@ -1027,10 +1033,13 @@ extern "C" int kore_moe_grouped_gemm(const void* x, int64_t ldx, const void* w, 
   p.abm = BM;
   p.out = (uint16_t*)out;
   p.ldo = ldo;
-  const bool buf_ok =
-      K % 64 == 0 && M * ldx * 2 + 4 * K < (1ll << 32) && N * K * 2 < (1ll << 32) && !g_force_generic;
   if (BM == 32) {
     rc = buf_ok ? launch_moe_decode<MOE_PLAIN, 128, 7>(p, cap, st) : launch_moe_gemm<MOE_PLAIN, 32, 128, 1, 4>(p, cap, st);
+  } else if (BM == 128) {
+    // four stages where every tile has a CU to itself, else two workgroups of two per CU
+    // (M=4096 E=16 N=1024 K=2048 53.5 against 61.3 us; M=600 E=8 above 50.0 against 65.4)
+    rc = grouped_tiles256(M, E, N) < 80 ? launch_moe_decode<MOE_PLAIN, 128, 4, 128>(p, cap, st)
+                                        : launch_moe_decode<MOE_PLAIN, 128, 2, 128>(p, cap, st);
   } else if (buf_ok) {
     rc = N % 256 == 0 ? launch_moe_buf<MOE_PLAIN, 256, 256>(p, cap, st) : launch_moe_buf<MOE_PLAIN, 256, 128>(p, cap, st);
   } else {

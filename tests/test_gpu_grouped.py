@@ -57,6 +57,23 @@ def test_grouped_gemm_ragged(gpu, M, E, N, K):
     verdict(out, ref, "grouped", "bf16", f"M{M} E{E} N{N} K{K}")
 
 
+@pytest.mark.parametrize("M,E,N,K", [(384, 8, 256, 256), (385, 8, 256, 256), (448, 8, 256, 320), (449, 8, 256, 320),
+                                     (512, 8, 512, 256), (513, 8, 512, 256), (1000, 8, 2048, 128),
+                                     (3000, 16, 1792, 192), (2048, 32, 2048, 256), (2049, 32, 2048, 256)])
+def test_grouped_block_choice(gpu, M, E, N, K):
+    """Both sides of the block-row rules of the bf16 (48, 56 and 64 rows per expert; 80, 130 and
+    192 tiles of 256x256) and fp8 (64 rows, 100 tiles) grouped GEMMs, jagged routing with some
+    ids outside [0, E) whose rows must be zero."""
+    hidden, w, ids = W.grouped_inputs(M, E, N, K, seed=M + N, router_bias=W.jagged_bias(E))
+    ids = torch.where(torch.arange(M) % 11 == 5, torch.full_like(ids, E), ids)
+    out = kore_amd.grouped_gemm(hidden.to(gpu), w.to(gpu), ids.to(gpu)).cpu()
+    verdict(out, grouped_gemm_ref(hidden, w, ids), "grouped", "bf16", f"{M} {E} {N} {K}")
+    K8 = -(-K // 128) * 128
+    xq, wq, xs, ws, _ = W.grouped_fp8_inputs(M, E, N, K8, seed=M + N, router_bias=W.jagged_bias(E))
+    out = kore_amd.grouped_gemm_fp8(xq.to(gpu), wq.to(gpu), xs.to(gpu), ws.to(gpu), ids.to(gpu)).cpu()
+    verdict(out, grouped_gemm_fp8_ref(xq, wq, xs, ws, ids), "grouped_fp8", "fp8", f"{M} {E} {N} {K8}")
+
+
 def test_grouped_gemm_invalid_ids_and_determinism(gpu):
     M, E, N, K = 300, 6, 256, 256
     hg, wg, tg = W.grouped_inputs(M, E, N, K, seed=3, device=gpu)
