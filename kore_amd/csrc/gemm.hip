@@ -179,8 +179,8 @@ __global__ void __launch_bounds__(kEngineThreads)
 
 // Buffer resources and per-lane byte offsets of the direct-to-LDS engines.  Rows of A
 // and of B^T past the tile's last valid row re-read that row; N-contiguous B is read
-// as K-rows of the n0 column block whose chunks past N (N % 8 == 0) re-read the last
-// chunk.  Either way the extra values only feed outputs that are never stored.
+// as K-rows of the n0 column block whose chunks past N re-read the last chunk (which runs
+// into the next K-row where N % 8 != 0).  Either way the extra values only feed outputs that are never stored.
 template <typename E, int BM, int BN, int BL>
 __device__ __forceinline__ void setup_operands(E& eng, const TileParams& p, int batch, int m0, int n0, int wave,
                                                int lane) {
@@ -190,12 +190,12 @@ __device__ __forceinline__ void setup_operands(E& eng, const TileParams& p, int 
     // M-contiguous A (element (m, k) at a[k * lda + m], M % 8 == 0): K-rows of the tile's
     // BM columns; chunks past M re-read the last one (their rows are never stored)
     const uint16_t* A = p.a + batch * p.sa + m0;
-    eng.ra = make_rsrc(A, (uint32_t)(((int64_t)(p.K - 1) * p.lda + rows_a) * 2));
+    eng.ra = make_rsrc(A, (uint32_t)(((int64_t)(kv - 1) * p.lda + rows_a) * 2));
     eng.a_kstep = (uint32_t)(kBK * p.lda * 2);
 #pragma unroll
     for (int j = 0; j < E::AJ; ++j) {
       const int kr = E::amc_krow(wave, lane, j);
-      eng.a_voff[j] = (uint32_t)(((int64_t)kr * p.lda + min(8 * E::amc_chunk(kr, lane), rows_a - 8)) * 2);
+      eng.a_voff[j] = (uint32_t)(((int64_t)kr * p.lda + 8 * min(E::amc_chunk(kr, lane), (rows_a - 1) / 8)) * 2);
     }
   } else {
     const uint16_t* A = p.a + batch * p.sa + (int64_t)m0 * p.lda;
@@ -221,7 +221,7 @@ __device__ __forceinline__ void setup_operands(E& eng, const TileParams& p, int 
 #pragma unroll
     for (int j = 0; j < E::BJ; ++j) {
       const int kr = E::nc_krow(wave, lane, j);
-      eng.b_voff[j] = (uint32_t)(((int64_t)kr * p.ldb + min(8 * E::nc_chunk(kr, lane), rows_b - 8)) * 2);
+      eng.b_voff[j] = (uint32_t)(((int64_t)kr * p.ldb + 8 * min(E::nc_chunk(kr, lane), (rows_b - 1) / 8)) * 2);
     }
   }
 }
@@ -269,19 +269,29 @@ __global__ void __launch_bounds__(64 * NWV)
 // Mid-size problems (a few hundred tiles, long K) on the deep ring engine: NSLOT - 1
 // K stages in flight per CU instead of one or two.  Either B layout, K % 64 == 0 (KT:
 // K tails read in place, the ring engine's K-tail mode).
-template <typename T, int BM, int BN, int WM, int WN, int NSLOT, int BL, bool KT = false>
+template <typename T, int BM, int BN, int WM, int WN, int NSLOT, int BL, bool KT = false, int AL = A_KC>
 __global__ void __launch_bounds__(256) gemm_deep_kernel(const TileParams p) {
-  using E = RingEngine<T, BM, BN, WM, WN, NSLOT, BL>;
+  using E = RingEngine<T, BM, BN, WM, WN, NSLOT, BL, kCpolDefault, AL>;
   __shared__ __attribute__((aligned(16))) uint16_t lds[E::LDS_ELEMS];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   int batch, m0, n0;
   tile_coords(p, BM, BN, batch, m0, n0);
   E eng;
   setup_operands<E, BM, BN, BL>(eng, p, batch, m0, n0, wave, lane);
-  if constexpr (KT) {  // last stage at K - 64 (bytes along a row / over N-contiguous K-rows)
-    eng.a_klast = (uint32_t)((p.kreal - kBK) * 2);
-    eng.b_klast = BL == B_NC ? (uint32_t)((int64_t)(p.kreal - kBK) * p.ldb * 2) : eng.a_klast;
+  if constexpr (KT) {  // last stage at K - 64 (bytes along a row / over K-rows)
+    const uint32_t kl = (uint32_t)((p.kreal - kBK) * 2);
+    eng.a_klast = AL == A_MC ? (uint32_t)((int64_t)(p.kreal - kBK) * p.lda * 2) : kl;
+    eng.b_klast = BL == B_NC ? (uint32_t)((int64_t)(p.kreal - kBK) * p.ldb * 2) : kl;
     eng.kdup = p.K - p.kreal;
+    const int rows_a = min(BM, p.M - m0), rows_b = min(BN, p.N - n0);
+    if (AL == A_MC && (rows_a & 1) != 0) {
+      eng.patch_a = (kBK - 1) * BM + ((((rows_a - 1) >> 3) ^ nc_x((kBK - 1) & 3)) << 3) + ((rows_a - 1) & 7);
+      eng.patch_av = p.a[batch * p.sa + (int64_t)(p.kreal - 1) * p.lda + m0 + rows_a - 1];
+    }
+    if (BL == B_NC && (rows_b & 1) != 0) {
+      eng.patch_b = (kBK - 1) * BN + ((((rows_b - 1) >> 3) ^ nc_x((kBK - 1) & 3)) << 3) + ((rows_b - 1) & 7);
+      eng.patch_bv = p.b[batch * p.sb + (int64_t)(p.kreal - 1) * p.ldb + n0 + rows_b - 1];
+    }
   }
   f32x16_t acc[E::MI][E::NI];
   E::zero(acc);
@@ -1232,7 +1242,7 @@ int launch_buf(const GemmDesc& d, hipStream_t stream) {
   return check_launch("gemm_buf_kernel");
 }
 
-template <typename T, int BM, int BN, int WM, int WN, int NSLOT, int BL, bool KT = false>
+template <typename T, int BM, int BN, int WM, int WN, int NSLOT, int BL, bool KT = false, int AL = A_KC>
 int launch_deep(const GemmDesc& d, hipStream_t stream) {
   TileParams p{};
   p.a = (const uint16_t*)d.a;
@@ -1243,7 +1253,7 @@ int launch_deep(const GemmDesc& d, hipStream_t stream) {
   p.N = (int)d.N;
   p.K = (int)d.K;
   p.kb = (int)(d.kvalid > 0 ? d.kvalid : d.K);
-  p.lda = d.sam;
+  p.lda = AL == A_MC ? d.sak : d.sam;
   p.ldb = (BL == B_KC) ? d.sbn : d.sbk;
   p.ldc = d.scm;
   p.sa = d.sa;
@@ -1262,7 +1272,7 @@ int launch_deep(const GemmDesc& d, hipStream_t stream) {
     p.kreal = (int)d.K;
     p.K = (int)((d.K + kBK - 1) / kBK * kBK);
   }
-  hipLaunchKernelGGL((gemm_deep_kernel<T, BM, BN, WM, WN, NSLOT, BL, KT>), dim3((unsigned)blocks), dim3(256), 0, stream,
+  hipLaunchKernelGGL((gemm_deep_kernel<T, BM, BN, WM, WN, NSLOT, BL, KT, AL>), dim3((unsigned)blocks), dim3(256), 0, stream,
                      p);
   return check_launch("gemm_deep_kernel");
 }
@@ -1571,6 +1581,7 @@ int launch_engine(const GemmDesc& d, hipStream_t stream) {
 template <typename T, int BL>
 int launch_deep_kt(const GemmDesc& d, hipStream_t stream) {
   switch (pick_tile(d)) {
+    case TILE_256x256:  // (ragged ring; the 256x256 engine has its own K-tail path)
     case TILE_256x128: return launch_deep<T, 256, 128, 2, 2, 3, BL, true>(d, stream);
     case TILE_128x128: return launch_deep<T, 128, 128, 2, 2, 4, BL, true>(d, stream);
     case TILE_64x128: return launch_deep<T, 64, 128, 2, 2, 6, BL, true>(d, stream);
@@ -1592,6 +1603,37 @@ inline bool padded_fits(const GemmDesc& d) {
   const int64_t Kp = (d.K + 63) / 64 * 64;
   return d.M < (1ll << 31) && d.N < (1ll << 31) && Kp * 2 * 256 + Kp * 2 < (1ll << 31) && d.batch <= 65535;
 }
+// Ragged ring: operands with a unit stride along either index, at any 2-byte alignment, any
+// sizes with K >= 64, read in place (the K-tail mode of the deep ring; rows that are K-rows
+// may have any length).  Against the pack pass and its launches, or the generic kernel, one
+// process: backward 273 x 455 x 320 58.7 -> 16.2 us, 504 x 1472 x 2991 63.7 -> 33.6, linear
+// 1026 x 5663 x 768 41.6 -> 21.7, 6520 x 1247 x 1231 63.7 -> 45.1, batched 55 x 832 x 320 x 82
+// 70.8 -> 30.2.  Packed operands run the faster 256x256 tiles, so they stay from 2^34 products
+// on (4097^3); where B is read in place anyway, from 2^30 on for an M-contiguous A (dW of a
+// 300 x 4096 x 4096 backward, 57.7 against 63.7 us for the two) and for few tiles along a long
+// K, which reads misaligned rows of A once per column tile (496 x 768 x 9657 44.2 against 46.5).
+inline bool ragged_ring_ok(const GemmDesc& d) {
+  const bool akc = d.sak == 1, bkc = d.sbk == 1;
+  const int64_t mnk = d.M * d.N * d.K * d.batch;
+  if (d.K < 64 || !(akc || d.sam == 1) || !(bkc || d.sbn == 1) || mnk >= (1ll << 34)) return false;
+  if (d.sam < 0 || d.sak < 0 || d.sbk < 0 || d.sbn < 0) return false;
+  if (padded_b_inplace(d) && mnk >= (1ll << 30)) {
+    if (!akc) return false;
+    if (d.K > 4096 && (d.M + 127) / 128 * ((d.N + 127) / 128) * d.batch < 64) return false;
+  }
+  const int64_t lim = 1ll << 31;
+  return (akc ? d.sam * 2 * 256 + d.K * 2 : d.sak * 2 * (d.K + 64) + 512) < lim &&
+         (bkc ? d.sbn * 2 * 256 + d.K * 2 : d.sbk * 2 * (d.K + 64) + 512) < lim;
+}
+template <typename T>
+int launch_ragged_ring(const GemmDesc& d, hipStream_t stream) {
+  const bool bkc = d.sbk == 1;
+  if (d.sak != 1)
+    return bkc ? launch_deep<T, 128, 128, 2, 2, 4, B_KC, true, A_MC>(d, stream)
+               : launch_deep<T, 128, 128, 2, 2, 4, B_NC, true, A_MC>(d, stream);
+  return bkc ? launch_deep_kt<T, B_KC>(d, stream) : launch_deep_kt<T, B_NC>(d, stream);
+}
+
 template <typename T>
 int launch_padded(const GemmDesc& d, Ws& ws, hipStream_t stream) {
   const int64_t Kp = (d.K + 63) / 64 * 64;
@@ -1776,6 +1818,11 @@ int dispatch_typed(const GemmDesc& d, Ws& ws, hipStream_t stream) {
     }
     if (big && !short_k) return launch_tile<T, B_NC, 256, 256>(d, stream);
     return small ? launch_tile<T, B_NC, 64, 64>(d, stream) : launch_tile<T, B_NC, 128, 128>(d, stream);
+  }
+  // Any other problem whose operands have a unit stride: read in place on the ring tiles.
+  if (ragged_ring_ok(d) && fits32) {
+    if (ws.plan) return KORE_OK;
+    return launch_ragged_ring<T>(d, stream);
   }
   // Large problems in other layouts: pack, then the engines (small ones are cheaper on
   // the generic kernel than a pack pass).

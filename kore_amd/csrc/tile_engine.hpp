@@ -1079,9 +1079,15 @@ namespace kore {
 // BCPOL is the cache policy of the B loads: non-temporal where every B element is read
 // by one workgroup only (the split-K decode GEMM streams its weights once).
 // ---------------------------------------------------------------------------------
-template <typename T, int BM, int BN, int WM, int WN, int NSLOT, int BL, int BCPOL = kCpolDefault>
+template <typename T, int BM, int BN, int WM, int WN, int NSLOT, int BL, int BCPOL = kCpolDefault, int AL = A_KC>
 struct RingEngine {
-  static constexpr bool AMC = false;  // A is K-contiguous
+  static constexpr bool AMC = AL == A_MC;  // A staged as K-rows, like an N-contiguous B
+  static_assert(!AMC || BM == 128 || BM == 256, "M-contiguous A tile height");
+  static constexpr int NCRA = 512 / BM, NCHA = BM / 8;  // A_MC: K-rows per load, chunks per K-row
+  static __device__ __forceinline__ int amc_krow(int wave, int lane, int j) {
+    return (wave + WM * WN * j) * NCRA + lane / NCHA;
+  }
+  static __device__ __forceinline__ int amc_chunk(int krow, int lane) { return (lane % NCHA) ^ nc_x(krow & 3); }
   static constexpr int NW = 4;
   static_assert(WM * WN == NW, "4 waves");
   static constexpr int WROWS = BM / WM, WCOLS = BN / WN;
@@ -1106,39 +1112,54 @@ struct RingEngine {
   __amdgpu_buffer_rsrc_t ra, rb;
   uint32_t a_voff[AJ], b_voff[BJ];
   uint32_t b_kstep;  // NC: bytes of B between consecutive 64-row K stages
+  uint32_t a_kstep;  // A_MC: bytes of A between consecutive 64-row K stages
   // K tail (mainloop<true>, K % 64 != 0): the last stage is read from K - 64 (scalar byte
   // offsets a_klast, b_klast) and its first kdup columns, which the stage before already
   // covered, are zeroed in LDS in both operands once it has landed.
   uint32_t a_klast, b_klast;
   int kdup;
 
+  // K-row operands (NC, A_MC) with an odd count of columns in the last tile: on the last K-row
+  // the buffer range check cuts the chunk off by whole dwords, the last element with it; it is
+  // put into the last stage by hand (position in the stage, -1: none).
+  int patch_a = -1, patch_b = -1;
+  uint16_t patch_av = 0, patch_bv = 0;
+
   // Zero K columns [0, kdup) of both operands of the stage at st (every thread takes part).
   __device__ __forceinline__ void zero_dup(uint16_t* st) const {
     const int tid = threadIdx.x;
-    for (int idx = tid; idx < BM * kdup; idx += NW * 64) {
-      const int r = idx / kdup, k = idx - r * kdup;
-      st[r * kBK + (((k >> 3) ^ swz8(r)) << 3) + (k & 7)] = 0;
+    auto cols = [&](uint16_t* op, int rows) {  // 128-byte rows: whole 16-byte chunks
+      for (int r = tid; r < rows; r += NW * 64)
+        for (int c = 0; 8 * c < kdup; ++c) {
+          u32x4_t* q = (u32x4_t*)(op + r * kBK + ((c ^ swz8(r)) << 3));
+          *q = zero_lead(*q, 2 * kdup - 16 * c);
+        }
+    };
+    auto krows = [&](uint16_t* op, int width) {
+      for (int idx = tid; idx < kdup * width / 8; idx += NW * 64) *(u32x4_t*)(op + 8 * idx) = zero4();
+    };
+    if constexpr (AMC) krows(st, BM);
+    else cols(st, BM);
+    if constexpr (NC) krows(st + B_OFF, BN);
+    else cols(st + B_OFF, BN);
+    if constexpr (AMC) {
+      if (tid == 0 && patch_a >= 0) st[patch_a] = patch_av;
     }
     if constexpr (NC) {
-      for (int idx = tid; idx < kdup * BN; idx += NW * 64) st[B_OFF + idx] = 0;  // whole K-rows
-    } else {
-      for (int idx = tid; idx < BN * kdup; idx += NW * 64) {
-        const int r = idx / kdup, k = idx - r * kdup;
-        st[B_OFF + r * kBK + (((k >> 3) ^ swz8(r)) << 3) + (k & 7)] = 0;
-      }
+      if (tid == 0 && patch_b >= 0) st[B_OFF + patch_b] = patch_bv;
     }
   }
 
-  __device__ __forceinline__ void issue(uint16_t* lds, int slot, uint32_t soff, uint32_t soffb, int wave) const {
+  __device__ __forceinline__ void issue(uint16_t* lds, int slot, uint32_t soffa, uint32_t soffb, int wave) const {
     uint16_t* st = lds + slot * STAGE;
     auto ld = [&](__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t so, uint16_t* dst, auto cpol_tag) {
       constexpr int CP = decltype(cpol_tag)::value;
-      if constexpr (NC) buf_lds16_asm<CP>(r, voff, so, dst);
+      if constexpr (NC || AMC) buf_lds16_asm<CP>(r, voff, so, dst);
       else buf_lds16_cp<CP>(r, voff, so, dst);
     };
 #pragma unroll
     for (int j = 0; j < AJ; ++j)
-      ld(ra, a_voff[j], soff, st + (wave + NW * j) * 8 * kBK, std::integral_constant<int, kCpolDefault>{});
+      ld(ra, a_voff[j], soffa, st + (wave + NW * j) * 8 * kBK, std::integral_constant<int, kCpolDefault>{});
 #pragma unroll
     for (int j = 0; j < BJ; ++j)
       ld(rb, b_voff[j], soffb, st + B_OFF + (wave + NW * j) * 8 * kBK, std::integral_constant<int, BCPOL>{});
@@ -1169,7 +1190,7 @@ struct RingEngine {
     const int lr = lane & 31, hh = lane >> 5;
     const int rowA0 = wm * WROWS, rowB0 = wn * WCOLS;
     // fragment row R + lr (R % 32 == 0): swz8(R + lr) = (lr & 7) ^ (lr >> 3) ^ (4 * ((R / 32) & 1))
-    int offA[2][4], offB[2][4], offNC[NI];
+    int offA[2][4], offB[2][4], offNC[NI], offMC[MI];
 #pragma unroll
     for (int par = 0; par < 2; ++par) {
       const int qa = (wm * MI + par) & 1, qb = (wn * NI + par) & 1;
@@ -1182,17 +1203,22 @@ struct RingEngine {
       }
     }
     if constexpr (NC) nc_frag_offsets<BN, NI>(lane, rowB0, offNC);
+    if constexpr (AMC) nc_frag_offsets<BM, MI>(lane, rowA0, offMC);
     const int nk = (k_end - k_begin) / kBK, kb0 = k_begin / kBK;
     auto soff_of = [&](int stage) -> uint32_t {
       if (KT && stage >= nk - 1) return a_klast;
       return (uint32_t)(kb0 + min(stage, nk - 1)) * (kBK * 2);
     };
     auto soffb_of = [&](int stage) -> uint32_t {
-      if (KT && NC && stage >= nk - 1) return b_klast;
+      if (KT && stage >= nk - 1) return b_klast;
       return NC ? (uint32_t)(kb0 + min(stage, nk - 1)) * b_kstep : soff_of(stage);
     };
+    auto soffa_of = [&](int stage) -> uint32_t {
+      if (KT && AMC && stage >= nk - 1) return a_klast;
+      return AMC ? (uint32_t)(kb0 + min(stage, nk - 1)) * a_kstep : soff_of(stage);
+    };
 #pragma unroll
-    for (int s = 0; s < NSLOT - 1; ++s) issue(lds, s, soff_of(s), soffb_of(s), wave);
+    for (int s = 0; s < NSLOT - 1; ++s) issue(lds, s, soffa_of(s), soffb_of(s), wave);
     int slot = 0;
     for (int s = 0; s < nk; ++s) {
       wait_vmcnt<(NSLOT - 2) * LPS>();
@@ -1205,12 +1231,20 @@ struct RingEngine {
         }
       }
       const int nslot = slot == 0 ? NSLOT - 1 : slot - 1;  // slot of stage s - 1
-      issue(lds, nslot, soff_of(s + NSLOT - 1), soffb_of(s + NSLOT - 1), wave);
-      const uint16_t* sA = lds + slot * STAGE + rowA0 * kBK;
+      issue(lds, nslot, soffa_of(s + NSLOT - 1), soffb_of(s + NSLOT - 1), wave);
+      const uint16_t* sA = lds + slot * STAGE + (AMC ? 0 : rowA0 * kBK);
       const uint16_t* sB = lds + slot * STAGE + B_OFF;
       auto read = [&](int ks, u32x4_t (&af)[MI], u32x4_t (&bf)[NI]) {
 #pragma unroll
-        for (int i = 0; i < MI; ++i) af[i] = *(const u32x4_t*)(sA + i * 32 * kBK + offA[i & 1][ks]);
+        for (int i = 0; i < MI; ++i) {
+          if constexpr (AMC) {
+            const uint16_t* q = sA + offMC[i] + 16 * ks * BM;
+            const u32x2_t lo = lds_read_tr16(q), hi = lds_read_tr16(q + 4 * BM);
+            af[i] = u32x4_t{lo[0], lo[1], hi[0], hi[1]};
+          } else {
+            af[i] = *(const u32x4_t*)(sA + i * 32 * kBK + offA[i & 1][ks]);
+          }
+        }
 #pragma unroll
         for (int j = 0; j < NI; ++j) {
           if constexpr (NC) {

@@ -813,3 +813,41 @@ def test_gemm_skinny_nc(gpu, dtype, M, N, K):
         want[:, N - 1] = True
         nz = (a2[:, K - 61] != 0)  # inf * 0 is NaN in the reference too
         assert torch.equal(got.isinf()[nz], want[nz])
+
+
+@pytest.mark.parametrize("layout", ["kc_kc", "kc_nc", "mc_kc", "mc_nc"])
+@pytest.mark.parametrize("M,N,K", [(129, 1, 64), (200, 7, 65), (131, 129, 127), (273, 455, 320), (345, 895, 1001),
+                                   (513, 640, 128), (1026, 1663, 191), (2049, 1001, 100), (300, 4097, 257)])
+def test_gemm_ragged_ring(gpu, layout, M, N, K):
+    """Any sizes with K >= 64 and any row alignment on the ring tiles, A along K or along M (a
+    transposed view), B along K or along N: row, column and K tails, the last element of an
+    odd K-row operand, operands as views with odd strides inside NaN, and an infinity in a
+    column that the last stage repeats, which must reach exactly its own row and column."""
+    g = torch.Generator().manual_seed(M + N + K)
+    a = (torch.randn((M, K), generator=g) / K ** 0.5).bfloat16()
+    b = torch.randn((K, N), generator=g).bfloat16()
+    a[:, K - 1] = 0.5  # the last K column carries weight everywhere
+    b[K - 1] = 8.0
+
+    def place(t, along_cols, pad):  # unit stride along the columns of t, or along its rows
+        u = t if along_cols else t.t()
+        buf = torch.full((u.shape[0] * (u.shape[1] + pad) + 1,), float("nan"), dtype=t.dtype, device=gpu)
+        v = buf[1:].view(u.shape[0], u.shape[1] + pad)[:, :u.shape[1]]
+        v.copy_(u)
+        return v if along_cols else v.t()
+
+    ref = matmul_ref(a, b)
+    for pad in (0, 3):
+        av, bv = place(a, layout[:2] == "kc", pad), place(b, layout[3:] == "nc", pad)
+        out = kore_amd.gemm(av, bv)
+        assert bit_equal(kore_amd.gemm(av, bv), out)
+        pair_only(out.cpu(), ref, "bf16", f"ragged ring {layout} {M}x{N}x{K} pad {pad}")
+    if K % 64 != 0 and K > 64:
+        a2, b2 = a.float().abs().bfloat16() + 1, b.float().abs().bfloat16() + 1
+        a2[M - 1, K - 60] = float("inf")
+        b2[K - 61, N - 1] = float("inf")
+        got = kore_amd.gemm(place(a2, layout[:2] == "kc", 1), place(b2, layout[3:] == "nc", 1)).cpu()
+        want = torch.zeros(M, N, dtype=torch.bool)
+        want[M - 1, :] = True
+        want[:, N - 1] = True
+        assert torch.equal(got.isinf(), want)
