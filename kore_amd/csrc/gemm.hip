@@ -1611,7 +1611,8 @@ inline bool padded_fits(const GemmDesc& d) {
 // 70.8 -> 30.2.  Packed operands run the faster 256x256 tiles, so they stay from 2^34 products
 // on (4097^3); where B is read in place anyway, from 2^30 on for an M-contiguous A (dW of a
 // 300 x 4096 x 4096 backward, 57.7 against 63.7 us for the two) and for few tiles along a long
-// K, which reads misaligned rows of A once per column tile (496 x 768 x 9657 44.2 against 46.5).
+// K, which reads misaligned rows of A once per column tile (496 x 768 x 9657 44.2 against
+// 46.5).  Two misaligned K-contiguous operands along a long K are packed too.
 inline bool ragged_ring_ok(const GemmDesc& d) {
   const bool akc = d.sak == 1, bkc = d.sbk == 1;
   const int64_t mnk = d.M * d.N * d.K * d.batch;
@@ -1619,8 +1620,9 @@ inline bool ragged_ring_ok(const GemmDesc& d) {
   if (d.sam < 0 || d.sak < 0 || d.sbk < 0 || d.sbn < 0) return false;
   if (padded_b_inplace(d) && mnk >= (1ll << 30)) {
     if (!akc) return false;
-    if (d.K > 4096 && (d.M + 127) / 128 * ((d.N + 127) / 128) * d.batch < 64) return false;
+    if (d.K >= 2048 && (d.M + 127) / 128 * ((d.N + 127) / 128) * d.batch < 64) return false;
   }
+  if (akc && bkc && d.K >= 4000 && mnk >= (1ll << 30)) return false;
   const int64_t lim = 1ll << 31;
   return (akc ? d.sam * 2 * 256 + d.K * 2 : d.sak * 2 * (d.K + 64) + 512) < lim &&
          (bkc ? d.sbn * 2 * 256 + d.K * 2 : d.sbk * 2 * (d.K + 64) + 512) < lim;
@@ -1705,7 +1707,10 @@ int dispatch_typed(const GemmDesc& d, Ws& ws, hipStream_t stream) {
     const bool aligned = a_ok && b_nc && d.K % 64 == 0;
     const int64_t cus = device_cus();
     const SkinnyPick k = pick_skinny_nc(d, a_ok, b_nc, cus);
-    if (k.us * 1.15 < skinny_nc_alternative_us(d, aligned, b_nc, cus)) {
+    // (up to 128 workgroups along a K of 4096 or more would leave half of the CUs idle for
+    // long: split-K spreads those over all of them)
+    const bool few = aligned && d.K >= 4096 && d.N <= 2048;
+    if (!few && k.us * 1.15 < skinny_nc_alternative_us(d, aligned, b_nc, cus)) {
       if (ws.plan) return KORE_OK;
       return launch_skinny_nb<T, B_NC>(d, k.nb, stream);
     }
