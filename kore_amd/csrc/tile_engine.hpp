@@ -1128,12 +1128,16 @@ struct RingEngine {
   // Zero K columns [0, kdup) of both operands of the stage at st (every thread takes part).
   __device__ __forceinline__ void zero_dup(uint16_t* st) const {
     const int tid = threadIdx.x;
-    auto cols = [&](uint16_t* op, int rows) {  // 128-byte rows: whole 16-byte chunks
-      for (int r = tid; r < rows; r += NW * 64)
-        for (int c = 0; 8 * c < kdup; ++c) {
-          u32x4_t* q = (u32x4_t*)(op + r * kBK + ((c ^ swz8(r)) << 3));
-          *q = zero_lead(*q, 2 * kdup - 16 * c);
-        }
+    // 128-byte rows: whole 16-byte chunks, then single elements.  Stores only: reading the last
+    // chunk back to zero a part of it puts an LDS round trip between the two barriers
+    // (bf16 300 x 1000 x 585 10.1 -> 9.1 us, 512 x 4096 x 4033 35.1 -> 34.5, K = 4095 34.2 -> 34.0).
+    auto cols = [&](uint16_t* op, int rows) {
+      for (int r = tid; r < rows; r += NW * 64) {
+        int c = 0;
+        for (; 8 * c + 8 <= kdup; ++c) *(u32x4_t*)(op + r * kBK + ((c ^ swz8(r)) << 3)) = zero4();
+        uint16_t* q = op + r * kBK + ((c ^ swz8(r)) << 3);
+        for (int k = 8 * c; k < kdup; ++k) q[k & 7] = 0;
+      }
     };
     auto krows = [&](uint16_t* op, int width) {
       for (int idx = tid; idx < kdup * width / 8; idx += NW * 64) *(u32x4_t*)(op + 8 * idx) = zero4();
