@@ -1618,9 +1618,12 @@ inline bool ragged_ring_ok(const GemmDesc& d) {
   const int64_t mnk = d.M * d.N * d.K * d.batch;
   if (d.K < 64 || !(akc || d.sam == 1) || !(bkc || d.sbn == 1) || mnk >= (1ll << 34)) return false;
   if (d.sam < 0 || d.sak < 0 || d.sbk < 0 || d.sbn < 0) return false;
-  if (padded_b_inplace(d) && mnk >= (1ll << 30)) {
-    if (!akc) return false;
-    if (d.K >= 2048 && (d.M + 127) / 128 * ((d.N + 127) / 128) * d.batch < 64) return false;
+  if (padded_b_inplace(d)) {
+    const bool skinny_m = d.batch == 1 && d.M <= 128;  // packed A goes on to split-K
+    if (mnk >= (1ll << 30) && !akc) return false;
+    if (mnk >= (1ll << (skinny_m ? 27 : 30)) && (skinny_m || d.K >= 2048) &&
+        (d.M + 127) / 128 * ((d.N + 127) / 128) * d.batch < 64)
+      return false;
   }
   if (akc && bkc && d.K >= 4000 && mnk >= (1ll << 30)) return false;
   const int64_t lim = 1ll << 31;
@@ -1707,9 +1710,18 @@ int dispatch_typed(const GemmDesc& d, Ws& ws, hipStream_t stream) {
     const bool aligned = a_ok && b_nc && d.K % 64 == 0;
     const int64_t cus = device_cus();
     const SkinnyPick k = pick_skinny_nc(d, a_ok, b_nc, cus);
-    // (up to 128 workgroups along a K of 4096 or more would leave half of the CUs idle for
-    // long: split-K spreads those over all of them)
-    const bool few = aligned && d.K >= 4096 && d.N <= 2048;
+    // Weights that come from memory cost a workgroup one cache line per K-row, however few of
+    // its columns it owns, so a long K is left to split-K, which gives the K-rows to more
+    // workgroups, unless many rows and columns pay for it.  512 MiB flushed before each call /
+    // repeated calls, split-K against this kernel in us: 1x4096x4096 13.4 / 9.4 against
+    // 22.7 / 8.7, 16x4096x2048 12.0 / 8.5 against 14.8 / 4.8, 128x2048x2048 14.4 / 9.7 against
+    // 20.0 / 12.0; on this kernel's side of the line 16x4096x1024 10.5 / 8.8 against 10.0 / 4.5,
+    // 64x8192x2048 21.0 / 17.0 against 19.8 / 9.9, 64x4096x2048 15.0 / 11.8 against 15.8 / 7.9.
+    // 65 rows and more on up to 2048 columns lose as well (128x1024x1024 10.8 against 11.7
+    // flushed, packed 128x2048x2047 13.8 against 15.8 repeated).
+    const bool packs = b_nc && d.M * d.N * d.K >= (1ll << 27);
+    const bool few = (aligned && d.K >= 2048 && (d.M <= 32 || d.N < 4096)) ||
+                     ((aligned || packs) && d.M > 64 && d.N <= 2048);
     if (!few && k.us * 1.15 < skinny_nc_alternative_us(d, aligned, b_nc, cus)) {
       if (ws.plan) return KORE_OK;
       return launch_skinny_nb<T, B_NC>(d, k.nb, stream);
