@@ -67,13 +67,14 @@ int kore_abi_version(void);
  * (v_mfma_f32_32x32x2_f32, no reduced-precision inputs), fast path K % 64 == 0.
  *   A element (m,k) at a[m*lda_m + k*lda_k]; B element (k,n) at b[k*ldb_k + n*ldb_n];
  *   C element (m,n) at c[m*ldc_m + n]; bias may be NULL (no bias), else [N] contiguous.
- * Any strides are accepted; the MFMA fast path needs unit stride along K for A and
- * along K or N for B and 16-byte aligned rows.  K tails (e.g. K = 4095) with A K-contiguous
- * are read in place on large problems (16-bit: >= 128 tiles of 128x128 and K >= 256, or a
- * 256x256 grid; fp32: M*N*K >= 2^26), rows at any 2-byte alignment;
- * other layouts are packed into `workspace` first when the problem is large, or run a
- * slower generic kernel when it is small; decode-sized M splits K and sums fp32
- * partials held in `workspace`.  M, N >= 1, K >= 0 (K == 0 gives act(bias); a and b
+ * Any strides are accepted.  With a unit stride along either index of each operand the
+ * MFMA engines read A and B in place: any K from 64 in 16 bits (rows at any 2-byte
+ * alignment; fp32: 16-byte rows, K % 64 == 0, K tails from M*N*K >= 2^26); long K tails,
+ * very large problems and other layouts are packed into `workspace` first where the
+ * packed engines are faster, and small problems without a unit stride run a slower
+ * generic kernel.  M <= 128 in 16 bits streams the weights through one kernel without
+ * scratch, or splits K and sums fp32 partials held in `workspace`, whichever is
+ * estimated faster.  M, N >= 1, K >= 0 (K == 0 gives act(bias); a and b
  * may then be NULL).  `workspace` must hold kore_gemm_workspace_bytes(<same args>).
  * Replaces: gemm(a, b)            kore/tasks/gemm_bf16/seed_triton.py:64-86
  *           <op>(a, b[, bias])    kore/tasks/_genops.py:715-731 (_GEMM_TMPL entry,
