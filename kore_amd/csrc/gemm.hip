@@ -180,15 +180,20 @@ __global__ void __launch_bounds__(kEngineThreads)
 // Buffer resources and per-lane byte offsets of the direct-to-LDS engines.  Rows of A
 // and of B^T past the tile's last valid row re-read that row; N-contiguous B is read
 // as K-rows of the n0 column block whose chunks past N re-read the last chunk (which runs
-// into the next K-row where N % 8 != 0).  Either way the extra values only feed outputs that are never stored.
+// into the next K-row where N % 8 != 0).  Either way the extra values only feed outputs that
+// are never stored.  With an odd count of columns the resource, which ends with the last
+// K-row, cuts that row's last element off (the range check works on whole dwords); the KT
+// ring puts it back (patch_a, patch_b).  That is the only K-row cut off as long as the others
+// start at least one element earlier: the K-row stride is 1 or more (ragged_ring_ok), or the
+// count of columns even.
 template <typename E, int BM, int BN, int BL>
 __device__ __forceinline__ void setup_operands(E& eng, const TileParams& p, int batch, int m0, int n0, int wave,
                                                int lane) {
   const int rows_a = min(BM, p.M - m0), rows_b = min(BN, p.N - n0);
   const int kv = p.kreal > 0 ? p.kreal : p.K;  // K the operands hold
   if constexpr (E::AMC) {
-    // M-contiguous A (element (m, k) at a[k * lda + m], M % 8 == 0): K-rows of the tile's
-    // BM columns; chunks past M re-read the last one (their rows are never stored)
+    // M-contiguous A (element (m, k) at a[k * lda + m]): K-rows of the tile's BM columns;
+    // chunks past M re-read the last one (their rows are never stored)
     const uint16_t* A = p.a + batch * p.sa + m0;
     eng.ra = make_rsrc(A, (uint32_t)(((int64_t)(kv - 1) * p.lda + rows_a) * 2));
     eng.a_kstep = (uint32_t)(kBK * p.lda * 2);
@@ -1594,9 +1599,11 @@ int launch_deep_kt(const GemmDesc& d, hipStream_t stream) {
 // K-rows, are packed K-contiguous with the K tail zero-padded to a multiple of 64
 // into the caller's workspace.
 // An N-contiguous B is read in place: its buffer resource ends at the last real
-// K-row, so the padded rows read as zero.  The caller checks padded_fits first.
+// K-row, so the padded rows read as zero.  K-rows that overlap (sbk < N) are packed: the
+// padded rows would read elements of B, and an infinity times A's zero padding is a NaN.
+// The caller checks padded_fits first.
 inline bool padded_b_inplace(const GemmDesc& d) {
-  return d.sbn == 1 && d.sbk % 8 == 0 && aligned16(d.b) && d.sb % 8 == 0 && d.N % 8 == 0 &&
+  return d.sbn == 1 && d.sbk % 8 == 0 && d.sbk >= d.N && aligned16(d.b) && d.sb % 8 == 0 && d.N % 8 == 0 &&
          d.sbk * 2 * d.K + d.N * 2 < (1ll << 31);
 }
 inline bool padded_fits(const GemmDesc& d) {
@@ -1618,6 +1625,9 @@ inline bool ragged_ring_ok(const GemmDesc& d) {
   const int64_t mnk = d.M * d.N * d.K * d.batch;
   if (d.K < 64 || !(akc || d.sam == 1) || !(bkc || d.sbn == 1) || mnk >= (1ll << 34)) return false;
   if (d.sam < 0 || d.sak < 0 || d.sbk < 0 || d.sbn < 0) return false;
+  // K-rows that all start at one element (an operand expanded over K) would all be cut off at
+  // the end of the resource, not only the last one, which is patched (setup_operands)
+  if ((!akc && d.sak == 0) || (!bkc && d.sbk == 0)) return false;
   if (padded_b_inplace(d)) {
     const bool skinny_m = d.batch == 1 && d.M <= 128;  // packed A goes on to split-K
     if (mnk >= (1ll << 30) && !akc) return false;

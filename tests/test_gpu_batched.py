@@ -88,3 +88,27 @@ def test_dense_short_k(gpu):
     out = kore_amd.gemm(a.to(gpu), w.to(gpu).t())
     from oracle.gemm import matmul_ref
     verdict(out, matmul_ref(a, w.t()), "gemm", "bf16", "short-K dense 4000x4104x128")
+
+
+@pytest.mark.parametrize("Bn,M,N,K", [(3, 129, 64, 64), (2, 64, 255, 65), (5, 128, 128, 96), (2, 300, 513, 1001)])
+@pytest.mark.parametrize("kind", ["a over k", "b over k", "both over k", "a over m", "a over batch"])
+def test_batched_repeated_operands(gpu, Bn, M, N, K, kind):
+    """Operands expanded along K, along the rows or over the batch (strides of 0): odd and even
+    M and N, with and without a K tail."""
+    g = torch.Generator().manual_seed(M + N + K)
+    a, b = torch.randn((Bn, M, K), generator=g).bfloat16(), (torch.randn((Bn, N, K), generator=g) / K ** 0.5).bfloat16()
+    ag, bg = a.to(gpu), b.to(gpu)
+
+    def over_k(t):
+        return t[..., 0].contiguous()[..., None].expand(t.shape)
+
+    if kind in ("a over k", "both over k"):
+        a, ag = over_k(a), over_k(ag)
+    if kind in ("b over k", "both over k"):
+        b, bg = over_k(b), over_k(bg)
+    if kind == "a over m":
+        a, ag = a[:, :1].expand(a.shape), ag[:, :1].expand(a.shape)
+    if kind == "a over batch":
+        a, ag = a[:1].expand(a.shape), ag[:1].expand(a.shape)
+    out = kore_amd.batched_gemm(ag, bg).cpu()
+    pair_only(out, batched_gemm_ref(a.contiguous(), b.contiguous()), "bf16", f"{kind} B{Bn} {M}x{N}x{K}")

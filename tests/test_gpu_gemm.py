@@ -851,3 +851,69 @@ def test_gemm_ragged_ring(gpu, layout, M, N, K):
         want[M - 1, :] = True
         want[:, N - 1] = True
         assert torch.equal(got.isinf(), want)
+
+
+# Operands that repeat elements: an index of stride 0 (a vector expanded over the columns or
+# the rows, as the gradient of a broadcast gives) and overlapping windows (stride 2 < row length).
+_REPEATED = {
+    "a over k": lambda s, M, N, K: (s[:M][:, None].expand(M, K), None),
+    "a over m": lambda s, M, N, K: (s[:K][None, :].expand(M, K), None),
+    "a windows": lambda s, M, N, K: (s.as_strided((M, K), (1, 2)), None),
+    "b over k": lambda s, M, N, K: (None, s[:N][None, :].expand(K, N)),
+    "b over n": lambda s, M, N, K: (None, s[:K][:, None].expand(K, N)),
+    "b windows": lambda s, M, N, K: (None, s.as_strided((K, N), (2, 1))),
+}
+
+
+@pytest.mark.parametrize("kind", sorted(_REPEATED) + ["both over k"])
+@pytest.mark.parametrize("M,N,K", [(129, 127, 64), (128, 128, 200), (33, 7, 65), (256, 255, 320), (257, 96, 128),
+                                   (300, 1003, 1001), (513, 512, 1000), (2049, 1001, 100)])
+def test_gemm_repeated_operands(gpu, kind, M, N, K):
+    """An operand whose stride along K (or M, N) is 0 or smaller than its row: odd and even M
+    and N on both sides of 128, K tails, the other operand along either index, every type.
+    With a stride of 0 along K every K-row ends where the operand ends, and every one of them
+    has to count in the last row and column."""
+    g = torch.Generator().manual_seed(M + N + K)
+    for dtype, name in ((torch.bfloat16, "bf16"), (torch.float16, "fp16"), (torch.float32, "fp32")):
+        src = (torch.randn((M + 2 * N + 4 * K,), generator=g) / K ** 0.5).to(dtype)
+        srcg = src.to(gpu)
+        if kind == "both over k":
+            a, b = _REPEATED["a over k"](src, M, N, K)[0], _REPEATED["b over k"](src[M:], M, N, K)[1]
+            operands = [(_REPEATED["a over k"](srcg, M, N, K)[0], _REPEATED["b over k"](srcg[M:], M, N, K)[1])]
+        else:
+            a, b = _REPEATED[kind](src, M, N, K)
+            ag, bg = _REPEATED[kind](srcg, M, N, K)
+            full = torch.randn((M, K) if a is None else (K, N), generator=g).to(dtype)
+            fg = full.to(gpu)
+            a, b = (full, b) if a is None else (a, full)
+            operands = [(f, bg) if ag is None else (ag, f) for f in (fg, fg.t().contiguous().t())]
+        bias = torch.randn((N,), generator=g).to(dtype)
+        ref = gemm_fusion_ref(a.contiguous(), b.contiguous(), bias, "relu")
+        for x, w in operands:
+            out = kore_amd.gemm_fused(x, w, bias.to(gpu), "relu")
+            label = f"{kind} {name} {M}x{N}x{K} strides {x.stride()} {w.stride()}"
+            if dtype == torch.float32:
+                # Two fp32 sums of K products and a bias differ by at most 2 (K + 1) u S (u = 2^-24,
+                # S the sum of the magnitudes); relu does not widen that.  A relative bound at
+                # results that cancel to near zero would be none.
+                mag = a.abs().double() @ b.abs().double() + bias.abs().double()
+                assert bool(((out.cpu().double() - ref.double()).abs() <= 2 * (K + 1) * 2.0 ** -24 * mag).all()), label
+            else:
+                pair_only(out.cpu(), ref, name, label)
+
+
+@pytest.mark.parametrize("sbk", [0, 8])
+def test_gemm_repeated_b_infinity(gpu, sbk):
+    """A large product with a K tail whose B has K-rows that start 0 or 8 elements apart: no
+    element of B may meet the padding of a packed A, so an infinity stays one in its own
+    columns and reaches no other."""
+    M, N, K = 512, 512, 1001
+    src = torch.full((N + sbk * K,), 0.5, dtype=torch.bfloat16)
+    src[sbk * (K - 1) + 40] = float("inf")  # (K - 1, 40), and with windows (K - 2, 48), ...
+    a = torch.full((M, K), 0.25, dtype=torch.bfloat16)
+    b, bg = src.as_strided((K, N), (sbk, 1)), src.to(gpu).as_strided((K, N), (sbk, 1))
+    ref = matmul_ref(a, b.contiguous())
+    ag = a.to(gpu)
+    for x in (ag, ag.t().contiguous().t()):
+        out = kore_amd.gemm(x, bg).cpu()
+        assert torch.equal(out.isnan(), ref.isnan()) and torch.equal(out.isinf(), ref.isinf())

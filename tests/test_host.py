@@ -194,6 +194,31 @@ def test_gemm_workspace_queries_without_gpu(lib):
                                                   0, 4096, 4096) == 0
 
 
+def test_gemm_repeated_operand_routes_without_gpu(lib):
+    """Operands expanded over K (a K-row stride of 0) leave the ring that reads K-rows in place,
+    which patches the end of the last K-row alone: they are packed, here or by the batch.  The
+    same with a K-row stride of 1 or more stays in place.  A large K tail packs a B whose
+    K-rows overlap along with A, since the padding behind its last K-row reads B itself."""
+    fake = ctypes.c_void_p(256)
+
+    def need(sam, sak, sbk, sbn, M, N, K):
+        return lib.kore_gemm_workspace_bytes(0, 0, fake, sam, sak, fake, sbk, sbn, None, fake, N, M, N, K)
+
+    M, N, K = 513, 515, 1001
+    kp = 1024
+    both = kp * 2 * (M + N)
+    for strides in ((1, 0, N, 1), (K, 1, 0, 1), (1, 0, 0, 1), (1, 0, 1, K)):
+        assert both <= need(*strides, M, N, K) <= both + 1024, strides
+    for strides in ((1, M, N, 1), (K, 1, N, 1), (K, 1, 1, K), (1, 2, N, 1), (K, 1, 2, 1), (0, 1, 1, 0)):
+        assert need(*strides, M, N, K) == 0, strides
+    N = 512
+    for sbk in (0, 8):
+        assert kp * 2 * (M + N) <= need(1, 0, sbk, 1, M, N, K) <= kp * 2 * (M + N) + 1024
+    assert kp * 2 * M <= need(1, 0, N, 1, M, N, K) <= kp * 2 * M + 1024
+    assert lib.kore_batched_gemm_workspace_bytes(0, fake, 0, 1, 0, fake, 515 * K, K, 1, fake, 513 * 515, 515,
+                                                 4, 513, 515, K) >= 4 * kp * 2 * (513 + 515)
+
+
 # --------------------------------------------------------------------------- #
 # drop-in candidates: signatures and the reference's static scanner rules
 # (kore/reward/reward.py:70-179, restated)
