@@ -1610,35 +1610,65 @@ inline bool padded_fits(const GemmDesc& d) {
   const int64_t Kp = (d.K + 63) / 64 * 64;
   return d.M < (1ll << 31) && d.N < (1ll << 31) && Kp * 2 * 256 + Kp * 2 < (1ll << 31) && d.batch <= 65535;
 }
+// ---------------------------------------------------------------------------------
+// Estimated times in us, by which the dispatch picks among the kernels that can take a
+// 16-bit problem: a fixed part, the rounds of tiles that a CU runs one after the other (each
+// with its own fixed part and its K steps), and what is streamed from memory.  The constants
+// were fitted (bf16, one process) to the geometric mean of repeated calls and of calls after
+// a 512 MiB flush, over 3,100 drawn shapes in every layout; over those, picking by them costs
+// 1% against the faster of ring and pack.
+// ---------------------------------------------------------------------------------
+constexpr struct {
+  int bm, bn;
+  double us, ns;  // of a round: fixed part, one column of K
+} kTileCost[] = {{256, 256, 12.6, 17.5}, {256, 128, 6.3, 17.0}, {128, 128, 3.4, 9.1}, {64, 128, 2.7, 5.5}, {32, 128, 1.7, 4.0}};
+inline double tile_rounds(const GemmDesc& d, TileShape t) {
+  const int64_t bm = kTileCost[t].bm, bn = kTileCost[t].bn, cus = device_cus();
+  return (double)(((d.M + bm - 1) / bm * ((d.N + bn - 1) / bn) * d.batch + cus - 1) / cus);
+}
+inline double tiles_us(const GemmDesc& d, TileShape t) {
+  return 2.3 + tile_rounds(d, t) * (kTileCost[t].us + (double)d.K * kTileCost[t].ns * 1e-3);
+}
+// Pack passes (re-striding K-contiguous rows moves 4.8 TB/s, transposing 3.3), then the tiles.
+inline double packed_us(const GemmDesc& d) {
+  const bool akc = d.sak == 1, bkc = d.sbk == 1;
+  double us = 5.3 + tiles_us(d, pick_tile(d)) + (double)(d.batch * d.M * d.K * 4) / (akc ? 4.8e6 : 3.3e6);
+  if (!padded_b_inplace(d))
+    us += (bkc ? 3.2 : 7.4) + (double)(d.batch * d.N * d.K * 4) / (bkc ? 4.8e6 : 3.3e6);
+  return us;
+}
+// Ring tiles that read their rows in place at any alignment; an M-contiguous A has 128x128
+// tiles only.
+inline double ragged_ring_us(const GemmDesc& d) {
+  TileShape t = d.sak != 1 ? TILE_128x128 : pick_tile(d);
+  if (t == TILE_256x256) t = TILE_256x128;
+  const bool in_place = padded_b_inplace(d);
+  const double slow = d.sak != 1 ? (in_place ? 0.97 : 1.11) : d.sbk == 1 ? 1.72 : in_place ? 1.3 : 1.45;
+  return 2.3 + tile_rounds(d, t) * (5.3 + (double)d.K * kTileCost[t].ns * 1e-3 * slow);
+}
 // Ragged ring: operands with a unit stride along either index, at any 2-byte alignment, any
 // sizes with K >= 64, read in place (the K-tail mode of the deep ring; rows that are K-rows
-// may have any length).  Against the pack pass and its launches, or the generic kernel, one
-// process: backward 273 x 455 x 320 58.7 -> 16.2 us, 504 x 1472 x 2991 63.7 -> 33.6, linear
-// 1026 x 5663 x 768 41.6 -> 21.7, 6520 x 1247 x 1231 63.7 -> 45.1, batched 55 x 832 x 320 x 82
-// 70.8 -> 30.2.  Packed operands run the faster 256x256 tiles, so they stay from 2^34 products
-// on (4097^3); where B is read in place anyway, from 2^30 on for an M-contiguous A (dW of a
-// 300 x 4096 x 4096 backward, 57.7 against 63.7 us for the two) and for few tiles along a long
-// K, which reads misaligned rows of A once per column tile (496 x 768 x 9657 44.2 against
-// 46.5).  Two misaligned K-contiguous operands along a long K are packed too.
+// may have any length).  Against the generic kernel, which takes what is too small to pack,
+// and against the pack pass where it is estimated faster; one process: backward 273 x 455 x
+// 320 58.7 -> 16.2 us, linear 1026 x 5663 x 768 41.6 -> 21.7, 6520 x 1247 x 1231 63.7 -> 45.1,
+// batched 55 x 832 x 320 x 82 70.8 -> 30.2.  A long K stays with the pack pass, which reads
+// misaligned rows once and not once per tile (A along M, repeated / flushed: 448 x 449 x 4689
+// 58 / 76 us on the ring, 35 / 40 packed; both along K, 320 x 192 x 9423 67 / 98 against
+// 54 / 54).  Packed operands run the faster 256x256 tiles, so they stay from 2^34 products on
+// (4097^3).
 inline bool ragged_ring_ok(const GemmDesc& d) {
   const bool akc = d.sak == 1, bkc = d.sbk == 1;
-  const int64_t mnk = d.M * d.N * d.K * d.batch;
-  if (d.K < 64 || !(akc || d.sam == 1) || !(bkc || d.sbn == 1) || mnk >= (1ll << 34)) return false;
+  if (d.K < 64 || !(akc || d.sam == 1) || !(bkc || d.sbn == 1) || d.M * d.N * d.K * d.batch >= (1ll << 34)) return false;
   if (d.sam < 0 || d.sak < 0 || d.sbk < 0 || d.sbn < 0) return false;
   // K-rows that all start at one element (an operand expanded over K) would all be cut off at
   // the end of the resource, not only the last one, which is patched (setup_operands)
   if ((!akc && d.sak == 0) || (!bkc && d.sbk == 0)) return false;
-  if (padded_b_inplace(d)) {
-    const bool skinny_m = d.batch == 1 && d.M <= 128;  // packed A goes on to split-K
-    if (mnk >= (1ll << 30) && !akc) return false;
-    if (mnk >= (1ll << (skinny_m ? 27 : 30)) && (skinny_m || d.K >= 2048) &&
-        (d.M + 127) / 128 * ((d.N + 127) / 128) * d.batch < 64)
-      return false;
-  }
-  if (akc && bkc && d.K >= 4000 && mnk >= (1ll << 30)) return false;
   const int64_t lim = 1ll << 31;
-  return (akc ? d.sam * 2 * 256 + d.K * 2 : d.sak * 2 * (d.K + 64) + 512) < lim &&
-         (bkc ? d.sbn * 2 * 256 + d.K * 2 : d.sbk * 2 * (d.K + 64) + 512) < lim;
+  if ((akc ? d.sam * 2 * 256 + d.K * 2 : d.sak * 2 * (d.K + 64) + 512) >= lim ||
+      (bkc ? d.sbn * 2 * 256 + d.K * 2 : d.sbk * 2 * (d.K + 64) + 512) >= lim)
+    return false;
+  // (by a twentieth: what the two estimates differ by where they are off)
+  return d.M * d.N * d.K < (1ll << 27) || !padded_fits(d) || 1.05 * ragged_ring_us(d) < packed_us(d);
 }
 template <typename T>
 int launch_ragged_ring(const GemmDesc& d, hipStream_t stream) {

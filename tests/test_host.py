@@ -219,6 +219,21 @@ def test_gemm_repeated_operand_routes_without_gpu(lib):
                                                  4, 513, 515, K) >= 4 * kp * 2 * (513 + 515)
 
 
+@pytest.mark.parametrize("M,N,K,a_along_m,b_along_n,packed", [
+    (448, 449, 4689, True, False, True), (340, 448, 7851, True, False, True), (387, 64, 9344, True, True, True),
+    (320, 192, 9423, False, False, True), (576, 320, 3653, True, True, True), (300, 8064, 425, True, True, False),
+    (504, 1472, 700, True, False, False), (6520, 1247, 1231, False, True, False), (1026, 5663, 768, False, True, False),
+    (455, 320, 273, True, True, False)])
+def test_gemm_long_k_packs_without_gpu(lib, M, N, K, a_along_m, b_along_n, packed):
+    """Ragged operands with a long K are packed once instead of being read misaligned once per
+    tile; the same layouts with a short K stay on the ring, in place (no workspace)."""
+    fake = ctypes.c_void_p(256)
+    a = (1, M) if a_along_m else (K, 1)
+    b = (N, 1) if b_along_n else (1, K)
+    need = lib.kore_gemm_workspace_bytes(0, 0, fake, *a, fake, *b, None, fake, N, M, N, K)
+    assert need >= M * K * 2 if packed else need == 0
+
+
 # --------------------------------------------------------------------------- #
 # drop-in candidates: signatures and the reference's static scanner rules
 # (kore/reward/reward.py:70-179, restated)
