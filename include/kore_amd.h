@@ -73,8 +73,8 @@ int kore_abi_version(void);
  * very large problems and other layouts are packed into `workspace` first where the
  * packed engines are faster, and small problems without a unit stride run a slower
  * generic kernel.  M <= 128 in 16 bits streams the weights through one kernel without
- * scratch, or splits K and sums fp32 partials held in `workspace`, whichever is
- * estimated faster.  M, N >= 1, K >= 0 (K == 0 gives act(bias); a and b
+ * scratch where that is estimated faster than the tiles and than splitting K, which sums
+ * fp32 partials held in `workspace`.  M, N >= 1, K >= 0 (K == 0 gives act(bias); a and b
  * may then be NULL).  `workspace` must hold kore_gemm_workspace_bytes(<same args>).
  * Replaces: gemm(a, b)            kore/tasks/gemm_bf16/seed_triton.py:64-86
  *           <op>(a, b[, bias])    kore/tasks/_genops.py:715-731 (_GEMM_TMPL entry,

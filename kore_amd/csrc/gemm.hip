@@ -1445,82 +1445,6 @@ int launch_skinny(const GemmDesc& d, hipStream_t stream) {
   return check_launch("gemm_skinny_kernel");
 }
 
-// Columns per workgroup (16 nb) of the skinny kernel, by its estimated time in us: a fixed
-// 2.5 us, and the longer of what a CU takes in for its workgroups, (M + 16 nb) rows of K, at
-// 60 (M <= 32) or 70 KB/us, and the weights' stream at 5.6 TB/s; rows off 16-byte alignment
-// cost half as much again.  Measured (bf16, one process, M = 1 / 16 / 64 / 128), nb = 1 | 2 | 4:
-//   4096 x 4096     6.6 7.4 11.3 18.0 | 6.5 9.7 14.7 21.6 | 12.1 13.8 20.1 33.0
-//   7168 x 2048     7.9 8.5 13.2 19.3 | 6.5 6.8  9.0 12.9 |  8.1  8.6 11.7 19.8
-//   14336 x 4096   23.2 25.8 45.7 69.2 | 23.0 24.6 33.8 46.0 | 19.2 19.3 25.0 35.0
-// and 4096 x 4095 (odd rows) 8.2 10.6 18.0 28.6 with nb = 1.
-struct SkinnyPick {
-  int nb;
-  double us;
-};
-inline SkinnyPick pick_skinny(const GemmDesc& d, bool aligned, int64_t cus) {
-  const double stream_us = (double)(d.N * d.K * 2) / 5.6e6;
-  SkinnyPick best{1, 1e300};
-  for (int nb : {1, 2, 4}) {
-    const int64_t wgs = (d.N + 16 * nb - 1) / (16 * nb);
-    const double intake_us = (double)((wgs + cus - 1) / cus * (d.M + 16 * nb) * d.K * 2) / (d.M <= 32 ? 60e3 : 70e3);
-    const double us = 2.5 + std::max(intake_us, stream_us) * (aligned ? 1.0 : 1.5);
-    if (us < best.us) best = {nb, us};
-  }
-  return best;
-}
-// Estimated time of the path an aligned problem (K % 64 == 0) takes otherwise.  32x128 ring
-// tiles: 3 us and 160 rows of K per round at 80 KB/us (bf16 200 x 4096 x 4096 19.4, 64 x
-// 14336 x 4096 20.3, 100 x 14336 x 4096 36.7, 128 x 8192 x 8192 34.5, 100 x 7168 x 2048 11.3
-// us).  With K split (few tiles): two launches, about 8 us back to back, and a share of the
-// weights' stream (32 x 4096 x 4096 11.3, 64 14.6, 128 19.6; 32 x 2048 x 7168 11.2, 64 12.6;
-// 64 x 1024 x 8192 10.0, 128 11.5 us).  Wider problems run the mid-size
-// tiles, which win from M = 33 on.
-inline double skinny_alternative_us(const GemmDesc& d, int64_t cus, double beyond_caches = 1.2) {
-  const int64_t t32 = (d.M + 31) / 32 * ((d.N + 127) / 128);
-  if ((d.M + 127) / 128 * ((d.N + 127) / 128) >= 128) return d.M <= 32 ? 1e300 : 0.0;
-  if (d.K >= 1024 && t32 * 2 <= cus) {
-    // (beyond the 48 MB or so that caches help with, M = 1: 8192 x 8192 45.7 us, N-contiguous 24.7)
-    const double bytes = (double)(d.N * d.K * 2);
-    return 8.0 + bytes / 5.6e6 * (d.M <= 32 ? (bytes > 48e6 ? beyond_caches : 0.4) : d.M <= 64 ? 1.0 : 1.8);
-  }
-  return 3.0 + (double)((t32 + cus - 1) / cus * 160 * d.K * 2) / 80e3;
-}
-// The same for N-contiguous B: 2 us per round plus the longest of the weights' stream
-// (slower through short row pieces: 32, 64 or 128 bytes), a workgroup's own weights (64-column
-// ones leave CUs idle and pull 30 KB/us), and what a CU takes in, at 65 KB/us with most CUs
-// busy; misaligned rows cost half as much again.  Measured (bf16, M = 1 / 16 / 64 / 128, best
-// nb) against the split-K, ring, tile, packed and generic paths: 4096 x 1024 4.7 4.7 5.2 6.8
-// (8.4 8.5 9.0 12.2), 1024 x 1024 4.2 4.2 4.3 6.5 (7.9 8.0 8.2 8.3), 7168 x 2048 6.4 6.9 9.2
-// 12.9 (9.6 9.7 15.2 11.4), 4096 x 4096 8.6 10.4 14.0 18.7 (10.2 9.9 14.9 19.5), 823 x 1984 5.4
-// 5.4 7.6 10.2 (96 96 99 21), 320 x 1816 4.5 4.5 5.8 9.5 (24), 9473 x 565 6.2 6.4 9.3 13.5 (33
-// 32 21 22), 4096 x 4095 8.8 11.2 18.2 27.3 (191 21.5 21.9 22.0 us).
-inline SkinnyPick pick_skinny_nc(const GemmDesc& d, bool a_ok, bool b_nc, int64_t cus) {
-  SkinnyPick best{1, 1e300};
-  for (int nb : {1, 2, 4}) {
-    const int64_t bn = 16 * nb, wgs = (d.N + bn - 1) / bn, rounds = (wgs + cus - 1) / cus;
-    const double k2 = (double)(d.K * 2);
-    const double stream = (double)d.N * k2 / (nb == 1 ? 4.2e6 : nb == 2 ? 5.5e6 : 5.8e6);
-    const double own = (double)(rounds * bn) * k2 / (nb == 4 ? 30e3 : 60e3);
-    const double intake = (double)(rounds * (d.M + bn)) * k2 / (wgs >= 128 ? 65e3 : 105e3);
-    double slow = 1.0;
-    if (!a_ok) slow += 0.5 * (double)d.M / (double)(d.M + bn);
-    if (!b_nc) slow += 0.5 * (double)bn / (double)(d.M + bn);
-    const bool two_waves = nb == 4 && d.M > 64;  // what the LDS holds
-    double us = std::max(std::max(stream, own), two_waves ? 1.35 * intake : intake) * slow;
-    us += 0.5 + 2.0 * (double)rounds + (two_waves ? 2.0 : 0.0);
-    if (us < best.us) best = {nb, us};
-  }
-  return best;
-}
-// Its alternatives: the aligned paths, or with rows off 16-byte alignment a pack of A (and of
-// B unless it is read in place) before them; small unaligned problems have only the generic
-// kernel, one workgroup per 128 x 128 tile.
-inline double skinny_nc_alternative_us(const GemmDesc& d, bool aligned, bool b_nc, int64_t cus) {
-  const double us = d.K < 512 ? 5.5 : skinny_alternative_us(d, cus, 0.7);
-  if (aligned) return us;
-  if (d.M * d.N * d.K < (1ll << 27)) return 1e300;
-  return us + 6.0 + (b_nc ? 0.0 : 2.0 + (double)(d.N * d.K * 4) / 4.5e6);
-}
 template <typename T, int BL>
 int launch_skinny_nb(const GemmDesc& d, int nb, hipStream_t st) {
   // waves and stages per configuration: as much in flight as 160 KiB of LDS holds
@@ -1615,8 +1539,8 @@ inline bool padded_fits(const GemmDesc& d) {
 // 16-bit problem: a fixed part, the rounds of tiles that a CU runs one after the other (each
 // with its own fixed part and its K steps), and what is streamed from memory.  The constants
 // were fitted (bf16, one process) to the geometric mean of repeated calls and of calls after
-// a 512 MiB flush, over 3,100 drawn shapes in every layout; over those, picking by them costs
-// 1% against the faster of ring and pack.
+// a 512 MiB flush, over 6,500 drawn shapes in every layout; over those, picking by them costs
+// 1% against the faster of ring and pack, and 1 to 2% against the fastest kernel for M <= 128.
 // ---------------------------------------------------------------------------------
 constexpr struct {
   int bm, bn;
@@ -1718,6 +1642,92 @@ int launch_padded(const GemmDesc& d, Ws& ws, hipStream_t stream) {
   return rc;
 }
 
+// Split-K over 32x128 tiles, one slice of K per workgroup; one tile of 64 or 128 rows where
+// 32-row tiles would read a large weight matrix two to four times (N-contiguous B, same
+// process: 64 x 4096 x 4096 17.3 -> 14.6 us, 128 x 4096 x 4096 28.6 -> 19.6 us, with a slice
+// of K for every other CU: twice the slices, 15.8 and 23.7 us, write and read more partials
+// than they save).  32 rows stay for weights up to 24 MB (64 x 1024 x 8192 9.9 against 11.0
+// us) and where they leave at least five slices of K (64 x 2048 x 7168 13.1 against 14.5 us).
+struct SplitPlan {
+  int rows, splits, kper;
+};
+inline SplitPlan splitk_plan(const GemmDesc& d) {
+  const int64_t cus = device_cus(), nk = d.K / 64, tn = (d.N + 127) / 128, t32 = (d.M + 31) / 32 * tn;
+  const bool tall = d.M > 32 && d.M <= 128 && t32 * 4 >= cus && d.N * d.K * 2 > (24ll << 20);
+  const int64_t want = tall ? std::max<int64_t>(1, std::min<int64_t>(cus / 2 / tn, nk / 4))
+                            : std::min<int64_t>(cus / t32, nk / 4);
+  const int64_t per = (nk + want - 1) / want;
+  return {!tall ? 32 : d.M <= 64 ? 64 : 128, (int)((nk + per - 1) / per), (int)per * 64};
+}
+
+// Skinny kernel: columns per workgroup (16 nb) and estimated time.  A round of workgroups has
+// a fixed part and takes in (M + 16 nb) rows of K per CU, at 50 to 60 KB/us, a quarter more
+// where half of the CUs have none (64-column workgroups of many rows have fewer waves to do
+// it, and few of them do not reach the memory's rate); rows off 16-byte alignment cost 1.4
+// times as much.  N-contiguous weights cost a workgroup one cache line per K-row however few
+// of its columns it owns, and up to two where the rows start off the 128-byte lines: that
+// slows their stream and what one workgroup gets of it.  Measured (bf16, one process,
+// repeated / flushed calls), nb = 1 | 2 | 4:
+//   W.t() 4 x 4096 x 4096     6.9 / 12.0 |  6.7 / 11.1 | 12.4 / 16.1
+//   W.t() 16 x 14336 x 2048  16.0 / 19.4 | 12.7 / 16.1 | 11.0 / 14.6
+//   W.t() 96 x 9024 x 512    11.9 / 16.3 | 10.8 / 14.2 |  9.2 / 12.2
+//   W.t() 32 x 32000 x 1024  24.7 / 28.4 | 17.1 / 20.5 | 13.7 / 17.6
+//   [K,N] 32 x 5120 x 1536    8.5 / 19.5 |  5.1 / 14.8 |  6.7 / 14.5
+//   [K,N] 16 x 17000 x 4096  90.6 / 101  | 60.2 / 72.1 | 56.4 / 59.5
+struct SkinnyPick {
+  int nb;
+  double us;
+};
+// rows16: 16-byte rows, of both operands or, for N-contiguous weights, of A
+inline SkinnyPick pick_skinny(const GemmDesc& d, bool nc, bool rows16) {
+  static const double nc_stream[] = {2.0e6, 2.8e6, 4.6e6}, nc_own[] = {23e3, 42e3, 50e3}, off_lines[] = {1.4, 1.4, 1.8};
+  const int64_t cus = device_cus();
+  const bool lines = d.sbk % 64 == 0 && ((uintptr_t)d.b & 127u) == 0;
+  SkinnyPick best{1, 1e300};
+  for (int i = 0; i < 3; ++i) {
+    const int64_t nb = 1 << i, bn = 16 * nb, wgs = (d.N + bn - 1) / bn, rounds = (wgs + cus - 1) / cus;
+    const double rows = (double)(d.M + bn);
+    const double few_waves = nb < 4 || d.M <= 32 ? 1.0 : d.M <= 64 ? (nc ? 1.25 : 1.1) : (nc ? 1.6 : 1.4);
+    double k = (double)(d.K * 2), us;  // bytes of a row
+    if (nc) {
+      const double off = lines ? 1.0 : off_lines[i];
+      if (!rows16) k *= 1.0 + 0.4 * (double)d.M / rows;
+      us = 1.9 + std::max((double)rounds * (2.1 + few_waves * k * std::max(rows / 50e3, off * (double)bn / nc_own[i])),
+                          k * off * (double)d.N / nc_stream[i]);
+    } else {
+      if (!rows16) k *= 1.4;
+      const double rate = (nb == 1 ? 60e3 : 51e3) * (nb < 4 && 2 * wgs < cus ? 1.25 : 1.0);
+      const double stream = nb < 4 ? 5.2e6 : 5.5e6 * std::min(1.0, (double)wgs / (0.6 * (double)cus));
+      us = 2.7 + std::max((double)rounds * (1.5 + few_waves * k * rows / rate), k * (double)d.N / stream);
+    }
+    if (us < best.us) best = {(int)nb, us};
+  }
+  return best;
+}
+// Estimated time of the route that an M <= 128 problem takes otherwise (the order is that of
+// dispatch_typed below); `rows_ok`: 16-byte rows and K % 8 == 0.
+inline double skinny_alternative_us(const GemmDesc& d, bool nc, bool rows_ok) {
+  const int64_t cus = device_cus(), mid = (d.M + 127) / 128 * ((d.N + 127) / 128);
+  const int64_t t32 = (d.M + 31) / 32 * ((d.N + 127) / 128);
+  const double mb = (double)(d.N * d.K * 2) * 1e-6;
+  const bool deep = mid >= 128 && d.K >= 256;
+  if (rows_ok && d.K % 64 == 0) {
+    if (deep) return std::max(tiles_us(d, pick_tile(d)), 4.9 + mb / 4.1);
+    if (mid < 128 && d.K >= 1024 && t32 * 2 <= cus) {
+      const SplitPlan s = splitk_plan(d);
+      const bool tall = s.rows > 32;
+      return (tall ? 4.0 : 6.0) + std::max(s.kper * 8.5e-3, mb / (tall ? 5.3 : 6.1)) +
+             (double)(d.M * d.N * s.splits * 8) / (tall ? 1.6e6 : 2.8e6);
+    }
+    if (mid < 128 && d.K >= 512) return 3.5 + std::max((double)((t32 + cus - 1) / cus * d.K) * 6.5e-3, mb / 3.5);
+  }
+  if (rows_ok && !deep) return mid < 128 ? 3.5 + (double)d.K * (nc ? 12.7e-3 : 8.5e-3) + mb / 8.0 : 5.4 + mb / 3.2;
+  // (the weights' stream, which few and misaligned tiles read slowly, beside the tiles' time)
+  const double ring = std::max(ragged_ring_us(d), 2.3 + mb / (nc ? 2.9 : 1.9));
+  if (deep) return std::max(ring, 7.0 + mb / 4.1);
+  return d.M * d.N * d.K < (1ll << 27) ? ring : std::min(ring, packed_us(d) + mb / 4.1);
+}
+
 // Picks the kernel path for d and launches it; in plan mode (ws.plan) it launches
 // nothing and only records the workspace that path needs.
 template <typename T>
@@ -1728,41 +1738,30 @@ int dispatch_typed(const GemmDesc& d, Ws& ws, hipStream_t stream) {
   const bool b_kc = d.sbk == 1 && d.sbn % 8 == 0 && aligned16(d.b) && d.sb % 8 == 0;
   const bool b_nc = d.sbn == 1 && d.sbk % 8 == 0 && aligned16(d.b) && d.sb % 8 == 0 && d.N % 8 == 0;
   const bool fits32 = d.M < (1ll << 31) && d.N < (1ll << 31) && d.K < (1ll << 31);
-  // M <= 128 against K-contiguous weights: the skinny kernel, unless the aligned paths below
-  // are estimated faster, or K < 512: 64x64 tiles then, which have no cross-wave sum to pay
-  // for (20 x 11000 x 256 4.8 us against 6.0).
-  if (d.batch == 1 && d.sak == 1 && d.sbk == 1 && d.M <= 128 && d.K >= 64 && fits32 &&
-      (d.sam >= d.K || d.M == 1) && (d.sbn >= d.K || d.N == 1) && d.M * d.sam * 2 + d.K * 2 < (1ll << 31) &&
-      64 * d.sbn * 2 + d.K * 2 < (1ll << 31)) {
-    const bool aligned = a_ok && b_kc && d.K % 64 == 0;
-    if (!aligned || d.K >= 512) {
-      const int64_t cus = device_cus();
-      const SkinnyPick k = pick_skinny(d, aligned, cus);
-      if (!aligned || k.us < skinny_alternative_us(d, cus)) {
+  // M <= 128: the skinny kernel where it is estimated faster than the paths below.
+  const bool a16 = d.sam % 8 == 0 && aligned16(d.a), skinny_a = d.batch == 1 && d.sak == 1 && d.M <= 128 &&
+             d.K >= 64 && fits32 && (d.sam >= d.K || d.M == 1) && d.M * d.sam * 2 + d.K * 2 < (1ll << 31);
+  if (skinny_a && d.sbk == 1 && (d.sbn >= d.K || d.N == 1) && 64 * d.sbn * 2 + d.K * 2 < (1ll << 31)) {
+    // K-contiguous weights.  K < 512: 64x64 tiles, which have no cross-wave sum to pay for
+    // (20 x 11000 x 256 4.8 us against 6.0).  More than 32 rows and 128 tiles of 128 columns:
+    // the mid-size tiles (repeated / flushed, 64 x 32000 x 4000 44.7 / 108 us against 65.5 /
+    // 70.2, 128 x 50257 x 1000 35 / 66 against 61 / 66, 128 x 32000 x 4096 51 / 128 against
+    // 74 / 79).
+    const bool rows_ok = a_ok && b_kc, wide = d.M > 32 && d.N > 127 * 128 && d.K >= 256;
+    if (!wide && (!rows_ok || d.K % 64 != 0 || d.K >= 512)) {
+      const SkinnyPick k = pick_skinny(d, false, a16 && b_kc);
+      if (k.us < skinny_alternative_us(d, false, rows_ok)) {
         if (ws.plan) return KORE_OK;
         return launch_skinny_nb<T, B_KC>(d, k.nb, stream);
       }
     }
   }
-  if (d.batch == 1 && d.sak == 1 && d.sbn == 1 && d.sbk != 1 && d.M <= 128 && d.K >= 64 && fits32 &&
-      (d.sam >= d.K || d.M == 1) && d.sbk >= d.N && d.M * d.sam * 2 + d.K * 2 < (1ll << 31) &&
-      (d.K + 64) * d.sbk * 2 < (1ll << 31)) {
-    const bool aligned = a_ok && b_nc && d.K % 64 == 0;
-    const int64_t cus = device_cus();
-    const SkinnyPick k = pick_skinny_nc(d, a_ok, b_nc, cus);
-    // Weights that come from memory cost a workgroup one cache line per K-row, however few of
-    // its columns it owns, so a long K is left to split-K, which gives the K-rows to more
-    // workgroups, unless many rows and columns pay for it.  512 MiB flushed before each call /
-    // repeated calls, split-K against this kernel in us: 1x4096x4096 13.4 / 9.4 against
-    // 22.7 / 8.7, 16x4096x2048 12.0 / 8.5 against 14.8 / 4.8, 128x2048x2048 14.4 / 9.7 against
-    // 20.0 / 12.0; on this kernel's side of the line 16x4096x1024 10.5 / 8.8 against 10.0 / 4.5,
-    // 64x8192x2048 21.0 / 17.0 against 19.8 / 9.9, 64x4096x2048 15.0 / 11.8 against 15.8 / 7.9.
-    // 65 rows and more on up to 2048 columns lose as well (128x1024x1024 10.8 against 11.7
-    // flushed, packed 128x2048x2047 13.8 against 15.8 repeated).
-    const bool packs = b_nc && d.M * d.N * d.K >= (1ll << 27);
-    const bool few = (aligned && d.K >= 2048 && (d.M <= 32 || d.N < 4096)) ||
-                     ((aligned || packs) && d.M > 64 && d.N <= 2048);
-    if (!few && k.us * 1.15 < skinny_nc_alternative_us(d, aligned, b_nc, cus)) {
+  if (skinny_a && d.sbn == 1 && d.sbk != 1 && d.sbk >= d.N && (d.K + 64) * d.sbk * 2 < (1ll << 31)) {
+    // N-contiguous weights, by a twentieth: at equal means this kernel is the slower one from
+    // memory (512 MiB flushed before each call / repeated, split-K against this kernel:
+    // 1x4096x4096 13.4 / 9.4 against 22.7 / 8.7 us).
+    const SkinnyPick k = pick_skinny(d, true, a16);
+    if (k.us * 1.05 < skinny_alternative_us(d, true, a_ok && b_nc)) {
       if (ws.plan) return KORE_OK;
       return launch_skinny_nb<T, B_NC>(d, k.nb, stream);
     }
@@ -1843,27 +1842,15 @@ int dispatch_typed(const GemmDesc& d, Ws& ws, hipStream_t stream) {
     // Few 32x128 tiles for the CUs and a long K (decode-sized M): split K.
     const int64_t t32 = ((d.M + 31) / 32) * ((d.N + 127) / 128);
     if (d.batch == 1 && (b_kc ? buf_ok : buf_nc_ok) && d.K >= 1024 && t32 * 2 <= device_cus()) {
-      const int nk = (int)(d.K / 64);
-      // One tile of 64 or 128 rows where 32-row tiles would read a large weight matrix two to
-      // four times (N-contiguous B, same process: 64 x 4096 x 4096 17.3 -> 14.6 us, 128 x
-      // 4096 x 4096 28.6 -> 19.6 us, with a slice of K for every other CU: twice the slices,
-      // 15.8 and 23.7 us, write and read more partials than they save).  32 rows stay for
-      // weights up to 24 MB (64 x 1024 x 8192 9.9 against 11.0 us) and where they leave at
-      // least five slices of K (64 x 2048 x 7168 13.1 against 14.5 us).
-      if (d.M > 32 && d.M <= 128 && t32 * 4 >= device_cus() && d.N * d.K * 2 > (24ll << 20)) {
-        const int64_t tn = (d.N + 127) / 128;
-        const int want = (int)std::max<int64_t>(1, std::min<int64_t>(device_cus() / 2 / tn, nk / 4));
-        const int per = (nk + want - 1) / want, splits = (nk + per - 1) / per;
-        if (d.M <= 64)
-          return b_kc ? launch_splitk<T, B_KC, 64, 128, 2, 2, 6>(d, splits, per * 64, ws, stream)
-                      : launch_splitk<T, B_NC, 64, 128, 2, 2, 6>(d, splits, per * 64, ws, stream);
-        return b_kc ? launch_splitk<T, B_KC, 128, 128, 2, 2, 4>(d, splits, per * 64, ws, stream)
-                    : launch_splitk<T, B_NC, 128, 128, 2, 2, 4>(d, splits, per * 64, ws, stream);
-      }
-      const int want = (int)std::min<int64_t>(device_cus() / t32, nk / 4);
-      const int per = (nk + want - 1) / want, splits = (nk + per - 1) / per;
-      return b_kc ? launch_splitk<T, B_KC, 32, 128, 1, 4, 7>(d, splits, per * 64, ws, stream)
-                  : launch_splitk<T, B_NC, 32, 128, 1, 4, 7>(d, splits, per * 64, ws, stream);
+      const SplitPlan sp = splitk_plan(d);
+      if (sp.rows == 64)
+        return b_kc ? launch_splitk<T, B_KC, 64, 128, 2, 2, 6>(d, sp.splits, sp.kper, ws, stream)
+                    : launch_splitk<T, B_NC, 64, 128, 2, 2, 6>(d, sp.splits, sp.kper, ws, stream);
+      if (sp.rows == 128)
+        return b_kc ? launch_splitk<T, B_KC, 128, 128, 2, 2, 4>(d, sp.splits, sp.kper, ws, stream)
+                    : launch_splitk<T, B_NC, 128, 128, 2, 2, 4>(d, sp.splits, sp.kper, ws, stream);
+      return b_kc ? launch_splitk<T, B_KC, 32, 128, 1, 4, 7>(d, sp.splits, sp.kper, ws, stream)
+                  : launch_splitk<T, B_NC, 32, 128, 1, 4, 7>(d, sp.splits, sp.kper, ws, stream);
     }
     if (ws.plan) return KORE_OK;
     // few tiles and a long K: the latency-bound case, on the deep direct-to-LDS ring

@@ -917,3 +917,28 @@ def test_gemm_repeated_b_infinity(gpu, sbk):
     for x in (ag, ag.t().contiguous().t()):
         out = kore_amd.gemm(x, bg).cpu()
         assert torch.equal(out.isnan(), ref.isnan()) and torch.equal(out.isinf(), ref.isinf())
+
+
+@pytest.mark.parametrize("dtype,act", [(torch.bfloat16, "gelu"), (torch.float16, "relu")])
+@pytest.mark.parametrize("M,N,K,layout", [(128, 4096, 4096, "kn"), (113, 4096, 8192, "nk"), (65, 4104, 4096, "kn"),
+                                          (113, 3996, 8192, "nk"), (64, 4096, 14336, "nk"), (60, 4100, 16384, "nk"),
+                                          (64, 4096, 8192, "kn"), (50, 4104, 8192, "kn")])
+def test_gemm_splitk_tall(gpu, dtype, act, M, N, K, layout):
+    """Split-K over one tile of 64 or 128 rows (M > 32 and more than 24 MiB of weights), both
+    weight layouts: full tiles, row remainders and an N off the 128-column tile.  The planned
+    workspace shows that the shape takes split-K: fp32 partials of two slices or more."""
+    from kore_amd import _lib
+    g = torch.Generator().manual_seed(M + N + K)
+    a = (torch.randn((M, K), generator=g) / K ** 0.5).to(dtype)
+    w = torch.randn((K, N) if layout == "kn" else (N, K), generator=g).to(dtype)
+    bias = torch.randn((N,), generator=g).to(dtype)
+    b, bd = (w, w.to(gpu)) if layout == "kn" else (w.t(), w.to(gpu).t())
+    ag = a.to(gpu)
+    out = kore_amd.gemm_fused(ag, bd, bias.to(gpu), act)
+    need = _lib.load().kore_gemm_workspace_bytes(0 if dtype == torch.bfloat16 else 1, 0, ag.data_ptr(), *ag.stride(),
+                                                 bd.data_ptr(), *bd.stride(), None, out.data_ptr(), out.stride(0),
+                                                 M, N, K)
+    assert need >= 2 * M * N * 4
+    name = "bf16" if dtype == torch.bfloat16 else "fp16"
+    pair_only(out.cpu(), gemm_fusion_ref(a, b, bias, act), name, f"tall split-K {M}x{N}x{K} {layout} {act}")
+    assert bit_equal(out, kore_amd.gemm_fused(ag, bd, bias.to(gpu), act))

@@ -234,6 +234,20 @@ def test_gemm_long_k_packs_without_gpu(lib, M, N, K, a_along_m, b_along_n, packe
     assert need >= M * K * 2 if packed else need == 0
 
 
+@pytest.mark.parametrize("M,N,K,b_along_n,split", [
+    (16, 2048, 12160, False, True), (32, 5120, 12160, False, True), (128, 2048, 8192, False, True),
+    (48, 5376, 5504, True, True), (16, 4096, 8192, True, True), (128, 4096, 4096, True, True),
+    (1, 4096, 4096, False, False), (64, 4096, 4096, False, False), (16, 14336, 4096, False, False),
+    (16, 4096, 1024, True, False), (64, 4096, 2048, True, False)])
+def test_gemm_skinny_route_without_gpu(lib, M, N, K, b_along_n, split):
+    """Both sides of the choice between the skinny kernel (no workspace) and split-K, at
+    shapes where the two are far apart."""
+    fake = ctypes.c_void_p(256)
+    b = (N, 1) if b_along_n else (1, K)
+    need = lib.kore_gemm_workspace_bytes(0, 0, fake, K, 1, fake, *b, None, fake, N, M, N, K)
+    assert need >= 2 * M * N * 4 if split else need == 0
+
+
 # --------------------------------------------------------------------------- #
 # drop-in candidates: signatures and the reference's static scanner rules
 # (kore/reward/reward.py:70-179, restated)
