@@ -1583,7 +1583,6 @@ inline double ragged_ring_us(const GemmDesc& d) {
 inline bool ragged_ring_ok(const GemmDesc& d) {
   const bool akc = d.sak == 1, bkc = d.sbk == 1;
   if (d.K < 64 || !(akc || d.sam == 1) || !(bkc || d.sbn == 1) || d.M * d.N * d.K * d.batch >= (1ll << 34)) return false;
-  if (d.sam < 0 || d.sak < 0 || d.sbk < 0 || d.sbn < 0) return false;
   // K-rows that all start at one element (an operand expanded over K) would all be cut off at
   // the end of the resource, not only the last one, which is patched (setup_operands)
   if ((!akc && d.sak == 0) || (!bkc && d.sbk == 0)) return false;
@@ -1732,6 +1731,16 @@ inline double skinny_alternative_us(const GemmDesc& d, bool nc, bool rows_ok) {
 // nothing and only records the workspace that path needs.
 template <typename T>
 int dispatch_typed(const GemmDesc& d, Ws& ws, hipStream_t stream) {
+  // Large problems in layouts that nothing below reads: pack, then the engines (small ones
+  // are cheaper on the generic kernel than a pack pass).
+  auto pack_or_generic = [&]() -> int {
+    if (d.M * d.N * d.K >= (1ll << 27) && d.K >= 64 && padded_fits(d)) return launch_padded<T>(d, ws, stream);
+    if (ws.plan) return KORE_OK;
+    return launch_generic<T>(d, stream);
+  };
+  // Rows or columns that run backwards: the engines address a tile through unsigned offsets
+  // from its first element.
+  if (std::min({d.sam, d.sak, d.sbk, d.sbn}) < 0) return pack_or_generic();
   // Fast-path preconditions: A K-contiguous with 16-byte aligned rows, K % 8 == 0,
   // B K- or N-contiguous with 16-byte aligned rows, C N-contiguous.
   const bool a_ok = d.sak == 1 && d.sam % 8 == 0 && aligned16(d.a) && d.sa % 8 == 0 && d.K % 8 == 0;
@@ -1868,11 +1877,7 @@ int dispatch_typed(const GemmDesc& d, Ws& ws, hipStream_t stream) {
     if (ws.plan) return KORE_OK;
     return launch_ragged_ring<T>(d, stream);
   }
-  // Large problems in other layouts: pack, then the engines (small ones are cheaper on
-  // the generic kernel than a pack pass).
-  if (d.M * d.N * d.K >= (1ll << 27) && d.K >= 64 && padded_fits(d)) return launch_padded<T>(d, ws, stream);
-  if (ws.plan) return KORE_OK;
-  return launch_generic<T>(d, stream);
+  return pack_or_generic();
 }
 
 int run_gemm(const GemmDesc& d, Ws& ws, void* stream) {

@@ -942,3 +942,27 @@ def test_gemm_splitk_tall(gpu, dtype, act, M, N, K, layout):
     name = "bf16" if dtype == torch.bfloat16 else "fp16"
     pair_only(out.cpu(), gemm_fusion_ref(a, b, bias, act), name, f"tall split-K {M}x{N}x{K} {layout} {act}")
     assert bit_equal(out, kore_amd.gemm_fused(ag, bd, bias.to(gpu), act))
+
+
+@pytest.mark.parametrize("M,N,K", [(64, 128, 128), (130, 96, 77), (1, 256, 256), (600, 640, 512), (513, 515, 1001)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_gemm_negative_strides(gpu, dtype, M, N, K):
+    """Operands read backwards along either index through the C ABI, packed or on the generic
+    kernel, against the oracle on flipped copies."""
+    from kore_amd import _lib
+    lib = _lib.load()
+    g = torch.Generator().manual_seed(M + N + K)
+    a, b = (torch.randn((M, K), generator=g) / K ** 0.5).to(dtype), torch.randn((K, N), generator=g).to(dtype)
+    ag, bg = a.to(gpu), b.to(gpu)
+    code, size = (0, 2) if dtype == torch.bfloat16 else (2, 4)
+    for fm, fk, fb, fn in ((1, 0, 0, 0), (0, 1, 0, 0), (0, 0, 1, 0), (0, 0, 0, 1), (1, 1, 1, 1)):
+        out = torch.empty((M, N), dtype=dtype, device=gpu)
+        args = (code, 0, ag.data_ptr() + size * (fm * (M - 1) * K + fk * (K - 1)), -K if fm else K, -1 if fk else 1,
+                bg.data_ptr() + size * (fb * (K - 1) * N + fn * (N - 1)), -N if fb else N, -1 if fn else 1, None,
+                out.data_ptr(), N, M, N, K)
+        need = lib.kore_gemm_workspace_bytes(*args)
+        ws = torch.empty((max(need, 1),), dtype=torch.uint8, device=gpu)
+        _lib.check(lib.kore_gemm(*args, ws.data_ptr(), need, torch.cuda.current_stream().cuda_stream))
+        dims_a, dims_b = [d for d, f in ((0, fm), (1, fk)) if f], [d for d, f in ((0, fb), (1, fn)) if f]
+        ref = gemm_fusion_ref(a.flip(dims_a) if dims_a else a, b.flip(dims_b) if dims_b else b, None, "none")
+        verdict(out.cpu(), ref, "gemm_fusion", str(dtype), f"{M}x{N}x{K} flips {fm}{fk}{fb}{fn}")

@@ -248,6 +248,24 @@ def test_gemm_skinny_route_without_gpu(lib, M, N, K, b_along_n, split):
     assert need >= 2 * M * N * 4 if split else need == 0
 
 
+def test_gemm_negative_strides_without_gpu(lib):
+    """Rows or columns that run backwards (which the C ABI takes, torch has none) are packed in
+    large problems and run the generic kernel in small ones: the engines, whose buffer offsets
+    are unsigned, would read outside the operands.  Forward, the same shapes stay in place."""
+    fake = ctypes.c_void_p(1 << 40)
+
+    def need(M, N, K, a, b, fn=lib.kore_gemm_workspace_bytes):
+        return fn(0, 0, fake, *a, fake, *b, None, fake, N, M, N, K)
+
+    for M, N, K in ((4096, 4096, 4096), (512, 4096, 4096), (3072, 4096, 4095), (64, 4096, 4096), (2048, 4096, 128)):
+        a_bytes = M * -(-K // 64) * 64 * 2
+        assert need(M, N, K, (K, 1), (1, K)) == 0
+        for a, b in (((-K, 1), (1, K)), ((-K, 1), (N, 1)), ((K, 1), (1, -K)), ((K, 1), (-N, 1)), ((K, -1), (1, K)),
+                     ((1, -M), (N, 1)), ((K, 1), (1, -K))):
+            assert need(M, N, K, a, b) >= a_bytes, (M, N, K, a, b)
+    assert need(64, 128, 128, (-128, 1), (1, 128)) == 0
+
+
 # --------------------------------------------------------------------------- #
 # drop-in candidates: signatures and the reference's static scanner rules
 # (kore/reward/reward.py:70-179, restated)
