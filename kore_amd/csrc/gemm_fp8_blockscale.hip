@@ -282,7 +282,7 @@ __device__ __forceinline__ i32x8_t lds_frag32(const uint8_t* row, const int (&of
 // at most kFp8GroupM row tiles (launched side by side, sharing it through L2), or, in
 // the grouped mode, by one expert's row blocks.  The policy is an instruction immediate,
 // hence a template flag (a branch would split the tile loop).
-// RAG (row-scale modes): ragged N, K and row alignment, see zero_lead above; the K tail is
+// RAG (row-scale modes): ragged N, K and row alignment, see above; the K tail is
 // multiplied before the pipelined loop, from registers, while the loop's first stages land.
 template <typename C, bool FULL_M, bool GROUPED = false, bool BNT = false, bool RAG = false>
 __global__ void __launch_bounds__(C::NW * 64)
@@ -1246,7 +1246,7 @@ struct SkinnyCfg {
 // M=16..64 within 3% -- the kernel's time is its L2-to-LDS operand stream, not LDS reads.
 __device__ __forceinline__ int sk_key(int r) { return (r ^ (r >> 3)) & 7; }
 
-// RAG: ragged N, K and row alignment (row-scale modes, see zero_lead).
+// RAG: ragged N, K and row alignment (row-scale modes), as in gemm_fp8_pipe_kernel.
 template <typename C, bool RAG = false>
 __global__ void __launch_bounds__(C::NW_ * 64)
     gemm_fp8_skinny_kernel(const Fp8Params p) {
@@ -1538,15 +1538,22 @@ extern "C" int kore_gemm_a8w8_blockscale(const void* xq, int64_t ldx, const void
     // where they fit one round, 4096 x 4096 16.9 -> 12.2, 3072 x 3840 15.0 -> 9.1, and
     // below, M = 64 4096 x 4096 10.1 -> 8.6, M = 32 7.8 -> 6.7 us.
     // Fewer than 16 K blocks or, up to M = 64, few workgroups (N < 2048) do not repay the copy
-    // (M = 65 4480 x 1152 6.4 against 6.8 us, M = 64 512 x 8192 10.6 against 13.1).
-    const bool pre = K / 128 >= 16 && K / 128 <= 64 && (M > 64 || N >= 2048);
+    // (M = 65 4480 x 1152 6.4 against 6.8 us, M = 64 512 x 8192 10.6 against 13.1).  Nor do
+    // fewer rows, or a second round of 32-column workgroups, with more K blocks, once weights
+    // and scales come from memory (repeated / after a 512 MiB flush, with the copy over
+    // without: 20 and 32 rows 1.00 / 1.03 at 16 to 22 blocks, 0.95 / 0.97 at 24 to 32; 48 and 64
+    // rows 0.96 / 1.06 at 16 and 18, 0.95 / 1.00 at 20 and 22; 128 x 14336 1.00 / 1.07 up to
+    // 22, 0.96 / 0.99 at 24 and 28).
+    const bool one_round = N <= 32ll * device_cus();
+    const int64_t nk_min = M <= 32 ? 24 : M <= 64 ? 20 : M > 96 && !one_round ? 24 : 16;
+    const bool pre = K / 128 >= nk_min && K / 128 <= 64 && (M > 64 || N >= 2048);
     const bool narrow = pre && N <= 16ll * device_cus();
     if (M <= 32)
       return narrow ? launch_fp8_skinny<SkinnyCfg<32, 8, 3, Q_BLOCK_FP8, 1, true>>(p, st)
-                           : launch_fp8_skinny<SkinnyCfg<32, 8, 2>>(p, st);
+                    : launch_fp8_skinny<SkinnyCfg<32, 8, 2>>(p, st);
     if (M <= 64)
       return narrow ? launch_fp8_skinny<SkinnyCfg<64, 7, 2, Q_BLOCK_FP8, 1, true>>(p, st)
-                           : launch_fp8_skinny<SkinnyCfg<64, 4, 3>>(p, st);
+                    : launch_fp8_skinny<SkinnyCfg<64, 4, 3>>(p, st);
     if (pre)
       return narrow ? launch_fp8_skinny<SkinnyCfg<128, 7, 1, Q_BLOCK_FP8, 1, true>>(p, st)
                     : launch_fp8_skinny<SkinnyCfg<128, 6, 1, Q_BLOCK_FP8, 2, true>>(p, st);

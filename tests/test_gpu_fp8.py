@@ -204,12 +204,14 @@ def test_fp8_skinny_layouts(gpu, M):
 
 @pytest.mark.parametrize("M", [17, 32, 33, 64, 65, 100, 128])
 @pytest.mark.parametrize("N,K", [(128, 128), (384, 896), (4096, 1024), (4224, 640), (256, 8192), (4224, 8192),
-                                 (128, 8320)])
+                                 (128, 8320), (2048, 2432), (2048, 2560), (2176, 2944), (4096, 3072), (2048, 8192),
+                                 (8320, 2944), (8320, 3072)])
 def test_fp8_skinny_scales_in_lds(gpu, M, N, K):
-    """17 <= M <= 128 with the scales copied to LDS first (up to 64 K blocks; 65 keep them in
-    the operand stream), in 16- and 32-column workgroups (N to 4096 and beyond), fewer K
-    blocks than waves, and K orders that start at the workgroup's own block.  Column-major
-    scales give the same bits; reruns too."""
+    """17 <= M <= 128 with the scales copied to LDS first and without: 16- and 32-column
+    workgroups (N to 4096 and beyond), one and two rounds of them, both sides of the counts
+    of K blocks from which the copy pays (16; 20 for M <= 64; 24 for M <= 32, and in two
+    rounds for M > 96) and of 64, where it ends, fewer K blocks than waves, and K orders that
+    start at the workgroup's own block.  Column-major scales give the same bits; reruns too."""
     xq, wq, xs, ws = W.fp8_inputs(M, N, K, seed=M + N + K, scale=0.2)
     out = _run(gpu, xq, wq, xs, ws)
     ref = matmul_blockscale_ref(xq, wq, xs, ws)
