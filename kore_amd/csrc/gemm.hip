@@ -1714,11 +1714,20 @@ inline double skinny_alternative_us(const GemmDesc& d, bool nc, bool rows_ok) {
     if (deep) return std::max(tiles_us(d, pick_tile(d)), 4.9 + mb / 4.1);
     if (mid < 128 && d.K >= 1024 && t32 * 2 <= cus) {
       const SplitPlan s = splitk_plan(d);
-      const bool tall = s.rows > 32;
-      return (tall ? 4.0 : 6.0) + std::max(s.kper * 8.5e-3, mb / (tall ? 5.3 : 6.1)) +
-             (double)(d.M * d.N * s.splits * 8) / (tall ? 1.6e6 : 2.8e6);
+      const double partials = (double)(d.M * d.N * s.splits * 8);
+      if (s.rows > 32) return 4.0 + std::max(s.kper * 8.5e-3, mb / 5.3) + partials / 1.6e6;
+      if (nc) return 6.0 + std::max(s.kper * 8.5e-3, mb / 6.1) + partials / 2.8e6;
+      // rows that lie a multiple of 8 KB apart crowd a few memory channels; an N off the
+      // multiples of 4 is summed without 16-byte loads, slice after slice (W.t(), repeated /
+      // flushed, split-K against this kernel: 1 x 8192 x 8192 44 / 45 against 25 / 29 us,
+      // 64 x 631 x 3008 21 / 25 against 6.9 / 13.2)
+      const double rate = d.sbn * 2 % 8192 == 0 ? 4.4 : 5.9;
+      return 5.6 + std::max(s.kper * 8.7e-3, mb / rate) + partials / 2.8e6 + s.splits * (d.N % 4 == 0 ? 0.09 : 0.8);
     }
-    if (mid < 128 && d.K >= 512) return 3.5 + std::max((double)((t32 + cus - 1) / cus * d.K) * 6.5e-3, mb / 3.5);
+    if (mid < 128 && d.K >= 512) {
+      const double n = (double)((t32 + cus - 1) / cus), k = (double)d.K;
+      return nc ? 3.5 + std::max(n * k * 6.5e-3, mb / 3.5) : 1.5 + std::max(n * (2.9 + k * 6.1e-3), mb / 3.1);
+    }
   }
   if (rows_ok && !deep) return mid < 128 ? 3.5 + (double)d.K * (nc ? 12.7e-3 : 8.5e-3) + mb / 8.0 : 5.4 + mb / 3.2;
   // (the weights' stream, which few and misaligned tiles read slowly, beside the tiles' time)
@@ -1751,13 +1760,13 @@ int dispatch_typed(const GemmDesc& d, Ws& ws, hipStream_t stream) {
   const bool a16 = d.sam % 8 == 0 && aligned16(d.a), skinny_a = d.batch == 1 && d.sak == 1 && d.M <= 128 &&
              d.K >= 64 && fits32 && (d.sam >= d.K || d.M == 1) && d.M * d.sam * 2 + d.K * 2 < (1ll << 31);
   if (skinny_a && d.sbk == 1 && (d.sbn >= d.K || d.N == 1) && 64 * d.sbn * 2 + d.K * 2 < (1ll << 31)) {
-    // K-contiguous weights.  K < 512: 64x64 tiles, which have no cross-wave sum to pay for
-    // (20 x 11000 x 256 4.8 us against 6.0).  More than 32 rows and 128 tiles of 128 columns:
-    // the mid-size tiles (repeated / flushed, 64 x 32000 x 4000 44.7 / 108 us against 65.5 /
-    // 70.2, 128 x 50257 x 1000 35 / 66 against 61 / 66, 128 x 32000 x 4096 51 / 128 against
-    // 74 / 79).
-    const bool rows_ok = a_ok && b_kc, wide = d.M > 32 && d.N > 127 * 128 && d.K >= 256;
-    if (!wide && (!rows_ok || d.K % 64 != 0 || d.K >= 512)) {
+    // K-contiguous weights.  More than 32 rows and 128 tiles of 128 columns: the mid-size tiles
+    // (repeated / flushed, 64 x 32000 x 4000 44.7 / 108 us against 65.5 / 70.2, 128 x 50257 x
+    // 1000 35 / 66 against 61 / 66, 128 x 32000 x 4096 51 / 128 against 74 / 79); aligned, with
+    // K < 512, any rows: 128x128 tiles.  Fewer tiles and a short K are the skinny kernel's
+    // (64x64 tiles against it, 18 x 2790 x 384 6.0 / 10.7 against 3.8 / 6.2 us).
+    const bool rows_ok = a_ok && b_kc, ragged = !rows_ok || d.K % 64 != 0;
+    if (d.N <= 127 * 128 || (d.M <= 32 ? ragged || d.K >= 512 : ragged && d.K < 256)) {
       const SkinnyPick k = pick_skinny(d, false, a16 && b_kc);
       if (k.us < skinny_alternative_us(d, false, rows_ok)) {
         if (ws.plan) return KORE_OK;

@@ -737,10 +737,12 @@ def test_workspace_paths_under_graph_capture(gpu):
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("M,N,K", [(1, 1, 64), (16, 17, 65), (17, 300, 900), (33, 823, 1984), (64, 4096, 512),
                                    (64, 513, 127), (65, 1000, 1001), (128, 4097, 129), (100, 7168, 2048),
-                                   (5, 14339, 640), (128, 16, 4095)])
+                                   (5, 14339, 640), (128, 16, 4095), (13, 4099, 129), (29, 4099, 200),
+                                   (47, 4099, 129), (32, 8197, 129), (60, 8197, 200), (101, 8197, 129),
+                                   (64, 100, 64), (2, 430, 2048)])
 def test_gemm_skinny(gpu, dtype, M, N, K):
     """M <= 128 against K-contiguous weights (the skinny kernel): row, column and K tails,
-    16-, 32- and 64-column workgroups, bias and activation, rows at odd element offsets (the
+    16-, 32- and 64-column workgroups of each height (16, 32, 64 and 128 rows), bias and activation, rows at odd element offsets (the
     same bits as aligned rows when both take this kernel), and an infinity in a column that
     the tail block repeats, which must reach exactly its own row and column."""
     g = torch.Generator().manual_seed(M + N + K)
@@ -780,11 +782,12 @@ def test_gemm_skinny(gpu, dtype, M, N, K):
 @pytest.mark.parametrize("M,N,K", [(1, 1, 64), (1, 7, 65), (16, 9, 127), (17, 823, 1984), (33, 320, 1816),
                                    (64, 512, 512), (64, 4095, 129), (65, 1001, 1000), (128, 9473, 565),
                                    (128, 4096, 256), (100, 7168, 2048), (5, 14337, 640), (128, 16, 4095),
-                                   (40, 1030, 192)])
+                                   (40, 1030, 192), (13, 4099, 129), (29, 4099, 200), (47, 4097, 129),
+                                   (32, 8197, 129), (60, 8197, 200), (101, 8197, 129)])
 def test_gemm_skinny_nc(gpu, dtype, M, N, K):
     """M <= 128 against N-contiguous weights on the skinny kernel: any N (the last element of
     B, which the buffer range check cuts off when an odd count of columns ends mid-dword),
-    K tails, 16- to 64-column workgroups, and a B that is a view with odd row stride and
+    K tails, 16- to 64-column workgroups of each height, and a B that is a view with odd row stride and
     offset, whose neighbours are NaN."""
     g = torch.Generator().manual_seed(M + N + K)
     a = (torch.randn((M, K), generator=g) / K ** 0.5).to(dtype)

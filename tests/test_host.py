@@ -237,6 +237,7 @@ def test_gemm_long_k_packs_without_gpu(lib, M, N, K, a_along_m, b_along_n, packe
 @pytest.mark.parametrize("M,N,K,b_along_n,split", [
     (16, 2048, 12160, False, True), (32, 5120, 12160, False, True), (128, 2048, 8192, False, True),
     (48, 5376, 5504, True, True), (16, 4096, 8192, True, True), (128, 4096, 4096, True, True),
+    (1, 8192, 8192, False, False), (2, 430, 11264, False, False), (64, 631, 3008, False, False),
     (1, 4096, 4096, False, False), (64, 4096, 4096, False, False), (16, 14336, 4096, False, False),
     (16, 4096, 1024, True, False), (64, 4096, 2048, True, False)])
 def test_gemm_skinny_route_without_gpu(lib, M, N, K, b_along_n, split):
