@@ -1159,6 +1159,7 @@ struct GemmDesc {
   int64_t sam, sak, sbk, sbn, scm;  // element strides; B given as (k, n)
   int64_t sa, sb, sc;               // batch strides
   int64_t kvalid = 0;               // > 0: K-rows of an N-contiguous B that exist (K is padded)
+  int64_t cus = device_cus();       // (a runtime call: once per problem)
 };
 
 inline bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
@@ -1308,12 +1309,12 @@ int launch_shortk(const GemmDesc& d, hipStream_t stream) {
   p.bias_vec = 0;
   const int64_t tiles = (int64_t)p.tiles_per_batch * d.batch;
   // segment length: about the tiles per CU, at most one column
-  const int64_t per_cu = tiles / device_cus();
+  const int64_t per_cu = tiles / d.cus;
   const int seg = (int)std::max<int64_t>(1, std::min<int64_t>(p.tiles_m, per_cu));
   const int64_t nseg = (p.tiles_m + seg - 1) / seg;
   const int64_t total = nseg * p.tiles_n * d.batch;
   if (total > 0x7fffffff || total * seg > 0x7fffffff) return set_error(KORE_EUNSUPPORTED, "gemm: grid too large");
-  const int grid = (int)std::min<int64_t>(total, device_cus());
+  const int grid = (int)std::min<int64_t>(total, d.cus);
   const dim3 gr((unsigned)grid), blk(512);
   if (BL == B_KC && d.K == 64) hipLaunchKernelGGL((gemm_shortk_kernel<T, 1, B_KC>), gr, blk, 0, stream, p, seg);
   if (BL == B_KC && d.K == 128) hipLaunchKernelGGL((gemm_shortk_kernel<T, 2, B_KC>), gr, blk, 0, stream, p, seg);
@@ -1467,7 +1468,7 @@ int launch_skinny_nb(const GemmDesc& d, int nb, hipStream_t st) {
 enum TileShape { TILE_256x256, TILE_256x128, TILE_128x128, TILE_64x128, TILE_32x128 };
 
 inline TileShape pick_tile(const GemmDesc& d) {
-  const int64_t cus = device_cus();
+  const int64_t cus = d.cus;
   struct Opt {
     TileShape t;
     int bm, bn;
@@ -1547,7 +1548,7 @@ constexpr struct {
   double us, ns;  // of a round: fixed part, one column of K
 } kTileCost[] = {{256, 256, 12.6, 17.5}, {256, 128, 6.3, 17.0}, {128, 128, 3.4, 9.1}, {64, 128, 2.7, 5.5}, {32, 128, 1.7, 4.0}};
 inline double tile_rounds(const GemmDesc& d, TileShape t) {
-  const int64_t bm = kTileCost[t].bm, bn = kTileCost[t].bn, cus = device_cus();
+  const int64_t bm = kTileCost[t].bm, bn = kTileCost[t].bn, cus = d.cus;
   return (double)(((d.M + bm - 1) / bm * ((d.N + bn - 1) / bn) * d.batch + cus - 1) / cus);
 }
 inline double tiles_us(const GemmDesc& d, TileShape t) {
@@ -1651,7 +1652,7 @@ struct SplitPlan {
   int rows, splits, kper;
 };
 inline SplitPlan splitk_plan(const GemmDesc& d) {
-  const int64_t cus = device_cus(), nk = d.K / 64, tn = (d.N + 127) / 128, t32 = (d.M + 31) / 32 * tn;
+  const int64_t cus = d.cus, nk = d.K / 64, tn = (d.N + 127) / 128, t32 = (d.M + 31) / 32 * tn;
   const bool tall = d.M > 32 && d.M <= 128 && t32 * 4 >= cus && d.N * d.K * 2 > (24ll << 20);
   const int64_t want = tall ? std::max<int64_t>(1, std::min<int64_t>(cus / 2 / tn, nk / 4))
                             : std::min<int64_t>(cus / t32, nk / 4);
@@ -1680,7 +1681,7 @@ struct SkinnyPick {
 // rows16: 16-byte rows, of both operands or, for N-contiguous weights, of A
 inline SkinnyPick pick_skinny(const GemmDesc& d, bool nc, bool rows16) {
   static const double nc_stream[] = {2.0e6, 2.8e6, 4.6e6}, nc_own[] = {23e3, 42e3, 50e3}, off_lines[] = {1.4, 1.4, 1.8};
-  const int64_t cus = device_cus();
+  const int64_t cus = d.cus;
   const bool lines = d.sbk % 64 == 0 && ((uintptr_t)d.b & 127u) == 0;
   SkinnyPick best{1, 1e300};
   for (int i = 0; i < 3; ++i) {
@@ -1706,7 +1707,7 @@ inline SkinnyPick pick_skinny(const GemmDesc& d, bool nc, bool rows16) {
 // Estimated time of the route that an M <= 128 problem takes otherwise (the order is that of
 // dispatch_typed below); `rows_ok`: 16-byte rows and K % 8 == 0.
 inline double skinny_alternative_us(const GemmDesc& d, bool nc, bool rows_ok) {
-  const int64_t cus = device_cus(), mid = (d.M + 127) / 128 * ((d.N + 127) / 128);
+  const int64_t cus = d.cus, mid = (d.M + 127) / 128 * ((d.N + 127) / 128);
   const int64_t t32 = (d.M + 31) / 32 * ((d.N + 127) / 128);
   const double mb = (double)(d.N * d.K * 2) * 1e-6;
   const bool deep = mid >= 128 && d.K >= 256;
@@ -1852,14 +1853,14 @@ int dispatch_typed(const GemmDesc& d, Ws& ws, hipStream_t stream) {
     const bool shortk = (d.K == 64 || d.K == 128) && d.act == KORE_ACT_NONE && d.bias == nullptr &&
                         d.N % 8 == 0 && d.scm % 8 == 0 && d.sc % 8 == 0 && aligned16(d.c) &&
                         d.sam * 2 * 128 + d.K * 2 < (1ll << 31) && (b_nc || d.sbn * 2 * 128 + d.K * 2 < (1ll << 31)) &&
-                        d.scm * 2 * 128 < (1ll << 31) && mid_tiles >= 4 * (int64_t)device_cus();
+                        d.scm * 2 * 128 < (1ll << 31) && mid_tiles >= 4 * d.cus;
     if (shortk) {
       if (ws.plan) return KORE_OK;
       return b_kc ? launch_shortk<T, B_KC>(d, stream) : launch_shortk<T, B_NC>(d, stream);
     }
     // Few 32x128 tiles for the CUs and a long K (decode-sized M): split K.
     const int64_t t32 = ((d.M + 31) / 32) * ((d.N + 127) / 128);
-    if (d.batch == 1 && (b_kc ? buf_ok : buf_nc_ok) && d.K >= 1024 && t32 * 2 <= device_cus()) {
+    if (d.batch == 1 && (b_kc ? buf_ok : buf_nc_ok) && d.K >= 1024 && t32 * 2 <= d.cus) {
       const SplitPlan sp = splitk_plan(d);
       if (sp.rows == 64)
         return b_kc ? launch_splitk<T, B_KC, 64, 128, 2, 2, 6>(d, sp.splits, sp.kper, ws, stream)

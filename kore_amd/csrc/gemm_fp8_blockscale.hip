@@ -1544,10 +1544,11 @@ extern "C" int kore_gemm_a8w8_blockscale(const void* xq, int64_t ldx, const void
     // without: 20 and 32 rows 1.00 / 1.03 at 16 to 22 blocks, 0.95 / 0.97 at 24 to 32; 48 and 64
     // rows 0.96 / 1.06 at 16 and 18, 0.95 / 1.00 at 20 and 22; 128 x 14336 1.00 / 1.07 up to
     // 22, 0.96 / 0.99 at 24 and 28).
-    const bool one_round = N <= 32ll * device_cus();
+    const int64_t cus = device_cus();
+    const bool one_round = N <= 32 * cus;
     const int64_t nk_min = M <= 32 ? 24 : M <= 64 ? 20 : M > 96 && !one_round ? 24 : 16;
     const bool pre = K / 128 >= nk_min && K / 128 <= 64 && (M > 64 || N >= 2048);
-    const bool narrow = pre && N <= 16ll * device_cus();
+    const bool narrow = pre && N <= 16 * cus;
     if (M <= 32)
       return narrow ? launch_fp8_skinny<SkinnyCfg<32, 8, 3, Q_BLOCK_FP8, 1, true>>(p, st)
                     : launch_fp8_skinny<SkinnyCfg<32, 8, 2>>(p, st);
