@@ -148,10 +148,11 @@ def test_a8w8_buffer_tile(gpu, kind, M, N, K):
 @pytest.mark.parametrize("kind", ["fp8", "int8"])
 @pytest.mark.parametrize("M,N,K", [(1, 1, 128), (16, 127, 129), (17, 513, 255), (64, 4096, 4095), (128, 129, 1000),
                                    (129, 300, 131), (600, 1000, 515), (1500, 2050, 641), (3000, 4095, 2049),
-                                   (2000, 8191, 129), (4, 8200, 384)])
+                                   (2000, 8191, 129), (1500, 4001, 300), (4, 8200, 384), (29, 8200, 385),
+                                   (60, 8321, 1000), (100, 8321, 300)])
 def test_a8w8_ragged(gpu, kind, M, N, K):
     """Any N, any K >= 128 and rows at any byte alignment on the MFMA kernels: skinny (M <= 128,
-    16- and 32-column workgroups), 128x128, 256x128 and 256x256 pipe tiles and the 4-wave buffer
+    16- and 32-column workgroups of each height), 128x128, 256x128 and 256x256 pipe tiles and the 4-wave buffer
     tile.  int8 sums are exact, so the result equals the zero-padded aligned problem's bit for
     bit; fp8 meets the oracle on a row sample.  A base one byte off the allocation and a row
     stride larger than K give the same bits.  A NaN code in the columns that the tail block
@@ -165,7 +166,7 @@ def test_a8w8_ragged(gpu, kind, M, N, K):
         buf = torch.empty(t.shape[0] * ld + 1, dtype=torch.uint8, device=gpu)
         v = buf[1:].view(t.shape[0], ld)[:, :t.shape[1]]
         v.copy_(t.view(torch.uint8))
-        return v.view(t.dtype) if t.dtype != torch.float8_e4m3fn else v.view(torch.float8_e4m3fn)
+        return v.view(t.dtype)
 
     assert bit_equal(kore_amd.gemm_a8w8(off(xg, K + 3), off(wg, K + 5), xsg, wsg), y)
     if kind == "int8":

@@ -59,7 +59,8 @@ def test_grouped_gemm_ragged(gpu, M, E, N, K):
 
 @pytest.mark.parametrize("M,E,N,K", [(384, 8, 256, 256), (385, 8, 256, 256), (448, 8, 256, 320), (449, 8, 256, 320),
                                      (512, 8, 512, 256), (513, 8, 512, 256), (1000, 8, 2048, 128),
-                                     (3000, 16, 1792, 192), (2048, 32, 2048, 256), (2049, 32, 2048, 256)])
+                                     (3000, 16, 1024, 192), (3000, 16, 1280, 192), (3000, 16, 1792, 192),
+                                     (2048, 32, 1792, 256), (2048, 32, 2048, 256), (2049, 32, 2048, 256)])
 def test_grouped_block_choice(gpu, M, E, N, K):
     """Both sides of the block-row rules of the bf16 (48, 56 and 64 rows per expert; 80, 130 and
     192 tiles of 256x256) and fp8 (64 rows, 100 tiles) grouped GEMMs, jagged routing with some

@@ -102,11 +102,12 @@ def test_fused_moe_128row_blocks(gpu, T, E, topk, D, I):
 
 @pytest.mark.parametrize("T,E,topk,D,I", [(416, 8, 1, 256, 256), (417, 8, 1, 256, 256), (1664, 8, 1, 256, 256),
                                           (1665, 8, 1, 256, 384), (448, 32, 8, 256, 512), (449, 32, 8, 256, 512),
-                                          (16, 64, 4, 384, 640), (100, 64, 8, 256, 512)])
+                                          (128, 64, 8, 256, 512), (129, 64, 8, 256, 512),
+                                          (16, 64, 4, 384, 640), (100, 64, 8, 256, 512), (40, 64, 4, 768, 256)])
 def test_fused_moe_block_choice(gpu, T, E, topk, D, I):
     """Both sides of the block-size and stage-count rules: 32 / 128 / 256 rows where one block
     per expert leaves the CUs half empty (E * I / 128 < 128: 52 and 208 slots per expert) and
-    where it does not (16 and 112), decode rings with one and two workgroups per CU, and
+    where it does not (16 and 112), decode rings of both products with one and two workgroups per CU, and
     256-row blocks whose padding rows lie outside the buffer resources.  Invalid ids add
     padding that no expert owns."""
     hidden, w1, w2, tw, ti = W.moe_inputs(T, E, topk, D, I, seed=T + 3, wscale=0.05)
