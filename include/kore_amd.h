@@ -100,8 +100,9 @@ int kore_gemm(int dtype, int act,
  * Same arguments and results as kore_gemm without the workspace: the packed-operand
  * and split-K scratch is a static device array of kore_gemm_noalloc_scratch_bytes()
  * (64 MiB) per GPU, held from the library's first use on that GPU until the process
- * exits.  Calls needing more fail with KORE_EWORKSPACE (use kore_gemm then); nothing
- * is allocated or freed.  All calls on one GPU share that array, which keeps the last
+ * exits.  Operands that would not fit packed are read in place where the ring tiles can
+ * (then the last bits may differ from kore_gemm's); other calls needing more fail with
+ * KORE_EWORKSPACE (use kore_gemm then); nothing is allocated or freed.  All calls on one GPU share that array, which keeps the last
  * call's contents: calls that overlap on one GPU (other streams, other host threads)
  * race -- serialise them.
  */

@@ -1535,6 +1535,15 @@ inline bool padded_fits(const GemmDesc& d) {
   const int64_t Kp = (d.K + 63) / 64 * 64;
   return d.M < (1ll << 31) && d.N < (1ll << 31) && Kp * 2 * 256 + Kp * 2 < (1ll << 31) && d.batch <= 65535;
 }
+struct PackedBytes {
+  size_t a, b;
+  size_t total() const { return a + b; }
+};
+inline PackedBytes packed_bytes(const GemmDesc& d) {
+  const int64_t Kp = (d.K + 63) / 64 * 64;
+  return {(size_t)(d.batch * d.M * Kp * 2 + 255) / 256 * 256,
+          padded_b_inplace(d) ? (size_t)0 : (size_t)(d.batch * d.N * Kp * 2)};
+}
 // ---------------------------------------------------------------------------------
 // Estimated times in us, by which the dispatch picks among the kernels that can take a
 // 16-bit problem: a fixed part, the rounds of tiles that a CU runs one after the other (each
@@ -1580,8 +1589,9 @@ inline double ragged_ring_us(const GemmDesc& d) {
 // misaligned rows once and not once per tile (A along M, repeated / flushed: 448 x 449 x 4689
 // 58 / 76 us on the ring, 35 / 40 packed; both along K, 320 x 192 x 9423 67 / 98 against
 // 54 / 54).  Packed operands run the faster 256x256 tiles, so they stay from 2^34 products on
-// (4097^3).
-inline bool ragged_ring_ok(const GemmDesc& d) {
+// (4097^3).  Scratch beyond `limit` bytes keeps a problem on the ring: kore_gemm_noalloc, which
+// cannot grow its scratch, takes in place what would not fit (4868 x 49 x 21042: 207 MB packed).
+inline bool ragged_ring_ok(const GemmDesc& d, size_t limit) {
   const bool akc = d.sak == 1, bkc = d.sbk == 1;
   if (d.K < 64 || !(akc || d.sam == 1) || !(bkc || d.sbn == 1) || d.M * d.N * d.K * d.batch >= (1ll << 34)) return false;
   // K-rows that all start at one element (an operand expanded over K) would all be cut off at
@@ -1592,7 +1602,8 @@ inline bool ragged_ring_ok(const GemmDesc& d) {
       (bkc ? d.sbn * 2 * 256 + d.K * 2 : d.sbk * 2 * (d.K + 64) + 512) >= lim)
     return false;
   // (by a twentieth: what the two estimates differ by where they are off)
-  return d.M * d.N * d.K < (1ll << 27) || !padded_fits(d) || 1.05 * ragged_ring_us(d) < packed_us(d);
+  return d.M * d.N * d.K < (1ll << 27) || !padded_fits(d) || 1.05 * ragged_ring_us(d) < packed_us(d) ||
+         packed_bytes(d).total() > limit;
 }
 template <typename T>
 int launch_ragged_ring(const GemmDesc& d, hipStream_t stream) {
@@ -1607,15 +1618,14 @@ template <typename T>
 int launch_padded(const GemmDesc& d, Ws& ws, hipStream_t stream) {
   const int64_t Kp = (d.K + 63) / 64 * 64;
   const bool b_nc = padded_b_inplace(d);
-  const size_t a_bytes = (size_t)(d.batch * d.M * Kp * 2 + 255) / 256 * 256;
-  const size_t b_bytes = b_nc ? 0 : (size_t)(d.batch * d.N * Kp * 2);
-  void* buf = ws.take(a_bytes + b_bytes);
+  const PackedBytes need = packed_bytes(d);
+  void* buf = ws.take(need.total());
   if (ws.plan) return KORE_OK;
   if (buf == nullptr)
     return set_error(KORE_EWORKSPACE, "gemm: packing the operands needs %zu workspace bytes (got %zu)",
-                     ws_bytes(a_bytes + b_bytes), ws.bytes);
+                     ws_bytes(need.total()), ws.bytes);
   uint16_t* ap = (uint16_t*)buf;
-  uint16_t* bp = (uint16_t*)((char*)buf + a_bytes);
+  uint16_t* bp = (uint16_t*)((char*)buf + need.a);
   int rc = launch_pack16((const uint16_t*)d.a, d.sam, d.sak, d.sa, ap, d.M * Kp, d.M, d.K, Kp, d.batch, stream);
   GemmDesc q = d;
   q.a = ap;
@@ -1883,7 +1893,7 @@ int dispatch_typed(const GemmDesc& d, Ws& ws, hipStream_t stream) {
     return small ? launch_tile<T, B_NC, 64, 64>(d, stream) : launch_tile<T, B_NC, 128, 128>(d, stream);
   }
   // Any other problem whose operands have a unit stride: read in place on the ring tiles.
-  if (ragged_ring_ok(d) && fits32) {
+  if (ragged_ring_ok(d, ws.limit) && fits32) {
     if (ws.plan) return KORE_OK;
     return launch_ragged_ring<T>(d, stream);
   }
@@ -2088,6 +2098,7 @@ extern "C" int kore_gemm_noalloc(int dtype, int act, const void* a, int64_t lda_
   if (rc != KORE_OK) return rc;
   Ws plan;
   plan.plan = true;
+  plan.limit = kNoAllocScratchBytes;
   rc = run_gemm(d, plan, nullptr);
   if (rc != KORE_OK) return rc;
   if (plan.need > kNoAllocScratchBytes)
@@ -2098,5 +2109,6 @@ extern "C" int kore_gemm_noalloc(int dtype, int act, const void* a, int64_t lda_
   Ws ws;
   ws.ptr = base;
   ws.bytes = kNoAllocScratchBytes;
+  ws.limit = kNoAllocScratchBytes;
   return run_gemm(d, ws, stream);
 }

@@ -222,6 +222,7 @@ struct Ws {
   size_t bytes = 0;
   bool plan = false;
   size_t need = 0;
+  size_t limit = SIZE_MAX;  // where a path without scratch exists, one that needs more is not picked
   // Scratch of `n` bytes (256-byte aligned start) for the chosen path: nullptr in
   // plan mode (after recording the need) or when the workspace is too small.
   void* take(size_t n) {

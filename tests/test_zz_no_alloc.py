@@ -1,7 +1,7 @@
 """GPU: kore_gemm_noalloc, the GEMM entry point that allocates nothing, against kore_gemm.
 
-Both entry points run the same kernels; the no-allocation one takes the scratch of its
-packed-operand and split-K paths from a static device array instead of a workspace.
+Both entry points run the same kernels (but where packing would not fit); the no-allocation
+one takes the scratch of its packed-operand and split-K paths from a static device array.
 Each case calls it twice in a row through the C ABI, the second time on a smaller
 problem (the array still holds the first call's contents), and both outputs must equal
 kore_gemm's bit for bit; the first problem of each pair is also checked against the
@@ -35,6 +35,12 @@ def _noalloc(a, b, bias, act):
     return rc, c
 
 
+def _need(a, b):
+    """Workspace bytes that kore_gemm plans for a @ b."""
+    return _lib.load().kore_gemm_workspace_bytes(DT_CODE[a.dtype], 0, a.data_ptr(), *a.stride(), b.data_ptr(),
+                                                 *b.stride(), None, 256, b.shape[1], a.shape[0], b.shape[1], a.shape[1])
+
+
 def _inputs(M, N, K, dtype, layout, bias, seed, dev, a_t=False):
     g = torch.Generator().manual_seed(seed)
     sc = 1.0 / K ** 0.5
@@ -53,9 +59,11 @@ def _inputs(M, N, K, dtype, layout, bias, seed, dev, a_t=False):
 # (first problem, second smaller problem), dtype, B layout, bias, act, path
 CASES = [
     (((512, 1024, 4095), (200, 520, 2047)), torch.bfloat16, "kn", False, "none", "packed A"),
-    (((384, 768, 999), (256, 640, 999)), torch.float16, "nk", True, "gelu", "packed A and B"),
+    (((384, 768, 999), (256, 640, 999)), torch.float16, "nk", True, "gelu", "no scratch"),
+    (((320, 192, 9423), (300, 150, 9423)), torch.float16, "nk", True, "gelu", "packed A and B"),
     (((1, 2048, 4096), (1, 1024, 4096)), torch.bfloat16, "kn", False, "none", "split-K"),
-    (((4, 4096, 4096), (2, 2048, 2048)), torch.float16, "nk", True, "silu", "split-K"),
+    (((4, 4096, 4096), (2, 2048, 2048)), torch.float16, "nk", True, "silu", "no scratch"),
+    (((16, 2048, 12160), (16, 1920, 12160)), torch.float16, "nk", True, "silu", "split-K"),
     (((512, 1024, 4095), (300, 600, 1023)), torch.float32, "kn_at", True, "relu", "fp32 packed"),
     (((256, 256, 512), (128, 128, 256)), torch.bfloat16, "nk", False, "none", "no scratch"),
 ]
@@ -69,6 +77,7 @@ def test_noalloc_matches_kore_gemm(gpu, shapes, dtype, layout, bias, act, path):
                                         dev=gpu, a_t=layout.endswith("_at"))
         rc, c = _noalloc(ad, bd, bsd, act)
         _lib.check(rc)
+        assert i > 0 or (_need(ad, bd) > 0) == (path != "no scratch")
         outs.append((c, ad, bd, bsd, a, b, bs, (M, N, K)))
     torch.cuda.synchronize()
     for i, (c, ad, bd, bsd, a, b, bs, (M, N, K)) in enumerate(outs):
@@ -94,3 +103,22 @@ def test_noalloc_rejects_oversized_scratch(gpu):
     assert b"static scratch" in lib.kore_last_error()
     torch.cuda.synchronize()
     assert torch.isnan(c).all(), "nothing may be written when the scratch is too small"
+
+
+@pytest.mark.parametrize("M,N,K,a_along_m,b_along_n", [(4868, 49, 21042, True, True), (205, 1181, 29732, True, True),
+                                                       (1909, 27, 23020, True, False), (2500, 11, 16389, False, False)])
+def test_noalloc_takes_long_k_in_place(gpu, M, N, K, a_along_m, b_along_n):
+    """Ragged operands with a long K that are packed elsewhere, into more than the static
+    scratch holds, run in place here."""
+    lib = _lib.load()
+    g = torch.Generator(device=gpu).manual_seed(M + N + K)
+    a = (torch.randn((M, K), generator=g, device=gpu) / K ** 0.5).bfloat16()
+    b = torch.randn((K, N), generator=g, device=gpu).bfloat16()
+    a = a.t().contiguous().t() if a_along_m else a
+    b = b if b_along_n else b.t().contiguous().t()
+    cap = lib.kore_gemm_noalloc_scratch_bytes()
+    assert _need(a, b) > cap
+    rc, c = _noalloc(a, b, None, "none")
+    assert rc == 0, (rc, lib.kore_last_error())
+    verdict(c.cpu(), gemm_fusion_ref(a.cpu(), b.cpu(), None, "none"), "gemm_fusion", "bfloat16",
+            f"noalloc in place {M}x{N}x{K}")
