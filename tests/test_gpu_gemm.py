@@ -222,21 +222,41 @@ def test_batched_deep_ring(gpu):
     verdict(out, batched_gemm_ref(a, b), "gemm", "bf16", "batched deep 16x512x512x512")
 
 
-@pytest.mark.parametrize("M,N,K,dtype,op,layout", [(512, 4096, 4095, torch.float16, "gemm_bias_gelu", "kn"),
-                                                    (512, 4096, 4095, torch.bfloat16, "gemm_bias_silu", "nk"),
-                                                    (1024, 2048, 2047, torch.bfloat16, "gemm_relu", "kn_at"),
-                                                    (300, 1000, 777, torch.float16, "gemm_bias", "nk_at"),
-                                                    (2048, 2048, 1000, torch.bfloat16, "gemm", "strided")])
-def test_gemm_packed_path(gpu, M, N, K, dtype, op, layout):
-    """Operands the engines cannot read in place -- K tails that leave rows unaligned (the
-    gen_gemm_* K = 4095 validation shape), a transposed A, a B with a row stride that is
-    not a multiple of 8 -- are packed into the caller's workspace first."""
+def _scratch(a, b, out):
+    """Workspace bytes that the call out = a @ b plans (bf16, fp16)."""
+    from kore_amd import _lib
+    return _lib.load().kore_gemm_workspace_bytes(0 if a.dtype == torch.bfloat16 else 1, 0, a.data_ptr(), *a.stride(),
+                                                 b.data_ptr(), *b.stride(), None, out.data_ptr(), out.stride(0),
+                                                 *out.shape, a.shape[1])
+
+
+# (the last value: whether the call packs, that is, plans scratch)
+@pytest.mark.parametrize("M,N,K,dtype,op,layout,packs", [
+    (512, 4096, 4095, torch.float16, "gemm_bias_gelu", "kn", False),
+    (512, 4096, 4095, torch.bfloat16, "gemm_bias_silu", "nk", False),
+    (1024, 2048, 2047, torch.bfloat16, "gemm_relu", "kn_at", True),
+    (300, 1000, 777, torch.float16, "gemm_bias", "nk_at", False),
+    (2048, 2048, 1000, torch.bfloat16, "gemm", "strided", False),
+    (576, 320, 3653, torch.float16, "gemm_bias_gelu", "kn_at", True),
+    (340, 448, 7851, torch.bfloat16, "gemm_bias_silu", "nk_at", True),
+    (320, 192, 9423, torch.bfloat16, "gemm_relu", "nk", True),
+    (256, 130, 9001, torch.float16, "gemm_bias", "strided", True),
+    (512, 520, 1021, torch.bfloat16, "gemm_bias_gelu", "gap_kn", True),
+    (500, 512, 1024, torch.float16, "gemm", "gap_nk", True)])
+def test_gemm_packed_path(gpu, M, N, K, dtype, op, layout, packs):
+    """Operands with rows off the 16-byte alignment -- K tails (the gen_gemm_* K = 4095
+    validation shape), a transposed A, a B with a row stride that is not a multiple of 8 --
+    are read in place by the ring tiles or, where that is slower (a long K), packed into the
+    caller's workspace first; an A without a unit stride ("gap") is always packed."""
     has_bias, act = kore_amd.GEMM_FUSION_OPS.get(op, (False, "none"))
     g = torch.Generator().manual_seed(M + 3 * N + K)
     sc = 1.0 / K ** 0.5
     a = (torch.randn((M, K), generator=g) * sc).to(dtype)
     ad = a.t().contiguous().to(gpu).t() if layout.endswith("_at") else a.to(gpu)
-    if layout.startswith("kn"):
+    if layout.startswith("gap"):
+        ad = torch.full((M, 2 * K), float("nan"), dtype=dtype, device=gpu)[:, ::2]
+        ad.copy_(a)
+    if "kn" in layout:
         b = (torch.randn((K, N), generator=g) * sc).to(dtype)
         bd = b.to(gpu)
     elif layout == "strided":
@@ -249,6 +269,7 @@ def test_gemm_packed_path(gpu, M, N, K, dtype, op, layout):
     out = kore_amd.gemm_fused(ad, bd, bias.to(gpu) if has_bias else None, act)
     ref = gemm_fusion_ref(a, b, bias, act)
     dt = "bf16" if dtype == torch.bfloat16 else "fp16"
+    assert (_scratch(ad, bd, out) > 0) == packs
     verdict(out, ref, "gemm_fusion", dt, f"packed {op} {M}x{N}x{K} {layout}")
     pair_only(out, ref, dt, f"packed {op} {M}x{N}x{K} {layout}")
     # a second call (with its own workspace): same result bit for bit
@@ -289,16 +310,23 @@ def test_gemm_transposed_a_in_place(gpu, M, N, K, dtype, op, layout):
     assert torch.equal(out, kore_amd.gemm_fused(ad, bd, bias.to(gpu) if has_bias else None, act))
 
 
-@pytest.mark.parametrize("M,N,K,dtype,op,layout", [(1, 4096, 4096, torch.bfloat16, "gemm", "kn"),
-                                                    (16, 11008, 4096, torch.float16, "gemm_bias_gelu", "kn"),
-                                                    (7, 1002, 2048, torch.bfloat16, "gemm_bias_relu", "nk"),
-                                                    (33, 3000, 1024, torch.float16, "gemm_sigmoid", "nk"),
-                                                    (64, 4096, 4096, torch.bfloat16, "gemm_bias_silu", "kn"),
-                                                    (1, 5120, 4096, torch.bfloat16, "gemm_bias", "nk")])
-def test_gemm_splitk(gpu, M, N, K, dtype, op, layout):
+# (the last value: whether K is split; the other decode shapes run the skinny kernel or ring)
+@pytest.mark.parametrize("M,N,K,dtype,op,layout,split", [
+    (1, 4096, 4096, torch.bfloat16, "gemm", "kn", True),
+    (16, 11008, 4096, torch.float16, "gemm_bias_gelu", "kn", False),
+    (7, 1002, 2048, torch.bfloat16, "gemm_bias_relu", "nk", False),
+    (33, 3000, 1024, torch.float16, "gemm_sigmoid", "nk", False),
+    (64, 4096, 4096, torch.bfloat16, "gemm_bias_silu", "kn", True),
+    (1, 5120, 4096, torch.bfloat16, "gemm_bias", "nk", False),
+    (16, 2048, 12160, torch.float16, "gemm_bias_gelu", "nk", True),
+    (7, 4096, 4096, torch.float16, "gemm_bias_relu", "kn", True),
+    (100, 1001, 8192, torch.bfloat16, "gemm_sigmoid", "nk", True),
+    (128, 2002, 8192, torch.float16, "gemm_bias_silu", "nk", True),
+    (300, 520, 4096, torch.bfloat16, "gemm_bias", "kn", True)])
+def test_gemm_splitk(gpu, M, N, K, dtype, op, layout, split):
     """Decode-sized M with a long K splits K over the CUs (32x128 ring per slice, fp32
     partials, fixed-order reduce with the epilogue): ragged N (not a multiple of 4 on the
-    W.t() layout: the 8-column scalar reduce), 2, 4, 6 and 8 slices (the 4-column reduce's
+    W.t() layout: the 8-column scalar reduce), two slices and more (the 4-column reduce's
     unrolled and remainder loops), and bit-identical repeated calls."""
     has_bias, act = kore_amd.GEMM_FUSION_OPS.get(op, (False, "none"))
     g = torch.Generator().manual_seed(M + N + K + 1)
@@ -315,6 +343,7 @@ def test_gemm_splitk(gpu, M, N, K, dtype, op, layout):
     out = kore_amd.gemm_fused(*args)
     ref = gemm_fusion_ref(a, b, bias, act)
     dt = "bf16" if dtype == torch.bfloat16 else "fp16"
+    assert (_scratch(args[0], bd, out) > 0) == split
     verdict(out, ref, "gemm_fusion", dt, f"splitk {op} {M}x{N}x{K} {layout}")
     pair_only(out, ref, dt, f"splitk {op} {M}x{N}x{K} {layout}")
     assert torch.equal(out, kore_amd.gemm_fused(*args))
@@ -323,11 +352,15 @@ def test_gemm_splitk(gpu, M, N, K, dtype, op, layout):
 @pytest.mark.parametrize("M,N,K,dtype,op,a_t,b_layout", [(512, 512, 511, torch.bfloat16, "gemm_bias_gelu", False, "kn"),
                                                            (200, 300, 1001, torch.float16, "gemm_relu", True, "nk"),
                                                            (130, 129, 77, torch.bfloat16, "gemm", True, "odd"),
-                                                           (1, 257, 33, torch.float16, "gemm_bias_silu", False, "odd")])
+                                                           (1, 257, 33, torch.float16, "gemm_bias_silu", False, "odd"),
+                                                           (200, 130, 77, torch.float16, "gemm_relu", False, "gap"),
+                                                           (130, 300, 129, torch.bfloat16, "gemm_bias_gelu", True, "gap"),
+                                                           (257, 129, 63, torch.bfloat16, "gemm", True, "kn")])
 def test_gemm_generic_mfma(gpu, M, N, K, dtype, op, a_t, b_layout):
-    """Problems too small for a pack pass in layouts the engines cannot read (odd K,
-    transposed A, B rows with an odd stride) run the generic MFMA kernel: element reads
-    along the unit-stride index, every read bounds-checked, ragged tiles on every edge."""
+    """Small problems off the engines' layouts: odd K, transposed A, B rows with an odd stride
+    run the ring tiles in place; K < 64 and a B without a unit stride ("gap") the generic MFMA
+    kernel: element reads along the unit-stride index, every read bounds-checked, ragged tiles
+    on every edge."""
     has_bias, act = kore_amd.GEMM_FUSION_OPS.get(op, (False, "none"))
     g = torch.Generator().manual_seed(M + N + K + 7)
     sc = 1.0 / K ** 0.5
@@ -339,6 +372,9 @@ def test_gemm_generic_mfma(gpu, M, N, K, dtype, op, a_t, b_layout):
     elif b_layout == "nk":
         w = (torch.randn((N, K), generator=g) * sc).to(dtype)
         b, bd = w.t(), w.to(gpu).t()
+    elif b_layout == "gap":
+        full = (torch.randn((K, 2 * N), generator=g) * sc).to(dtype)
+        b, bd = full[:, ::2], full.to(gpu)[:, ::2]
     else:
         full = (torch.randn((K, N + 5), generator=g) * sc).to(dtype)
         b, bd = full[:, 2:2 + N], full.to(gpu)[:, 2:2 + N]
@@ -405,15 +441,21 @@ def test_gemm_fp32_k_tail_in_place(gpu, K, layout):
     pair_only(out, ref, "fp32", f"fp32 K tail {K} {layout}")
 
 
-def test_batched_packed_path(gpu):
-    """A batched problem with an odd K runs the packed path per batch."""
+@pytest.mark.parametrize("Bn,M,N,K", [(4, 512, 384, 999), (2, 320, 192, 9423), (3, 200, 260, 8193)])
+def test_batched_packed_path(gpu, Bn, M, N, K):
+    """Batched problems with an odd K: a short one on the ring in place, long ones packed."""
+    from kore_amd import _lib
     from oracle.gemm import batched_gemm_ref
 
     g = torch.Generator().manual_seed(9)
-    a = (torch.randn((4, 512, 999), generator=g) / 999 ** 0.5).bfloat16()
-    b = (torch.randn((4, 384, 999), generator=g) / 999 ** 0.5).bfloat16()
-    out = kore_amd.batched_gemm(a.to(gpu), b.to(gpu))
-    verdict(out, batched_gemm_ref(a, b), "gemm", "bf16", "batched packed 4x512x384x999")
+    a = (torch.randn((Bn, M, K), generator=g) / K ** 0.5).bfloat16()
+    b = (torch.randn((Bn, N, K), generator=g) / K ** 0.5).bfloat16()
+    ag, bg = a.to(gpu), b.to(gpu)
+    out = kore_amd.batched_gemm(ag, bg)
+    need = _lib.load().kore_batched_gemm_workspace_bytes(0, ag.data_ptr(), *ag.stride(), bg.data_ptr(), *bg.stride(),
+                                                         out.data_ptr(), *out.stride()[:2], Bn, M, N, K)
+    assert (need > 0) == (K > 8000)
+    verdict(out, batched_gemm_ref(a, b), "gemm", "bf16", f"batched packed {Bn}x{M}x{N}x{K}")
 
 
 @pytest.mark.parametrize("B,M,N,K", [(4, 1024, 1024, 1023), (4, 2048, 2048, 2047)])
@@ -539,7 +581,7 @@ def test_gemm_repitch_k_tails(gpu, dtype, K, start):
 
 
 def test_batched_repitch_k_tail(gpu):
-    """Batched packed path with a K tail (K = 1001): per-batch re-stride of A and B^T."""
+    """Batched ragged rows with a K tail (K = 1001): per-batch offsets off the 16-byte alignment."""
     Bn, M, N, K = 4, 512, 512, 1001
     g = torch.Generator().manual_seed(1)
     a = (torch.randn((Bn, M, K), generator=g) * 0.1).bfloat16()
@@ -742,7 +784,8 @@ def test_workspace_paths_under_graph_capture(gpu):
                                    (64, 100, 64), (2, 430, 2048)])
 def test_gemm_skinny(gpu, dtype, M, N, K):
     """M <= 128 against K-contiguous weights (the skinny kernel): row, column and K tails,
-    16-, 32- and 64-column workgroups of each height (16, 32, 64 and 128 rows), bias and activation, rows at odd element offsets (the
+    16-, 32- and 64-column workgroups of 16, 32, 64 and 128 rows, bias and activation, rows at
+    odd element offsets (the
     same bits as aligned rows when both take this kernel), and an infinity in a column that
     the tail block repeats, which must reach exactly its own row and column."""
     g = torch.Generator().manual_seed(M + N + K)
@@ -930,7 +973,6 @@ def test_gemm_splitk_tall(gpu, dtype, act, M, N, K, layout):
     """Split-K over one tile of 64 or 128 rows (M > 32 and more than 24 MiB of weights), both
     weight layouts: full tiles, row remainders and an N off the 128-column tile.  The planned
     workspace shows that the shape takes split-K: fp32 partials of two slices or more."""
-    from kore_amd import _lib
     g = torch.Generator().manual_seed(M + N + K)
     a = (torch.randn((M, K), generator=g) / K ** 0.5).to(dtype)
     w = torch.randn((K, N) if layout == "kn" else (N, K), generator=g).to(dtype)
@@ -938,10 +980,7 @@ def test_gemm_splitk_tall(gpu, dtype, act, M, N, K, layout):
     b, bd = (w, w.to(gpu)) if layout == "kn" else (w.t(), w.to(gpu).t())
     ag = a.to(gpu)
     out = kore_amd.gemm_fused(ag, bd, bias.to(gpu), act)
-    need = _lib.load().kore_gemm_workspace_bytes(0 if dtype == torch.bfloat16 else 1, 0, ag.data_ptr(), *ag.stride(),
-                                                 bd.data_ptr(), *bd.stride(), None, out.data_ptr(), out.stride(0),
-                                                 M, N, K)
-    assert need >= 2 * M * N * 4
+    assert _scratch(ag, bd, out) >= 2 * M * N * 4
     name = "bf16" if dtype == torch.bfloat16 else "fp16"
     pair_only(out.cpu(), gemm_fusion_ref(a, b, bias, act), name, f"tall split-K {M}x{N}x{K} {layout} {act}")
     assert bit_equal(out, kore_amd.gemm_fused(ag, bd, bias.to(gpu), act))
