@@ -1577,7 +1577,7 @@ inline double ragged_ring_us(const GemmDesc& d) {
   TileShape t = d.sak != 1 ? TILE_128x128 : pick_tile(d);
   if (t == TILE_256x256) t = TILE_256x128;
   const bool in_place = padded_b_inplace(d);
-  const double slow = d.sak != 1 ? (in_place ? 0.97 : 1.11) : d.sbk == 1 ? 1.72 : in_place ? 1.3 : 1.45;
+  const double slow = d.sak != 1 ? (in_place ? 1.15 : 1.06) : d.sbk == 1 ? 1.8 : in_place ? 1.3 : 1.45;
   return 2.3 + tile_rounds(d, t) * (5.3 + (double)d.K * kTileCost[t].ns * 1e-3 * slow);
 }
 // Ragged ring: operands with a unit stride along either index, at any 2-byte alignment, any
@@ -1590,7 +1590,7 @@ inline double ragged_ring_us(const GemmDesc& d) {
 // 58 / 76 us on the ring, 35 / 40 packed; both along K, 320 x 192 x 9423 67 / 98 against
 // 54 / 54).  Packed operands run the faster 256x256 tiles, so they stay from 2^34 products on
 // (4097^3).  Scratch beyond `limit` bytes keeps a problem on the ring: kore_gemm_noalloc, which
-// cannot grow its scratch, takes in place what would not fit (4868 x 49 x 21042: 207 MB packed).
+// cannot grow its scratch, takes in place what would not fit (205 x 1181 x 29732: 82 MB packed).
 inline bool ragged_ring_ok(const GemmDesc& d, size_t limit) {
   const bool akc = d.sak == 1, bkc = d.sbk == 1;
   if (d.K < 64 || !(akc || d.sam == 1) || !(bkc || d.sbn == 1) || d.M * d.N * d.K * d.batch >= (1ll << 34)) return false;
@@ -1601,8 +1601,10 @@ inline bool ragged_ring_ok(const GemmDesc& d, size_t limit) {
   if ((akc ? d.sam * 2 * 256 + d.K * 2 : d.sak * 2 * (d.K + 64) + 512) >= lim ||
       (bkc ? d.sbn * 2 * 256 + d.K * 2 : d.sbk * 2 * (d.K + 64) + 512) >= lim)
     return false;
-  // (by a twentieth: what the two estimates differ by where they are off)
-  return d.M * d.N * d.K < (1ll << 27) || !padded_fits(d) || 1.05 * ragged_ring_us(d) < packed_us(d) ||
+  // (packed where that is estimated faster by a twentieth: over 703 drawn shapes 0.6% above the
+  // faster of the two; with the twentieth on the ring's side 1.0%, and twice as many shapes
+  // slower on the pack pass than they are in place)
+  return d.M * d.N * d.K < (1ll << 27) || !padded_fits(d) || ragged_ring_us(d) < 1.05 * packed_us(d) ||
          packed_bytes(d).total() > limit;
 }
 template <typename T>
