@@ -272,8 +272,9 @@ __global__ void __launch_bounds__(64 * NWV)
 }
 
 // Mid-size problems (a few hundred tiles, long K) on the deep ring engine: NSLOT - 1
-// K stages in flight per CU instead of one or two.  Either B layout, K % 64 == 0 (KT:
-// K tails read in place, the ring engine's K-tail mode).
+// K stages in flight per CU instead of one or two.  Either B layout, 16-byte rows and
+// K % 64 == 0; KT (the ring engine's K-tail mode): K tails and rows at any 2-byte alignment
+// read in place, A along K or, AL = A_MC, along M.
 template <typename T, int BM, int BN, int WM, int WN, int NSLOT, int BL, bool KT = false, int AL = A_KC>
 __global__ void __launch_bounds__(256) gemm_deep_kernel(const TileParams p) {
   using E = RingEngine<T, BM, BN, WM, WN, NSLOT, BL, kCpolDefault, AL>;

@@ -471,9 +471,10 @@ __global__ void __launch_bounds__(64 * NWV)
   if constexpr (MODE != MOE_DOWN) {
     // A padding row's offset lies at the end of the resource (as in moe_decode_kernel): its
     // loads return zeros with no memory traffic, and it is never stored.  Against re-reading
-    // token 0 (gate_up) and the unused H rows (down), one process: E=8 top-2 D=4096 I=14336
-    // T=4096 3.58 -> 3.45 ms, T=700 903 -> 863 us; E=32 top-8 D=1024 I=768 T=512 on 256-row
-    // blocks 74.8 -> 69.3 us.  The plain grouped GEMM did not change.
+    // token 0 (gate_up) and the unused H rows (down), repeated on one input: E=8 top-2 D=4096
+    // I=14336 T=700 903 -> 863 us, T=4096 3.58 -> 3.45 ms (3.50 -> 3.45, within the noise, where
+    // inputs change from call to call); E=32 top-8 D=1024 I=768 T=512 on 256-row blocks 74.8 ->
+    // 69.3 us.  The plain grouped GEMM did not change.
     const uint32_t bytes = (uint32_t)((int64_t)p.T * p.ldx * 2);
     eng.ra = make_rsrc(p.x, bytes);
 #pragma unroll
@@ -662,8 +663,8 @@ inline int64_t align_capacity(int64_t S, int64_t E, int64_t block) {
 // nearly every expert's weights are streamed once (padding rows cost MFMA cycles, which
 // are idle on these weight-bound shapes, but no memory traffic); beyond: 256.  At a mean of
 // 128 half of the experts spill into a second 128-row block and stream their weights
-// twice: 256-row blocks there measured, in one process, E=32 top-8 D=1024 I=768 T=512 98.5
-// -> 69.3 us, E=8 top-2 D=4096 I=14336 T=512 1021 -> 832 us (a mean of 100: 61.4 against
+// twice: 256-row blocks there measured, repeated on one input, E=32 top-8 D=1024 I=768 T=512
+// 98.5 -> 69.3 us (98.4 -> 79.5 where inputs change from call to call), E=8 top-2 D=4096 I=14336 T=512 1021 -> 832 us (a mean of 100: 61.4 against
 // 67.3, 648 against 788).  Where one block per expert leaves the CUs half empty (E * I / 128
 // below 128) the time is one tile's latency, so the smaller blocks last longer: E=8 top-2
 // D=1024 I=1408, T=200 / 300 / 512 / 800: 32 rows 47.7 / 61.4 / 76.1 / 121, 128 rows 55.5 /
@@ -854,7 +855,8 @@ extern "C" int kore_fused_moe(const void* hidden, int64_t ldh, const void* w1, c
   // Stages of the decode rings: what one workgroup keeps in flight, against two workgroups
   // per CU whose prologues and epilogues overlap.  With enough live tiles (one block per
   // expert that can receive a slot) two fit: 32 rows, 4 against 7 stages, E=64 top-4 D=2048
-  // I=1024 T=200 181 -> 167 us, E=8 top-2 D=4096 I=14336 T=64 474 -> 462, E=32 top-8 D=1024
+  // I=1024 T=200 181 -> 167 us, E=8 top-2 D=4096 I=14336 T=64 474 -> 462 (492 -> 480 where
+  // inputs change from call to call), E=32 top-8 D=1024
   // I=768 T=64 44.6 -> 42.7; with few tiles the deep ring wins (the last at T=1: 25.6 against
   // 30.4 us).  128 rows, 3 against 2 stages where no CU has two tiles: E=8 top-2 D=1024
   // I=1408 T=400 60.2 -> 52.7 us.  Down, 3 against 6 stages: E=64 as above, T=200 181 -> 176 us.
@@ -956,7 +958,8 @@ __global__ void __launch_bounds__(256)
 }
 
 // Tiles of 256x256 to expect: M / 256 full blocks, and for about half of the (unevenly
-// loaded) experts one more that is mostly padding.
+// loaded) experts one more that is mostly padding.  (The counts it is compared with below are
+// those of this chip's 256 CUs.)
 inline int64_t grouped_tiles256(int64_t M, int64_t E, int64_t N) { return (M / 256 + E / 2) * (N / 256); }
 
 // Block rows of the fp8 grouped tiles: 256x256 when experts average over 64 rows (one round

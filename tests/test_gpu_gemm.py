@@ -785,9 +785,9 @@ def test_workspace_paths_under_graph_capture(gpu):
 def test_gemm_skinny(gpu, dtype, M, N, K):
     """M <= 128 against K-contiguous weights (the skinny kernel): row, column and K tails,
     16-, 32- and 64-column workgroups of 16, 32, 64 and 128 rows, bias and activation, rows at
-    odd element offsets (the
-    same bits as aligned rows when both take this kernel), and an infinity in a column that
-    the tail block repeats, which must reach exactly its own row and column."""
+    odd element offsets (the same bits as aligned rows when both take this kernel), and an
+    infinity in a column that the tail block repeats, which must reach exactly its own row and
+    column."""
     g = torch.Generator().manual_seed(M + N + K)
     a = (torch.randn((M, K), generator=g) / K ** 0.5).to(dtype)
     w = torch.randn((N, K), generator=g).to(dtype)
