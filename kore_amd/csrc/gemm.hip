@@ -1674,12 +1674,13 @@ inline SplitPlan splitk_plan(const GemmDesc& d) {
 }
 
 // Skinny kernel: columns per workgroup (16 nb) and estimated time.  A round of workgroups has
-// a fixed part and takes in (M + 16 nb) rows of K per CU, at 50 to 60 KB/us, a quarter more
+// a fixed part and takes in (M + 16 nb) rows of K per CU, at 46 to 60 KB/us, a quarter more
 // where half of the CUs have none (64-column workgroups of many rows have fewer waves to do
-// it, and few of them do not reach the memory's rate); rows off 16-byte alignment cost 1.4
-// times as much.  N-contiguous weights cost a workgroup one cache line per K-row however few
-// of its columns it owns, and up to two where the rows start off the 128-byte lines: that
-// slows their stream and what one workgroup gets of it.  Measured (bf16, one process,
+// it, and few of them do not reach the memory's rate); rows off 16-byte alignment cost more
+// (W.t() 1.4 times, with [K,N] those of A 1.25).  N-contiguous weights cost a workgroup one
+// cache line per K-row however few of its columns it owns, and a 64-column one two where the
+// rows start off the 128-byte lines: that slows their stream and what one workgroup gets of
+// it.  Measured (bf16, one process,
 // repeated / flushed calls), nb = 1 | 2 | 4:
 //   W.t() 4 x 4096 x 4096     6.9 / 12.0 |  6.7 / 11.1 | 12.4 / 16.1
 //   W.t() 16 x 14336 x 2048  16.0 / 19.4 | 12.7 / 16.1 | 11.0 / 14.6
@@ -1693,19 +1694,19 @@ struct SkinnyPick {
 };
 // rows16: 16-byte rows, of both operands or, for N-contiguous weights, of A
 inline SkinnyPick pick_skinny(const GemmDesc& d, bool nc, bool rows16) {
-  static const double nc_stream[] = {2.0e6, 2.8e6, 4.6e6}, nc_own[] = {23e3, 42e3, 50e3}, off_lines[] = {1.4, 1.4, 1.8};
+  static const double nc_stream[] = {1.7e6, 2.9e6, 4.6e6}, nc_own[] = {25.5e3, 42e3, 37.5e3}, off_lines[] = {1.07, 1.0, 1.44};
   const int64_t cus = d.cus;
   const bool lines = d.sbk % 64 == 0 && ((uintptr_t)d.b & 127u) == 0;
   SkinnyPick best{1, 1e300};
   for (int i = 0; i < 3; ++i) {
     const int64_t nb = 1 << i, bn = 16 * nb, wgs = (d.N + bn - 1) / bn, rounds = (wgs + cus - 1) / cus;
     const double rows = (double)(d.M + bn);
-    const double few_waves = nb < 4 || d.M <= 32 ? 1.0 : d.M <= 64 ? (nc ? 1.25 : 1.1) : (nc ? 1.6 : 1.4);
+    const double few_waves = nb < 4 || d.M <= 32 ? 1.0 : d.M <= 64 ? (nc ? 1.0 : 1.1) : (nc ? 1.35 : 1.4);
     double k = (double)(d.K * 2), us;  // bytes of a row
     if (nc) {
       const double off = lines ? 1.0 : off_lines[i];
-      if (!rows16) k *= 1.0 + 0.4 * (double)d.M / rows;
-      us = 1.9 + std::max((double)rounds * (2.1 + few_waves * k * std::max(rows / 50e3, off * (double)bn / nc_own[i])),
+      if (!rows16) k *= 1.0 + 0.25 * (double)d.M / rows;
+      us = 1.9 + std::max((double)rounds * (2.05 + few_waves * k * std::max(rows / 46.5e3, off * (double)bn / nc_own[i])),
                           k * off * (double)d.N / nc_stream[i]);
     } else {
       if (!rows16) k *= 1.4;
